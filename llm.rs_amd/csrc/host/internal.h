@@ -151,6 +151,13 @@ struct GemvPlan {
   size_t lds = 0;
 };
 GemvPlan gemv_plan(int wt, const std::string& kind, int n, int k, int num_cus);
+// Launch plan of one skinny GEMM (sgemm.hip; epi: store, resid, silu).
+struct SgemmPlan {
+  std::string name;
+  unsigned grid = 1;
+};
+bool sgemm_serves(size_t m, size_t k);
+SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus);
 // LDS bytes of a GEMV's activation area (codes, scales, Q4 offsets) for input length k.
 inline size_t gemv_act_lds_host(int k) { return (size_t)k + 8 * (size_t)(k / 32); }
 

@@ -667,18 +667,18 @@ void ensure_prefill(llmrs_model* m) {
   if (m->pf_cap) return;
   const llmrs_model_config& c = m->c;
   const int cap = std::max(1, std::min(c.max_seq, env_int("LLMRS_PREFILL_CHUNK", 2048)));
-  const size_t M = (size_t)cap, H = c.hidden, F = c.ffn, qd = (size_t)c.n_heads * c.head_dim;
+  const size_t M = (size_t)cap, MA = llmrs::act_rows(M), H = c.hidden, F = c.ffn, qd = (size_t)c.n_heads * c.head_dim;
   const size_t kmax = std::max(H, std::max(F, qd));
   m->pf_x = m->dalloc<float>(M * H);
   m->pf_h = m->dalloc<float>(M * H);
   m->pf_qkv = m->dalloc<float>(M * m->qkv_rows);
   m->pf_q = m->dalloc<float>(M * qd);
-  m->pf_aq = m->dalloc<int8_t>(M * kmax);
-  m->pf_ad = m->dalloc<float>(M * kmax / 32);
-  m->pf_ctx_q = m->dalloc<int8_t>(M * qd);
-  m->pf_ctx_d = m->dalloc<float>(M * qd / 32);
-  m->pf_m_q = m->dalloc<int8_t>(M * F);
-  m->pf_m_d = m->dalloc<float>(M * F / 32);
+  m->pf_aq = m->dalloc<int8_t>(MA * kmax);
+  m->pf_ad = m->dalloc<float>(MA * kmax / 32);
+  m->pf_ctx_q = m->dalloc<int8_t>(MA * qd);
+  m->pf_ctx_d = m->dalloc<float>(MA * qd / 32);
+  m->pf_m_q = m->dalloc<int8_t>(MA * F);
+  m->pf_m_d = m->dalloc<float>(MA * F / 32);
   m->pf_start = m->dalloc<int>(1);
   LLMRS_HIP(hipStreamSynchronize(ctx().stream));
   m->pf_cap = cap;
@@ -688,32 +688,12 @@ std::string gemm_kernel(const llmrs_model* m, const char* epi) {
   return std::string("gemm_") + wt_tag(m->wt) + "_" + epi;
 }
 
-// Whether M prefill rows run their linear layers on the skinny GEMM's exact
-// launches (sgemm.hip, up to 64 rows; the activation codes then in its
-// operand order) rather than the 128 x 128-tile GEMM, which a short prompt
-// leaves mostly idle; both are bit-identical to the reference's block loop.
-// LLMRS_PREFILL_SKINNY=0 keeps every prefill on the tile GEMM.
+// Whether M prefill rows run their linear layers on the skinny GEMM (sgemm.hip;
+// the activation codes then in its operand order) rather than the 128 x
+// 128-tile GEMM; both are bit-identical to the reference's block loop.
 bool prefill_skinny(const llmrs_model* m, int M) {
   const llmrs_model_config& c = m->c;
-  return M <= 64 && c.hidden % 128 == 0 && c.ffn % 128 == 0 && (c.n_heads * c.head_dim) % 128 == 0 &&
-         env_int("LLMRS_PREFILL_SKINNY", 1) != 0;
-}
-
-// The skinny GEMM kernel of an epilogue for M rows (store, resid, silu);
-// exact: each output's blocks in one wave, in order (prompt prefill).
-std::string sgemm_kernel(const llmrs_model* m, const char* epi, int M, bool exact) {
-  return std::string("sgemm_") + wt_tag(m->wt) + "_" + epi + "_t" + (M <= 16 ? "1" : M <= 32 ? "2" : "4") +
-         (exact ? "_exact" : "");
-}
-
-// Launch shape of a skinny GEMM (sgemm.hip): SwiGLU 64 rows per 256-thread
-// workgroup; exact store / residual 16 rows per one-wave workgroup; else
-// residual 16 and store 32 rows per 256-thread workgroup.
-std::pair<dim3, dim3> sgemm_shape(const char* epi, int N, bool exact) {
-  const std::string e(epi);
-  const int rows = e == "silu" ? 64 : exact || e == "resid" ? 16 : 32;
-  const unsigned threads = exact && e != "silu" ? 64 : 256;
-  return {dim3((unsigned)((N + rows - 1) / rows)), dim3(threads)};
+  return sgemm_serves(M, c.hidden) && sgemm_serves(M, c.ffn) && sgemm_serves(M, (size_t)c.n_heads * c.head_dim);
 }
 
 dim3 gemm_grid(int M, int N) { return dim3((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128)); }
@@ -769,8 +749,8 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
     const double work = flops(M, W.n, W.k);
     if (skinny) {
       SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, layout};
-      const auto sh = sgemm_shape(epi, W.n, true);
-      L(sgemm_kernel(m, epi, M, true), work, sh.first, sh.second, 0, g);
+      const SgemmPlan p = sgemm_plan(m->wt, epi, M, W.n, ctx().num_cus);
+      L(p.name, work, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
     } else {
       PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, gemm_group_m()};
       L(gemm_kernel(m, epi), work, gemm_grid(M, W.n), blk, glds, g);
@@ -1891,27 +1871,39 @@ int llmrs_model_probe_prefill_layer(llmrs_model* m, int layer, size_t start_pos,
     p.ctx = pb.get<float>(M * qd);
     p.mf = pb.get<float>(M * F);
     LLMRS_HIP(hipMemcpyAsync(m->pf_x, x, M * H * sizeof(float), hipMemcpyHostToDevice, s));
+    const int layout = prefill_skinny(m, (int)M) ? llmrs::kActMfma : llmrs::kActNatural;
+    // codes and scales of the M rows, back in element order
+    auto copy_act = [&](int8_t* q, float* d, const int8_t* dev_q, const float* dev_d, size_t K) {
+      const size_t rows = llmrs::act_rows(M);
+      std::vector<int8_t> hq(rows * K);
+      std::vector<float> hd(rows * K / 32);
+      probe_copy(hq.data(), dev_q, hq.size());
+      probe_copy(hd.data(), dev_d, hd.size() * sizeof(float));
+      LLMRS_HIP(hipStreamSynchronize(s));
+      for (size_t t = 0; t < M; ++t) {
+        for (size_t k = 0; q && k < K; ++k)
+          q[t * K + k] = hq[llmrs::act_row(t, K, layout) + llmrs::act_offset((int)k, layout)];
+        for (size_t b = 0; d && b < K / 32; ++b)
+          d[t * (K / 32) + b] = hd[llmrs::act_scale_row(t, K / 32, layout) + llmrs::act_scale_offset((int)b, layout)];
+      }
+    };
     p.after = [&](int stage) {
       switch (stage) {
         case 0:
-          probe_copy(out->xq, m->pf_aq, M * H);
-          probe_copy(out->xd, m->pf_ad, M * H / 32 * sizeof(float));
+          copy_act(out->xq, out->xd, m->pf_aq, m->pf_ad, H);
           break;
         case 1: probe_copy(out->qkv, m->pf_qkv, M * m->qkv_rows * sizeof(float)); break;
         case 3:
           probe_copy(out->ctx, p.ctx, M * qd * sizeof(float));
-          probe_copy(out->ctx_q, m->pf_ctx_q, M * qd);
-          probe_copy(out->ctx_d, m->pf_ctx_d, M * qd / 32 * sizeof(float));
+          copy_act(out->ctx_q, out->ctx_d, m->pf_ctx_q, m->pf_ctx_d, qd);
           break;
         case 4: probe_copy(out->h, m->pf_h, M * H * sizeof(float)); break;
         case 5:
-          probe_copy(out->hq, m->pf_aq, M * H);
-          probe_copy(out->hd, m->pf_ad, M * H / 32 * sizeof(float));
+          copy_act(out->hq, out->hd, m->pf_aq, m->pf_ad, H);
           break;
         case 6:
           probe_copy(out->m, p.mf, M * F * sizeof(float));
-          probe_copy(out->m_q, m->pf_m_q, M * F);
-          probe_copy(out->m_d, m->pf_m_d, M * F / 32 * sizeof(float));
+          copy_act(out->m_q, out->m_d, m->pf_m_q, m->pf_m_d, F);
           break;
         case 7: probe_copy(out->out, m->pf_x, M * H * sizeof(float)); break;
       }
@@ -1919,21 +1911,6 @@ int llmrs_model_probe_prefill_layer(llmrs_model* m, int layer, size_t start_pos,
     };
     Launcher L{s};
     enqueue_prefill_layer(m, L, layer, start_pos, (int)M, &p, nullptr, nullptr, m->exact);
-    if (prefill_skinny(m, (int)M)) {  // codes back into element order
-      auto natural = [&](int8_t* rows, size_t K) {
-        if (!rows) return;
-        std::vector<int8_t> tmp(K);
-        for (size_t t = 0; t < M; ++t) {
-          int8_t* r = rows + t * K;
-          for (size_t k = 0; k < K; ++k) tmp[k] = r[llmrs::act_offset((int)k, llmrs::kActMfma)];
-          std::memcpy(r, tmp.data(), K);
-        }
-      };
-      natural(out->xq, H);
-      natural(out->ctx_q, qd);
-      natural(out->hq, H);
-      natural(out->m_q, F);
-    }
     m->begun = false;
   });
 }
@@ -1967,8 +1944,8 @@ struct llmrs_batch {
   // one XCD so that the weights stream from HBM about once and the other rows
   // read them from its L2; up to kBatchGemvMax sequences), on the skinny GEMM
   // (sgemm.hip; token tiles of 16, the activation codes in its operand order)
-  // or, beyond 64 sequences or for widths not a multiple of 128, on the
-  // prefill GEMM
+  // or, beyond its rows or for widths not a multiple of 128, on the prefill
+  // GEMM
   bool gemv = false;
   bool skinny = false;
   int layout = llmrs::kActNatural;
@@ -2010,7 +1987,7 @@ GemvPlan batch_gemv_plan(const llmrs_batch* b, const char* epi, const DevLinear&
 
 std::string batch_linear_kernel(const llmrs_batch* b, const char* epi, const DevLinear& W) {
   if (b->gemv) return batch_gemv_plan(b, epi, W).name;
-  return b->skinny ? sgemm_kernel(b->m, epi, b->B, false) : gemm_kernel(b->m, epi);
+  return b->skinny ? sgemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name : gemm_kernel(b->m, epi);
 }
 
 // One greedy step of every sequence of the batch.
@@ -2045,8 +2022,8 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
       L(name, wb, dim3(8u * (unsigned)B * ((p.grid + 7) / 8)), dim3(p.threads), p.lds, g);
     } else if (b->skinny) {
       SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, W.n, b->layout};
-      const auto sh = sgemm_shape(epi, W.n, false);
-      L(name, wb, sh.first, sh.second, 0, g);
+      const SgemmPlan p = sgemm_plan(m->wt, epi, B, W.n, ctx().num_cus);
+      L(p.name, wb, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
     } else {
       PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, silu ? W.n / 2 : W.n, gemm_group_m()};
       L(name, wb, gemm_grid(B, W.n), blk, glds, g);
@@ -2153,7 +2130,8 @@ int llmrs_batch_create(llmrs_model* m, int32_t batch, llmrs_batch** out) {
     b->B = batch;
     b->cap = m->cap;
     b->kv_bytes = align_up(kv_layer_elems(m) * kv_elem_bytes(m), 256);
-    const size_t B = (size_t)batch, H = c.hidden, F = c.ffn, qd = (size_t)c.n_heads * c.head_dim;
+    const size_t B = (size_t)batch, BA = llmrs::act_rows(B), H = c.hidden, F = c.ffn;
+    const size_t qd = (size_t)c.n_heads * c.head_dim;
     for (int li = 0; li < c.n_layers; ++li) {
       b->kc.push_back(b->dalloc<uint8_t>(B * b->kv_bytes));
       b->vc.push_back(b->dalloc<uint8_t>(B * b->kv_bytes));
@@ -2163,12 +2141,12 @@ int llmrs_batch_create(llmrs_model* m, int32_t batch, llmrs_batch** out) {
     b->qkv = b->dalloc<float>(B * m->qkv_rows);
     b->ctxv = b->dalloc<float>(B * qd);
     b->logits = b->dalloc<float>(B * c.vocab);
-    b->aq = b->dalloc<int8_t>(B * H);
-    b->ad = b->dalloc<float>(B * H / 32);
-    b->ctx_q = b->dalloc<int8_t>(B * qd);
-    b->ctx_d = b->dalloc<float>(B * qd / 32);
-    b->m_q = b->dalloc<int8_t>(B * F);
-    b->m_d = b->dalloc<float>(B * F / 32);
+    b->aq = b->dalloc<int8_t>(BA * H);
+    b->ad = b->dalloc<float>(BA * H / 32);
+    b->ctx_q = b->dalloc<int8_t>(BA * qd);
+    b->ctx_d = b->dalloc<float>(BA * qd / 32);
+    b->m_q = b->dalloc<int8_t>(BA * F);
+    b->m_d = b->dalloc<float>(BA * F / 32);
     b->part_o = b->dalloc<float>(B * qd * m->nsplit);
     b->part_ml = b->dalloc<float>(B * c.n_heads * llmrs::ml_stride(m->nsplit) * 2);
     b->counters = b->dalloc<int>((size_t)c.n_layers * B * c.n_kv_heads * llmrs::kTicketStride);
@@ -2181,18 +2159,17 @@ int llmrs_batch_create(llmrs_model* m, int32_t batch, llmrs_batch** out) {
     const int qdim = c.n_heads * c.head_dim;
     const std::string bg = env_str("LLMRS_BATCH_GEMM");  // gemv, skinny or prefill forces one
     b->gemv = bg == "gemv" || (bg.empty() && batch <= kBatchGemvMax);
-    b->skinny = !b->gemv && batch <= 64 && c.hidden % 128 == 0 && c.ffn % 128 == 0 && qdim % 128 == 0 &&
-                bg != "prefill";
+    b->skinny = !b->gemv && bg != "prefill" && sgemm_serves(batch, c.hidden) && sgemm_serves(batch, c.ffn) &&
+                sgemm_serves(batch, qdim);
     b->layout = b->skinny ? llmrs::kActMfma : llmrs::kActNatural;
     b->nsplit = std::max(1, std::min(m->nsplit, (2 * ctx().num_cus + batch * c.n_kv_heads - 1) /
                                                      (batch * c.n_kv_heads)));
     LLMRS_HIP(hipStreamSynchronize(ctx().stream));
     (void)kernel("argmax_batch", dim3(1024));
-    for (const char* epi : {"store", "resid", "silu"}) {
-      const DevLinear& W = std::string(epi) == "store" ? m->lm_head : std::string(epi) == "resid" ? m->layers[0].down
-                                                                                             : m->layers[0].gu;
-      (void)kernel(batch_linear_kernel(b.get(), epi, W), dim3(256));
-    }
+    const LayerBufs& L0 = m->layers[0];  // every linear layer's kernel, so graph capture never looks one up
+    for (const auto& [epi, W] : {std::pair<const char*, const DevLinear*>{"store", &L0.qkv}, {"store", &m->lm_head},
+                                 {"resid", &L0.o}, {"resid", &L0.down}, {"silu", &L0.gu}})
+      (void)kernel(batch_linear_kernel(b.get(), epi, *W), dim3(256));
     *out = b.release();
     ++m->live_batches;
   });

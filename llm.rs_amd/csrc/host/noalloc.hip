@@ -91,10 +91,22 @@ extern "C" int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmr
     LLMRS_REQUIRE(m <= 65535 * 128, LLMRS_E_INVALID, "matmul_transposed: too many rows");
     LLMRS_REQUIRE(cx.noalloc_scratch, LLMRS_E_NOINIT,
                   "the scratch's device address was not resolved at init: " + cx.noalloc_error);
+    // few rows of whole 128-element runs: the skinny GEMM, where its whole
+    // 16-row tiles fit the scratch too
+    size_t tile_off = 0;
+    const bool skinny = sgemm_serves(m, k) && scratch_need(act_rows(m), k, &tile_off) <= kNoAllocScratchBytes;
+    if (skinny) scale_off = tile_off;
     int8_t* xq = (int8_t*)cx.noalloc_scratch;
     float* xd = (float*)((uint8_t*)cx.noalloc_scratch + scale_off);
-    PrefillRowArgs r{(const float*)a->data, nullptr, xq, xd, (int)m, (int)k, 0.0f};
+    PrefillRowArgs r{(const float*)a->data, nullptr, xq, xd, (int)m, (int)k, 0.0f, skinny ? kActMfma : kActNatural};
     launch("prefill_rows_q8", dim3((unsigned)m), dim3(256), gemv_act_lds_host((int)k), s, r);
+    if (skinny) {
+      SgemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)out->data, nullptr, nullptr, nullptr,
+                  (int)m, (int)n, (int)k, (int)n, kActMfma};
+      const SgemmPlan p = sgemm_plan(b->wt, "store", (int)m, (int)n, cx.num_cus);
+      launch(p.name, dim3(p.grid), dim3(kSgemmThreads), 0, s, g);
+      return;
+    }
     PrefillGemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)out->data, nullptr,
                       nullptr, nullptr, (int)m, (int)n, (int)k, (int)n, gemm_group_m()};
     launch(std::string("gemm_") + wt_tag(b->wt) + "_store",

@@ -158,6 +158,34 @@ GemvPlan gemv_plan(int wt, const std::string& kind, int n, int k, int num_cus) {
   return p;
 }
 
+// Whether M rows run on the skinny GEMM rather than the 128 x 128-tile GEMM:
+// whole 128-element runs and up to 160 rows, beyond which its 16-row tiles'
+// work passes the time of the few tiles' serial block loops (8B widths at 130
+// rows, skinny / tile us: Q|K|V 36 / 106, O and down 61 / 249, gate|up 142 /
+// 157; its time grows by a ninth of that per 16 rows, the tile GEMM's by a
+// whole pass per 128).  LLMRS_PREFILL_SKINNY=0 keeps every GEMM on the tiles.
+bool sgemm_serves(size_t m, size_t k) {
+  const char* e = std::getenv("LLMRS_PREFILL_SKINNY");
+  return m <= 160 && k % 128 == 0 && !(e && *e == '0');
+}
+
+// Row tiles per workgroup (R = 1, 2 or 4 tiles of 16 rows; eight waves share
+// them): the most that still leave every CU two workgroups, since a
+// workgroup's rows share its activation loads (8B O and down at 23 rows: R = 1
+// 14.7 us, R = 2, 256 workgroups, 16.1); SwiGLU runs always span four.  The
+// grid deals eight row sets at a time, one per XCD, each over its token tiles.
+SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
+  const long nt = (m + 15) / 16;
+  int R = 4;
+  if (epi != "silu")
+    while (R > 1 && (n + 16 * R - 1) / (16 * R) * nt < 2 * num_cus) R /= 2;
+  const long rows = (n + 16 * R - 1) / (16 * R);
+  SgemmPlan p;
+  p.name = std::string("sgemm_") + wt_tag(wt) + "_" + epi + "_r" + std::to_string(R);
+  p.grid = (unsigned)(8 * nt * ((rows + 7) / 8));
+  return p;
+}
+
 // ---- allocator -------------------------------------------------------------
 void* Allocator::alloc(size_t bytes) {
   size_t sz = align_up(bytes ? bytes : 1, 256);

@@ -66,33 +66,49 @@ struct ArgmaxFinalArgs {
   int cap;
 };
 
-// Activation codes in the skinny GEMM's operand order (sgemm.hip).  Every
-// run of 4 blocks (128 elements) is stored as [4 lane groups][4 blocks][8
-// bytes]: lane group g's 8 bytes of a block are the elements its weight
-// dword multiplies - dword g of a device Q4 block holds elements 4g..4g+3 in
-// its low nibbles and 16+4g..16+4g+3 in its high ones (dwords g and g+4 of
-// a Q8 block the same elements) - so elements 4g..4g+3, then 16+4g..16+4g+3.
-// Aligned runs of 4 elements stay together.  Needs the row length a
-// multiple of 128.
+// Activation codes and scales in the skinny GEMM's operand order (sgemm.hip),
+// kActMfma: rows in tiles of 16 (buffers hold whole tiles), and a tile's run
+// of 4 blocks (128 elements) as [2 halves][4 lane groups][16 rows][16 bytes],
+// so that a wave's operand load is 1 KB of consecutive bytes in lane order.
+// Lane group g's 8 bytes of a block are the elements its weight dword
+// multiplies - dword g of a device Q4 block holds elements 4g..4g+3 in its
+// low nibbles and 16+4g..16+4g+3 in its high ones (dwords g and g+4 of a Q8
+// block the same elements) - and a half holds two blocks.  Aligned runs of 4
+// elements stay together.  Scales: [tile][block][16 rows].  A
+// row's element sits at act_row + act_offset, its block's scale at
+// act_scale_row + act_scale_offset.  Needs the row length K a multiple of 128.
 enum { kActNatural = 0, kActMfma = 1 };
 constexpr int act_offset(int k, int layout) {
   return layout == kActNatural ? k
-                               : ((k >> 5) >> 2) * 128 + ((k >> 5) & 3) * 8 + ((k & 31) >> 2 & 3) * 32 +
-                                     ((k & 31) >> 4) * 4 + (k & 3);
+                               : (k >> 7) * 2048 + ((k >> 6) & 1) * 1024 + ((k >> 2) & 3) * 256 + ((k >> 5) & 1) * 8 +
+                                     ((k >> 4) & 1) * 4 + (k & 3);
 }
+constexpr size_t act_row(size_t row, size_t K, int layout) {
+  return layout == kActNatural ? row * K : (row >> 4) * 16 * K + (row & 15) * 16;
+}
+constexpr int act_scale_offset(int b, int layout) {
+  return layout == kActNatural ? b : b * 16;
+}
+constexpr size_t act_scale_row(size_t row, size_t nb, int layout) {
+  return layout == kActNatural ? row * nb : (row >> 4) * 16 * nb + (row & 15);
+}
+// Rows an activation buffer of M rows holds, in either order.
+constexpr size_t act_rows(size_t M) { return (M + 15) / 16 * 16; }
 
-// Skinny GEMM of batched decode (sgemm.hip): Y[t][n] = sum_b isum_b(t, n) *
-// (d_w[n,b] * d_a[t,b]) over M <= 64 rows of Q8_0 activation codes (in the
-// operand order of the weight type) and an [N, K] quantised weight.
+// Skinny GEMM of short prompts and batched decode (sgemm.hip): Y[t][n] =
+// sum_b isum_b(t, n) * (d_w[n,b] * d_a[t,b]) over M rows of Q8_0 activation
+// codes (in the operand order kActMfma) and an [N, K] quantised weight, K a
+// multiple of 128.
+constexpr int kSgemmThreads = 512;
 struct SgemmArgs {
-  const int8_t* xq;      // [M][K] activation codes, act_offset order
-  const float* xd;       // [M][K/32] activation scales
+  const int8_t* xq;      // [M][K] activation codes, order kActMfma
+  const float* xd;       // [M][K/32] activation scales, order kActMfma
   const uint8_t* wq;     // weight codes [N][nb][B]
   const void* ws;        // weight scales [N][nb]
   float* y;              // [M][ldy] (STORE, RESID)
   const float* res;      // [M][N] residual (RESID; may alias y)
   int8_t* yq;            // SILU: [M][N/2] codes of m, in the order `layout`
-  float* yd;             // SILU: [M][N/64] scales of m
+  float* yd;             // SILU: [M][N/64] scales of m, in the order `layout`
   int M, N, K, ldy, layout;
 };
 
@@ -190,8 +206,8 @@ struct AttnArgs {
   unsigned long long* ts;  // profiling: 8 stage timestamps per item (null = off)
   // Batched decode (grid.z = sequences): sequence z's qkv, position, partials,
   // tickets and ctx rows follow sequence 0's at their natural strides, its
-  // K and V caches kv_batch_bytes after sequence 0's; ctx_q in the skinny
-  // GEMM's operand order ctx_layout (act_offset within the row).
+  // K and V caches kv_batch_bytes after sequence 0's; ctx_q and ctx_d in the
+  // operand order ctx_layout (act_row, act_offset).
   size_t kv_batch_bytes;
   int ctx_layout;
 };
@@ -285,8 +301,8 @@ constexpr size_t gemm_lds_bytes() {
 struct PrefillRowArgs {
   const float* x;        // [M][dim] input rows
   const float* w;        // [dim] RMSNorm weight (null: plain Q8_0)
-  int8_t* xq;            // [M][dim] codes (act_offset order `layout` within a row)
-  float* xd;             // [M][dim/32] scales
+  int8_t* xq;            // [M][dim] codes (operand order `layout`)
+  float* xd;             // [M][dim/32] scales (operand order `layout`)
   int M, dim;
   float eps;
   int layout;
@@ -314,7 +330,7 @@ struct PrefillAttnArgs {
   float* ctx_d;          // [M][nq*hd/32]
   int M, nq, nkv, max_seq, start_pos;
   float scale;           // fl(1 / fl(sqrt(hd)))
-  int ctx_layout;        // operand order of ctx_q within a row (act_offset)
+  int ctx_layout;        // operand order of ctx_q and ctx_d
 };
 
 // ints between the split tickets of two KV heads: each head's counter has a
@@ -325,8 +341,8 @@ constexpr int kTicketStride = 64;
 struct ExactNormArgs {
   const float* x;        // [rows][n] input rows
   const float* w;        // [n] RMSNorm weight
-  int8_t* xq;            // [rows][n] Q8_0 codes of the normed rows (act_offset order `layout`)
-  float* xd;             // [rows][n/32] their scales
+  int8_t* xq;            // [rows][n] Q8_0 codes of the normed rows (operand order `layout`)
+  float* xd;             // [rows][n/32] their scales (operand order `layout`)
   float* y;              // [rows][n] the normed rows (may be null)
   int n;
   float eps;

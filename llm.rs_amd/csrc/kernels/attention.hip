@@ -25,8 +25,8 @@ __device__ __forceinline__ AttnArgs sequence_args(const AttnArgs& a0) {
     a.part_ml += (size_t)z * a.nq * ml_stride(a.nsplit) * 2;
     a.counters += (size_t)z * a.nkv * kTicketStride;
     a.ctx += z * qd;
-    a.ctx_q += z * qd;
-    a.ctx_d += z * qd / 32;
+    a.ctx_q += act_row(z, qd, a.ctx_layout);
+    a.ctx_d += act_scale_row(z, qd / 32, a.ctx_layout);
     if (a.rope_now) a.rope_now += (size_t)z * HD;
     a.ts = nullptr;
   }

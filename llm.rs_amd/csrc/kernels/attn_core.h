@@ -596,7 +596,9 @@ __device__ __forceinline__ bool attn_item(const AttnArgs& a, int g, int split, i
       const int8_t q = amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(v[e], inv);
       dev_st8(a.ctx_q, act_offset((int)((size_t)h * HD + dd), a.ctx_layout), q);
     }
-    if ((lane % LPB) == 0) st_act<true>(a.ctx_d, ((size_t)h * HD + DPL * lane) / 32, amax == 0.0f ? 0.0f : d);
+    if ((lane % LPB) == 0)
+      st_act<true>(a.ctx_d, act_scale_offset((int)(((size_t)h * HD + DPL * lane) / 32), a.ctx_layout),
+                   amax == 0.0f ? 0.0f : d);
   }
   if (tid == 0) {
     if (loc) xcd_stu(a.counters, 4 * g * kTicketStride, 0u);

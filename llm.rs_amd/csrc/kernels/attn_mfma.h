@@ -597,7 +597,7 @@ __device__ __forceinline__ void attn_mfma_item(const AttnArgs& a, int pos, uint8
       a.ctx[e] = v[0];
       a.ctx_q[qo] = (int8_t)codes;
     }
-    if (lane % (32 / DPL) == 0) a.ctx_d[e / 32] = bmax == 0.0f ? 0.0f : d;
+    if (lane % (32 / DPL) == 0) a.ctx_d[act_scale_offset((int)(e / 32), a.ctx_layout)] = bmax == 0.0f ? 0.0f : d;
   }
   if (tid == 0) {  // every split has taken its ticket: the ticket restarts
     if (loc) xcd_stu(a.counters, 4 * g * kTicketStride, 0u);

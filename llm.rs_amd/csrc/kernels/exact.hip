@@ -209,7 +209,7 @@ __device__ __forceinline__ void norm_out(const NormRow& a, int i, float x, float
   float d;
   const int q = q8_group32(y, &d);
   a.xq[act_offset(i, a.layout)] = (int8_t)q;
-  if ((i & 31) == 0) a.xd[i >> 5] = d;
+  if ((i & 31) == 0) a.xd[act_scale_offset(i >> 5, a.layout)] = d;
   if (a.y) a.y[i] = y;
 }
 
@@ -235,7 +235,8 @@ __device__ __forceinline__ void norm_q8(const ExactNormArgs& args) {
   extern __shared__ __align__(16) float sq[];
   __shared__ FoldShared<kNW> sh;
   const size_t ro = (size_t)blockIdx.x * args.n;  // this workgroup's row
-  const NormRow a{args.x + ro, args.w, args.xq + ro, args.xd + ro / 32, args.y ? args.y + ro : nullptr,
+  const NormRow a{args.x + ro, args.w, args.xq + act_row(blockIdx.x, args.n, args.layout),
+                  args.xd + act_scale_row(blockIdx.x, args.n / 32, args.layout), args.y ? args.y + ro : nullptr,
                   args.n, args.layout, args.eps};
   switch (a.n) {
     case 2 * kNT: norm_q8_regs<2>(a, sq, sh); return;
@@ -823,8 +824,9 @@ __device__ __forceinline__ void attn_prefill(const PrefillAttnArgs& a) {
     if (a.ctx) a.ctx[(size_t)t * qd + e] = acc;
     float dq;
     const int q = q8_group32(acc, &dq);
-    a.ctx_q[(size_t)t * qd + act_offset(e, a.ctx_layout)] = (int8_t)q;
-    if ((tid & 31) == 0) a.ctx_d[(size_t)t * (qd / 32) + (e >> 5)] = dq;
+    a.ctx_q[act_row(t, qd, a.ctx_layout) + act_offset(e, a.ctx_layout)] = (int8_t)q;
+    if ((tid & 31) == 0)
+      a.ctx_d[act_scale_row(t, qd / 32, a.ctx_layout) + act_scale_offset(e >> 5, a.ctx_layout)] = dq;
   }
 }
 

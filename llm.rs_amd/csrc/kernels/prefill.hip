@@ -355,10 +355,12 @@ extern "C" __global__ __launch_bounds__(kThreads) void prefill_rows_q8(PrefillRo
     i32x4* dst = (i32x4*)(r.xq + (size_t)row * r.dim);
     for (int i = threadIdx.x; i < r.dim / 16; i += kThreads) dst[i] = src[i];
   } else {
-    int8_t* dst = r.xq + (size_t)row * r.dim;
-    for (int i = threadIdx.x; i < r.dim; i += kThreads) dst[act_offset(i, r.layout)] = s_q[i];
+    int8_t* dst = r.xq + act_row(row, r.dim, r.layout);
+    for (int i = 4 * threadIdx.x; i < r.dim; i += 4 * kThreads)  // aligned runs of 4 stay together
+      *(unsigned*)(dst + act_offset(i, r.layout)) = *(const unsigned*)(s_q + i);
   }
-  for (int b = threadIdx.x; b < nb; b += kThreads) r.xd[(size_t)row * nb + b] = s_d[b];
+  float* xd = r.xd + act_scale_row(row, nb, r.layout);
+  for (int b = threadIdx.x; b < nb; b += kThreads) xd[act_scale_offset(b, r.layout)] = s_d[b];
 }
 
 // RoPE of q and k (cpu.rs:326-357, per head, position start_pos + t) and the
@@ -548,10 +550,12 @@ __device__ __forceinline__ void attn_prefill_impl(const PrefillAttnArgs& a) {
 #pragma unroll
       for (int e = 0; e < DPT; ++e) {
         if (a.ctx) a.ctx[base + e] = v[e];
-        a.ctx_q[(size_t)t * qdim + act_offset(h * HD + DPT * ki + e, a.ctx_layout)] =
+        a.ctx_q[act_row(t, qdim, a.ctx_layout) + act_offset(h * HD + DPT * ki + e, a.ctx_layout)] =
             amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(v[e], inv);
       }
-      if ((ki % TPB) == 0) a.ctx_d[base / 32] = amax == 0.0f ? 0.0f : d;
+      if ((ki % TPB) == 0)
+        a.ctx_d[act_scale_row(t, qdim / 32, a.ctx_layout) +
+                act_scale_offset((h * HD + DPT * ki) / 32, a.ctx_layout)] = amax == 0.0f ? 0.0f : d;
     }
   }
 }
@@ -783,11 +787,13 @@ __device__ __forceinline__ void attn_prefill_mfma_impl(const PrefillAttnArgs& a)
             const int q8 = amax == 0.0f ? 0 : q8_code(v[4 * gq + c], inv);
             w |= ((unsigned)q8 & 0xFFu) << (8 * c);
           }
-          *(unsigned*)(a.ctx_q + (base - (size_t)h * HD) +
+          *(unsigned*)(a.ctx_q + act_row(myq, qdim, a.ctx_layout) +
                        act_offset(h * HD + 32 * d + 8 * gq + 4 * h2, a.ctx_layout)) = w;
           if (a.ctx) *(f32x4*)(a.ctx + e) = f32x4{v[4 * gq], v[4 * gq + 1], v[4 * gq + 2], v[4 * gq + 3]};
         }
-        if (h2 == 0) a.ctx_d[base / 32 + d] = amax == 0.0f ? 0.0f : dq;
+        if (h2 == 0)
+          a.ctx_d[act_scale_row(myq, qdim / 32, a.ctx_layout) + act_scale_offset(h * HD / 32 + d, a.ctx_layout)] =
+              amax == 0.0f ? 0.0f : dq;
       }
     }
   }

@@ -1,47 +1,52 @@
-// sgemm.hip - skinny GEMM of batched decode for gfx950.
+// sgemm.hip - skinny GEMM (short prompts, batched decode) for gfx950.
 //
 // Reference: the Q4/Q8 x Q8_0 block loop of CpuBackend::matmul_transposed
 // per activation row (cpu.rs:90-110; kernel_avx2 cpu.rs:888-941):
-// y[t][n] = sum over blocks b of fl(isum_b * fl(d_w[n,b] * d_a[t,b])), isum_b
-// the exact int32 dot of the block's weight and activation codes.
+// y[t][n] = (...((0 + isum_0 s_0) + isum_1 s_1) + ...), s_b = d_w[n,b] * d_a[t,b],
+// isum_b the exact int32 dot of the block's weight and activation codes.
+// Every output's terms are added in block order, so the results are
+// bit-identical to the reference's for the same activation codes.
 //
-// MI355X design: M <= 64 activation rows (the sequences of a batch) against
-// a weight streamed once.  One v_mfma_i32_16x16x32_i8 per block gives the 16
-// rows x 16 tokens of exact block sums, and one v_mfma_f32_16x16x1_4b_f32 per
-// four blocks every scale product d_w * d_a of the 16 x 16 tile as a single
-// IEEE product (lane 16 b + i supplies row / token i of block b; block b's
-// products sit in registers 4 b .. 4 b + 3 in the layout of the block sums);
-// the epilogue then multiplies and adds in f32 as the reference does.  Lane (r, g) of a wave (r = lane % 16, g = lane / 16) loads 16
-// bytes: one Q4 block of weight row r (four blocks per lane group), so each
-// load instruction reads 64 contiguous bytes of each of 16 rows; a 4x4 dword
-// transpose across the lane groups (v_permlane32_swap, v_permlane16_swap)
-// then gives lane group g dword g of each of the four blocks - its MFMA
-// operand (the nibbles unpacked to q - 8 in four instructions; the device
-// Q4 layout is the same for both Q4 storages, only their scales differ).
-// The activation codes are stored in the matching operand order
-// (act_offset), so a lane reads its four blocks' operands as 32 contiguous
-// bytes.
+// What bounds it: few rows leave few output tiles (N / 16 x M / 16 of them,
+// 256 for a 4096-row projection of up to 16 tokens on 256 CUs), so a wave
+// that walks a whole row of blocks alone has neither the bytes in flight nor
+// the issue slots to stream the weights.  Only the additions have an order:
+// the terms isum_b * s_b do not.  So a workgroup of eight waves takes 16 R
+// rows x 16 tokens (R = 1, 2, 4) and a wave the terms of 16 rows and an
+// eighth / quarter / half of each round of 64 / R blocks; the terms pass
+// through 64 KB of LDS, four blocks of one output per 16-byte chunk, and
+// every thread adds its own outputs' terms in block order.  The order thus
+// costs one dependent add per block (K / 32 of them) and no hand-over
+// between waves.
 //
-// Batched decode: a wave takes RT 16-row tiles, which share its activation
-// operands (the activation bytes a group loads are twice its weight bytes
-// per tile): two, or one for the residual projections, whose few rows would
-// leave too few workgroups.  A workgroup holds RS row sets of RT tiles and
-// splits the blocks of each over KP waves in contiguous parts, partial sums
-// added in part order.  STORE / RESID: one row set, KP = 4.  SILU: 64 rows
-// per workgroup - a run of 32 gate and 32 up rows, one row set each, KP = 2;
-// m = silu(gate) * up and its Q8_0 codes (one 32-element block per run) in
-// the operand order of the down projection.  (Same box, 8B: eight waves per
-// workgroup with twice the parts were slower at B = 16 and 64, e.g. the
-// SwiGLU launch 42.8 vs 39.7 us; plain instead of streaming weight loads
-// changed nothing.)
+// Per four blocks and 16 x 16 tile: one v_mfma_i32_16x16x32_i8 per block
+// gives its exact sums, one v_mfma_f32_16x16x1_4b_f32 every scale product
+// d_w * d_a as a single IEEE product (lane 16 b + i supplies row / token i of
+// block b; block b's products sit in registers 4 b .. 4 b + 3 in the layout
+// of the block sums).  A wave loads the eight blocks of a step from 16 rows as
+// they lie in memory, 128 contiguous bytes per row, and turns them through
+// its own LDS so that lane (r, g) (r = lane % 16, g = lane / 16) holds block
+// g of row r; a 4x4 dword transpose across the lane groups
+// (v_permlane32_swap, v_permlane16_swap) then gives lane group g dword g of
+// each of four blocks - its MFMA operand (Q4: the nibbles unpacked to q - 8;
+// Q8: dwords g and g + 4).  The activation codes are stored in the operand
+// order itself (act_offset), 1 KB of consecutive bytes per load.  Loads in
+// which neighbouring lanes read different rows bounded the kernel before: the
+// L1 serves one line per lane then, and the same kernel with row-strided
+// weight and activation loads took 34 us for the 8B gate|up at 16 rows
+// against 21.
 //
-// EXACT launches (prompt prefill) give each output row's blocks to one wave
-// in order, as the reference adds them, so the result is bit-identical to
-// the reference's for the same activation codes: STORE / RESID run one wave
-// (16 rows) per workgroup, SILU four (the run's 64 rows).
+// Workgroups are dealt to the XCDs so that the token tiles of one row set run
+// on one XCD back to back: the weights come from HBM about once and the other
+// token tiles read them from its L2.
 //
-// Each wave keeps PF groups of loads in flight (a ring of register sets, the
-// loop unrolled by PF so every set has a fixed place).
+// Measured (8B widths, us per launch at 16 rows, before -> now, where before
+// was one wave per 16 rows with row-strided loads): Q|K|V 12 -> 7.6, O and
+// down 14.5 -> 9.8, gate|up 35.7 -> 21.4 (66 MB of weights: 3.1 TB/s); exact
+// prompts of 23 rows: 15.1 -> 11.5, 30.5 -> 14.7, 55.5 -> 40; 37 rows: 29 ->
+// 15, 62 -> 19, 80 -> 52.  The rounds' phases (loads, products, LDS, adds)
+// overlap only across the two workgroups of a CU.
+
 #include "common.h"
 #include "exact_math.h"
 #include "gemv_core.h"
@@ -52,6 +57,15 @@ using namespace llmrs;
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kSgThreads = kSgemmThreads;   // eight waves
+constexpr int kSgWaves = kSgThreads / LLMRS_WAVE;
+constexpr int kStep = 8;                    // blocks of one wave per round
+
+template <int WT>
+__device__ __forceinline__ unsigned load_scale(const void* ws, size_t i) {
+  return WT == WT_Q4F ? ((const unsigned*)ws)[i] : ((const uint16_t*)ws)[i];
+}
 
 // q - 8 for four nibbles held one per byte (0..15): (v + 0x78) ^ 0x80 per
 // byte, no carry between bytes.
@@ -76,246 +90,228 @@ __device__ __forceinline__ void transpose4(unsigned x[4]) {
   x[3] = p[1];
 }
 
-// What one 128-element group needs in registers.
-template <int WT, int TT, int RT>
-struct Group {
-  u32x4 w[RT];          // Q4: this lane's block of each row tile (transposed after arrival)
-  unsigned w8[RT][4][2];  // Q8: dwords g and g + 4 of each block
-  unsigned dw[RT];       // raw scale of (row lane % 16, block lane / 16) per row tile
-  u32x4 x[TT][2];       // activation operands of 4 blocks, per token tile
-  float da[TT];         // scale of (token lane % 16, block lane / 16) per token tile
+// A wave's loads of eight blocks of 16 weight rows: the codes as they lie in
+// memory (lanes 8 i .. 8 i + 7 the 128 bytes of row i, or lanes 16 i .. of 256
+// bytes for Q8) and the scales of blocks g and 4 + g of row r.
+template <int WT>
+struct SgWeights {
+  static constexpr int WL = WT == WT_Q8H ? 4 : 2;  // 1 KB loads
+  u32x4 w[WL];
+  unsigned dw[2];                                  // raw
+};
+// And of 16 tokens: token r's operands and its scales of blocks g and 4 + g.
+struct SgTokens {
+  u32x4 x[2][2];  // [run of four blocks][half]
+  float da[2];
 };
 
-// Loads of group q for the wave's rows n0 .. n0 + 16 RT - 1.
-template <int WT, int TT, int RT>
-__device__ __forceinline__ void load_group(Group<WT, TT, RT>& G, const SgemmArgs& a, int q, int n0, int tok, int nb,
-                                           int g) {
+// Blocks b0 .. b0 + 7; runs of four past the row end clamped to its last one
+// (nb is a multiple of 4), never added; rows clamped to the last row.
+template <int WT>
+__device__ __forceinline__ void load_weights(SgWeights<WT>& G, const SgemmArgs& a, int b0, int row0, int nb, int lane) {
+  constexpr int BCH = WT == WT_Q8H ? 2 : 1;  // 16-byte chunks per block
+  constexpr int RCH = kStep * BCH;           // chunks of a row's eight blocks
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int wrow = min(n0 + 16 * rt + tok, a.N - 1);
-    if (WT == WT_Q8H) {
-      const unsigned* base = (const unsigned*)(a.wq + ((size_t)wrow * nb + 4 * q) * 32);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        G.w8[rt][j][0] = __builtin_nontemporal_load(base + 8 * j + g);
-        G.w8[rt][j][1] = __builtin_nontemporal_load(base + 8 * j + g + 4);
-      }
-    } else {
-      G.w[rt] = __builtin_nontemporal_load((const u32x4*)(a.wq + ((size_t)wrow * nb + 4 * q + g) * 16));
-    }
-    G.dw[rt] = load_wscale_raw<WT>(a.ws, (size_t)wrow * nb + 4 * q + g);
+  for (int j = 0; j < SgWeights<WT>::WL; ++j) {
+    const int q = LLMRS_WAVE * j + lane, c = q % RCH;
+    const int row = min(row0 + q / RCH, a.N - 1), blk = min(b0 + c / BCH, nb - 1);
+    G.w[j] = *(const u32x4*)(a.wq + ((size_t)row * nb + blk) * (16 * BCH) + 16 * (c % BCH));
   }
+  const size_t wi = (size_t)min(row0 + (lane & 15), a.N - 1) * nb + (lane >> 4);
 #pragma unroll
-  for (int tt = 0; tt < TT; ++tt) {
-    const int t = min(16 * tt + tok, a.M - 1);
-    const u32x4* xp = (const u32x4*)(a.xq + (size_t)t * a.K + (size_t)q * 128 + g * 32);
-    G.x[tt][0] = xp[0];
-    G.x[tt][1] = xp[1];
-    G.da[tt] = a.xd[(size_t)t * nb + 4 * q + g];
+  for (int u = 0; u < 2; ++u) G.dw[u] = load_scale<WT>(a.ws, wi + min(b0 + 4 * u, nb - 4));
+}
+__device__ __forceinline__ void load_tokens(SgTokens& G, const SgemmArgs& a, int b0, int tile, int nb, int lane) {
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int b = min(b0 + 4 * u, nb - 4);
+    const u32x4* p = (const u32x4*)(a.xq + (size_t)tile * 16 * a.K + (size_t)b * 512) + lane;
+    G.x[u][0] = p[0];
+    G.x[u][1] = p[LLMRS_WAVE];
+    G.da[u] = a.xd[(size_t)tile * 16 * nb + b * 16 + lane];
   }
 }
 
-// One group's MFMAs and epilogue into acc[rt][tt][i] (output row n0 + 16 rt
-// + 4 g + i, token 16 tt + tok).
-template <int WT, int TT, int RT>
-__device__ __forceinline__ void compute_group(Group<WT, TT, RT>& G, f32x4 (&acc)[RT][TT]) {
-  long op_a[RT][4];
+// The weights of a step through the wave's own LDS (1 KB per load), in which
+// the codes change from memory order (row, chunk) to one row per lane: chunk c
+// of row i sits at c ^ (i & 7) of its row, so that 16 rows' chunks spread over
+// the banks.
+template <int WT>
+__device__ __forceinline__ void stage_weights(const SgWeights<WT>& G, u32x4* stage, int lane) {
+  constexpr int RCH = kStep * (WT == WT_Q8H ? 2 : 1);
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    if (WT == WT_Q8H) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        op_a[rt][j] = (long)((unsigned long long)G.w8[rt][j][0] | ((unsigned long long)G.w8[rt][j][1] << 32));
-    } else {
-      unsigned wd[4] = {G.w[rt][0], G.w[rt][1], G.w[rt][2], G.w[rt][3]};
-      transpose4(wd);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const unsigned lo = nib_s8(wd[j] & 0x0F0F0F0Fu), hi = nib_s8((wd[j] >> 4) & 0x0F0F0F0Fu);
-        op_a[rt][j] = (long)((unsigned long long)lo | ((unsigned long long)hi << 32));
-      }
-    }
+  for (int j = 0; j < SgWeights<WT>::WL; ++j) {
+    const int q = LLMRS_WAVE * j + lane, i = q / RCH, c = q % RCH;
+    stage[i * RCH + (c ^ (i & 7))] = G.w[j];
   }
-  // Per token tile every MFMA first, then the epilogue: an MFMA result read
-  // right after its issue would stall the wave for the MFMA's latency.
-  float dw[RT];
+}
+
+// Four blocks' weights as MFMA operands (dwords lo[j], hi[j] of block j) and
+// the scale of block g.
+struct SgOperands {
+  unsigned lo[4], hi[4];
+  float dw;
+};
+template <int WT>
+__device__ __forceinline__ void unpack_weights(const SgWeights<WT>& G, const u32x4* stage, int u, int lane,
+                                               SgOperands& op) {
+  constexpr int BCH = WT == WT_Q8H ? 2 : 1, RCH = kStep * BCH;
+  const int r = lane & 15, g = lane >> 4;
+  op.dw = wscale<WT>(G.dw[u]);
+  const u32x4 w0 = stage[r * RCH + (((4 * u + g) * BCH) ^ (r & 7))];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) dw[rt] = wscale<WT>(G.dw[rt]);
+  for (int j = 0; j < 4; ++j) op.lo[j] = w0[j];
+  transpose4(op.lo);
+  if constexpr (WT == WT_Q8H) {
+    const u32x4 w1 = stage[r * RCH + (((4 * u + g) * BCH + 1) ^ (r & 7))];
 #pragma unroll
-  for (int tt = 0; tt < TT; ++tt) {
-    v16f sc[RT];  // sc[rt][4 j + i] = fl(d_w * d_a) of block j, row 4 g + i, token tok
-    i32x4 isum[RT][4];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) sc[rt] = __builtin_amdgcn_mfma_f32_16x16x1f32(dw[rt], G.da[tt], v16f{}, 0, 0, 0);
+    for (int j = 0; j < 4; ++j) op.hi[j] = w1[j];
+    transpose4(op.hi);
+  } else {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const unsigned b0 = G.x[tt][j >> 1][2 * (j & 1)], b1 = G.x[tt][j >> 1][2 * (j & 1) + 1];
-      const long op_b = (long)((unsigned long long)b0 | ((unsigned long long)b1 << 32));
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-        isum[rt][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(op_a[rt][j], op_b, i32x4{0, 0, 0, 0}, 0, 0, 0);
+      op.hi[j] = nib_s8((op.lo[j] >> 4) & 0x0F0F0F0Fu);
+      op.lo[j] = nib_s8(op.lo[j] & 0x0F0F0F0Fu);
     }
+  }
+}
+
+// Four blocks' terms isum_b * (d_w d_a) of a 16 x 16 tile, each operation
+// rounded as the reference rounds it: t[b][i] is row 4 g + i, token r of block
+// b.  Every MFMA is issued before the first result is read.
+__device__ __forceinline__ void block_terms(const SgOperands& op, const SgTokens& G, int u, float (&t)[4][4]) {
+  const v16f sc = __builtin_amdgcn_mfma_f32_16x16x1f32(op.dw, G.da[u], v16f{}, 0, 0, 0);
+  i32x4 isum[4];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
+  for (int j = 0; j < 4; ++j) {
+    const unsigned b0 = G.x[u][j >> 1][2 * (j & 1)], b1 = G.x[u][j >> 1][2 * (j & 1) + 1];
+    const long op_a = (long)((unsigned long long)op.lo[j] | ((unsigned long long)op.hi[j] << 32));
+    const long op_b = (long)((unsigned long long)b0 | ((unsigned long long)b1 << 32));
+    isum[j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(op_a, op_b, i32x4{0, 0, 0, 0}, 0, 0, 0);
+  }
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)  // cpu.rs:930-935
-          acc[rt][tt][i] = acc[rt][tt][i] + (float)isum[rt][j][i] * sc[rt][4 * j + i];
+    for (int i = 0; i < 4; ++i) t[j][i] = (float)isum[j][i] * sc[4 * j + i];
+}
+
+// Element 32 run + j of token t's SwiGLU product m (j = lane % 32: a 32-lane
+// group holds one Q8_0 block of m): the f32 value (test probes) and its code.
+__device__ __forceinline__ void swiglu_out(const SgemmArgs& a, int t, int run, int j, float m) {
+  float amax = fabsf(m);
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 32));
+  const float d = amax / 127.0f;
+  const float inv = amax == 0.0f ? 0.0f : 1.0f / d;
+  if (t < a.M) {
+    const int F = a.N / 2;
+    if (a.y) a.y[(size_t)t * a.ldy + 32 * run + j] = m;
+    a.yq[act_row(t, F, a.layout) + act_offset(32 * run + j, a.layout)] =
+        amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(m, inv);
+    if (j == 0) a.yd[act_scale_row(t, F / 32, a.layout) + act_scale_offset(run, a.layout)] = amax == 0.0f ? 0.0f : d;
   }
 }
 
-// Groups of loads in flight per wave (register sets of the ring).  Measured
-// on 8B batched decode: with one token tile the SwiGLU launch is fastest with
-// one group ahead (35.7 us against 37.6 with two and 39.5 with four), the
-// others with two (B = 16 step 3.35 ms with these depths, 3.63 with four
-// throughout, 4.09 with eight); the exact launches walk every block of a row
-// in one wave and keep deeper rings.
-template <int EPI, int TT, bool EXACT>
-constexpr int prefetch_depth() {
-  if (EXACT) return TT == 1 ? 4 : TT == 2 ? 3 : 2;
-  return TT == 1 && EPI == EPI_SILU ? 1 : 2;
-}
-
-// The rows' partial sums over groups [q0, q1) in group order, PF groups of
-// loads ahead (addresses past the range clamped to its last group).
-template <int WT, int TT, int RT, int PF>
-__device__ __forceinline__ void run_groups(const SgemmArgs& a, int q0, int q1, int n0, int tok, int nb, int g,
-                                           f32x4 (&acc)[RT][TT]) {
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) acc[rt][tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  // Wave-uniform bounds (they derive from the wave index): the loop and its
-  // tail test become scalar branches, which the memory counter is tracked
-  // through; a per-lane (exec-mask) loop would make every iteration wait for
-  // all outstanding loads, ring included.
-  q0 = __builtin_amdgcn_readfirstlane(q0);
-  q1 = __builtin_amdgcn_readfirstlane(q1);
-  if (q0 >= q1) return;
-  Group<WT, TT, RT> ring[PF];
-#pragma unroll
-  for (int s = 0; s < PF; ++s) load_group<WT, TT, RT>(ring[s], a, min(q0 + s, q1 - 1), n0, tok, nb, g);
-  // Whole rounds of PF groups without a branch (one block the scheduler can
-  // interleave), then the last partial round from the ring.
-  int q = q0;
-  for (; q + PF <= q1; q += PF) {
-#pragma unroll
-    for (int s = 0; s < PF; ++s) {
-      compute_group<WT, TT, RT>(ring[s], acc);
-      load_group<WT, TT, RT>(ring[s], a, min(q + s + PF, q1 - 1), n0, tok, nb, g);
-    }
-  }
-#pragma unroll
-  for (int s = 0; s < PF - 1; ++s)
-    if (q + s < q1) compute_group<WT, TT, RT>(ring[s], acc);
-}
-
-// Workgroup shape: RS row sets of RT 16-row tiles, each row set's blocks
-// split over KP waves (EXACT: KP = 1, every output's blocks in order in one
-// wave, as the reference adds them - bit-identical to it for the same
-// activation codes; prompt prefill).
-template <int EPI, bool EXACT, int KP>
-struct SgemmShape {
-  static constexpr int RT = EXACT || EPI == EPI_RESID ? 1 : 2;
-  static constexpr int RS = EPI == EPI_SILU ? 64 / (16 * RT) : 1;
-  static constexpr int WAVES = RS * KP;
-  static constexpr int THREADS = 64 * WAVES;
-  static_assert(!EXACT || KP == 1, "exact launches keep every output's blocks in one wave");
-};
-
-template <int WT, int EPI, int TT, bool EXACT, int KP>
+template <int WT, int EPI, int R>
 __device__ __forceinline__ void sgemm_impl(const SgemmArgs& a) {
-  typedef SgemmShape<EPI, EXACT, KP> S;
-  constexpr int RT = S::RT, RS = S::RS;
-  __shared__ f32x4 s_acc[S::WAVES][RT][TT][64];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int nb = a.K >> 5, ngroups = nb >> 2;
-  const int rs = w / KP, kp = w % KP;
-  f32x4 acc[RT][TT];
-  // row set rs: rows n0 .. n0 + 16 RT - 1 (SILU: the run's gate rows, then its up rows)
-  const int n0 = blockIdx.x * (16 * RT * RS) + 16 * RT * rs;
-  run_groups<WT, TT, RT, prefetch_depth<EPI, TT, EXACT>()>(a, kp * ngroups / KP, (kp + 1) * ngroups / KP, n0, r,
-                                                          nb, g, acc);
+  constexpr int KP = kSgWaves / R;            // waves that share a row tile's blocks
+  constexpr int ROUND = KP * kStep;           // blocks per round
+  constexpr int QUADS = ROUND / 4;
+  constexpr int OUT = R * 256;                // outputs of the workgroup
+  constexpr int PER = OUT > kSgThreads ? OUT / kSgThreads : 1;  // per adding thread
+  static_assert(EPI != EPI_SILU || R == 4, "SwiGLU: a run of 32 gate and 32 up rows per workgroup");
+  // four blocks' terms of output o = 256 rt + 64 i + lane (row 16 rt +
+  // 4 (lane / 16) + i, token lane % 16) at s_t[quad * OUT + o]
+  __shared__ f32x4 s_t[QUADS * OUT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4, rt = w % R, kp = w / R;
+  const int nb = a.K >> 5, nt = (a.M + 15) >> 4, nrow = (a.N + 16 * R - 1) / (16 * R);
+  const int slot = blockIdx.x >> 3, ty = slot % nt, tx = (slot / nt) * 8 + (blockIdx.x & 7);
+  if (tx >= nrow) return;
+  const int row0 = tx * 16 * R + 16 * rt;
 
-  if (EPI != EPI_SILU && EXACT) {
-    const int row0 = n0 + 4 * g;
+  float acc[PER];
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const int t = 16 * tt + r;
-      if (t < a.M) {
+  for (int p = 0; p < PER; ++p) acc[p] = 0.0f;
+  SgWeights<WT> W;
+  SgTokens X;
+  load_weights<WT>(W, a, kp * kStep, row0, nb, lane);
+  load_tokens(X, a, kp * kStep, ty, nb, lane);
+  for (int base = 0; base < nb; base += ROUND) {
+    if (base + kp * kStep < nb) {
+      u32x4* stage = (u32x4*)&s_t[2 * kp * OUT + rt * 256];  // the place of the wave's own terms
+      stage_weights<WT>(W, stage, lane);
+      SgOperands op[2];  // both read before the terms take the place
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = row0 + i;
-          if (row < a.N) {
-            float o = acc[0][tt][i];
-            if (EPI == EPI_RESID) o = o + a.res[(size_t)t * a.N + row];  // layer.rs:386,403
-            a.y[(size_t)t * a.ldy + row] = o;
-          }
-        }
+      for (int u = 0; u < 2; ++u) unpack_weights<WT>(W, stage, u, lane, op[u]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        float t[4][4];
+        block_terms(op[u], X, u, t);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s_t[(2 * kp + u) * OUT + rt * 256 + i * 64 + lane] = f32x4{t[0][i], t[1][i], t[2][i], t[3][i]};
       }
     }
-    return;
-  }
+    load_weights<WT>(W, a, base + ROUND + kp * kStep, row0, nb, lane);
+    load_tokens(X, a, base + ROUND + kp * kStep, ty, nb, lane);
+    __syncthreads();
+    if (OUT >= kSgThreads || tid < OUT) {  // cpu.rs:930-935, in block order
+      const int nq = min(QUADS, (nb - base) >> 2);
+      if (nq == QUADS) {
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
+        for (int q = 0; q < QUADS; ++q)
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) s_acc[w][rt][tt][lane] = acc[rt][tt];
-  __syncthreads();
-
-  if (EPI == EPI_SILU) {
-    // m = silu(gate) * up (layer.rs:72-79) for 8 tokens x 32 elements per
-    // pass; Q8_0 of the 32 elements of a token (one block of m)
-    const int run = blockIdx.x;
-    const int j = tid & 31;
-    // gate row j of the run: row set, row tile, lane group, register; the
-    // matching up row sits RS / 2 row sets later
-    const int gs = j / (16 * RT), rt = (j >> 4) % RT, gg = (j & 15) >> 2, ii = j & 3;
-    for (int t0 = tid >> 5; t0 < 16 * TT; t0 += S::THREADS / 32) {
-      const int tt = t0 >> 4, l = 16 * gg + (t0 & 15);
-      float gv = s_acc[gs * KP][rt][tt][l][ii], uv = s_acc[(RS / 2 + gs) * KP][rt][tt][l][ii];
+          for (int p = 0; p < PER; ++p) {
+            const f32x4 v = s_t[q * OUT + p * kSgThreads + tid];
+            acc[p] = acc[p] + v[0];
+            acc[p] = acc[p] + v[1];
+            acc[p] = acc[p] + v[2];
+            acc[p] = acc[p] + v[3];
+          }
+      } else {
+        for (int q = 0; q < nq; ++q)
 #pragma unroll
-      for (int k = 1; k < KP; ++k) {
-        gv = gv + s_acc[gs * KP + k][rt][tt][l][ii];
-        uv = uv + s_acc[(RS / 2 + gs) * KP + k][rt][tt][l][ii];
-      }
-      const float mv = (gv / (1.0f + exact_expf(-gv))) * uv;  // glibc expf (exact_math.h)
-      float amax = fabsf(mv);
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 32));
-      const float d = amax / 127.0f;
-      const float inv = amax == 0.0f ? 0.0f : 1.0f / d;
-      if (t0 < a.M) {
-        const int F = a.N / 2;
-        if (a.y) a.y[(size_t)t0 * a.ldy + 32 * run + j] = mv;  // the f32 product (test probes)
-        a.yq[(size_t)t0 * F + act_offset(32 * run + j, a.layout)] =
-            amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(mv, inv);
-        if (j == 0) a.yd[(size_t)t0 * (F / 32) + run] = amax == 0.0f ? 0.0f : d;
+          for (int p = 0; p < PER; ++p) {
+            const f32x4 v = s_t[q * OUT + p * kSgThreads + tid];
+            acc[p] = acc[p] + v[0];
+            acc[p] = acc[p] + v[1];
+            acc[p] = acc[p] + v[2];
+            acc[p] = acc[p] + v[3];
+          }
       }
     }
-    return;
+    __syncthreads();
   }
-  if (w != 0) return;
+
+  float* s_o = (float*)s_t;
+  if constexpr (EPI == EPI_SILU) {
+    // outputs tid and tid + 512 of a thread are a gate row and its up row
+    // (layer.rs:72-79); m by token into LDS, then Q8_0 of each token's run
+    const float gv = acc[0], uv = acc[PER - 1];
+    const float mv = (gv / (1.0f + exact_expf(-gv))) * uv;  // glibc expf (exact_math.h)
+    s_o[r * 33 + 16 * (tid >> 8) + 4 * g + ((tid >> 6) & 3)] = mv;
+    __syncthreads();
+    swiglu_out(a, 16 * ty + (tid >> 5), tx, tid & 31, s_o[(tid >> 5) * 33 + (tid & 31)]);
+  } else {
+    // rows of one token side by side, for whole-line stores
+    constexpr int LD = 16 * R + 1;
+    if (OUT >= kSgThreads || tid < OUT) {
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int row0 = n0 + 16 * rt + 4 * g;
+      for (int p = 0; p < PER; ++p) {
+        const int o = p * kSgThreads + tid;
+        s_o[r * LD + 16 * (o >> 8) + 4 * g + ((o >> 6) & 3)] = acc[p];
+      }
+    }
+    __syncthreads();
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const int t = 16 * tt + r;
-      f32x4 v = s_acc[0][rt][tt][lane];
-#pragma unroll
-      for (int k = 1; k < KP; ++k) v = v + s_acc[k][rt][tt][lane];
-      if (t < a.M) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = row0 + i;
-          if (row < a.N) {
-            float o = v[i];
-            if (EPI == EPI_RESID) o = o + a.res[(size_t)t * a.N + row];  // layer.rs:386,403
-            a.y[(size_t)t * a.ldy + row] = o;
-          }
-        }
+    for (int p = 0; p < PER; ++p) {
+      const int o = p * kSgThreads + tid, t = 16 * ty + o / (16 * R), n = tx * 16 * R + o % (16 * R);
+      if (o < OUT && t < a.M && n < a.N) {
+        float v = s_o[(o / (16 * R)) * LD + o % (16 * R)];
+        if (EPI == EPI_RESID) v = v + a.res[(size_t)t * a.N + n];  // layer.rs:386,403
+        a.y[(size_t)t * a.ldy + n] = v;
       }
     }
   }
@@ -323,24 +319,17 @@ __device__ __forceinline__ void sgemm_impl(const SgemmArgs& a) {
 
 }  // namespace
 
-// Kernels: sgemm_<weights>_<epilogue>_t<token tiles>[_exact].
-#define LLMRS_SGEMM(name, WT, EPI, TT, EXACT, KP)                                               \
-  extern "C" __global__ __launch_bounds__((SgemmShape<EPI, EXACT, KP>::THREADS)) void name(SgemmArgs a) { \
-    sgemm_impl<WT, EPI, TT, EXACT, KP>(a);                                                        \
-  }
-#define LLMRS_SGEMM_TILES(tag, WT, EPI, KP)                            \
-  LLMRS_SGEMM(sgemm_##tag##_t1, WT, EPI, 1, false, KP)                 \
-  LLMRS_SGEMM(sgemm_##tag##_t2, WT, EPI, 2, false, KP)                 \
-  LLMRS_SGEMM(sgemm_##tag##_t4, WT, EPI, 4, false, KP)                 \
-  LLMRS_SGEMM(sgemm_##tag##_t1_exact, WT, EPI, 1, true, 1)             \
-  LLMRS_SGEMM(sgemm_##tag##_t2_exact, WT, EPI, 2, true, 1)             \
-  LLMRS_SGEMM(sgemm_##tag##_t4_exact, WT, EPI, 4, true, 1)
-LLMRS_SGEMM_TILES(q4h_store, WT_Q4H, EPI_STORE, 4)
-LLMRS_SGEMM_TILES(q4h_resid, WT_Q4H, EPI_RESID, 4)
-LLMRS_SGEMM_TILES(q4h_silu, WT_Q4H, EPI_SILU, 2)
-LLMRS_SGEMM_TILES(q4f_store, WT_Q4F, EPI_STORE, 4)
-LLMRS_SGEMM_TILES(q4f_resid, WT_Q4F, EPI_RESID, 4)
-LLMRS_SGEMM_TILES(q4f_silu, WT_Q4F, EPI_SILU, 2)
-LLMRS_SGEMM_TILES(q8h_store, WT_Q8H, EPI_STORE, 4)
-LLMRS_SGEMM_TILES(q8h_resid, WT_Q8H, EPI_RESID, 4)
-LLMRS_SGEMM_TILES(q8h_silu, WT_Q8H, EPI_SILU, 2)
+// Kernels: sgemm_<weights>_<epilogue>_r<row tiles per workgroup>.
+#define LLMRS_SGEMM(name, WT, EPI, R) \
+  extern "C" __global__ __launch_bounds__(kSgThreads, 4) void name(SgemmArgs a) { sgemm_impl<WT, EPI, R>(a); }
+#define LLMRS_SGEMM_WT(tag, WT)                      \
+  LLMRS_SGEMM(sgemm_##tag##_store_r1, WT, EPI_STORE, 1) \
+  LLMRS_SGEMM(sgemm_##tag##_store_r2, WT, EPI_STORE, 2) \
+  LLMRS_SGEMM(sgemm_##tag##_store_r4, WT, EPI_STORE, 4) \
+  LLMRS_SGEMM(sgemm_##tag##_resid_r1, WT, EPI_RESID, 1) \
+  LLMRS_SGEMM(sgemm_##tag##_resid_r2, WT, EPI_RESID, 2) \
+  LLMRS_SGEMM(sgemm_##tag##_resid_r4, WT, EPI_RESID, 4) \
+  LLMRS_SGEMM(sgemm_##tag##_silu_r4, WT, EPI_SILU, 4)
+LLMRS_SGEMM_WT(q4h, WT_Q4H)
+LLMRS_SGEMM_WT(q4f, WT_Q4F)
+LLMRS_SGEMM_WT(q8h, WT_Q8H)
