@@ -5,6 +5,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <functional>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <stdexcept>
@@ -77,10 +78,18 @@ struct Context {
   int num_cus = 0;
   void* noalloc_scratch = nullptr;  // device address of the scratch on `device`
   std::string noalloc_error;        // why it is null
+  uint8_t* host_out = nullptr;      // pinned: what fetch brings back (kFetchBytes + 64)
   std::vector<hipModule_t> modules;
   std::map<std::string, KernelInfo> kernels;
   Allocator alloc;
 };
+
+// Largest copy that goes through the pinned buffer; larger ones are left to
+// the runtime (2 MB: 134 us either way, most of it the copy to the caller).
+constexpr size_t kFetchBytes = (size_t)1 << 20;
+// Waits for the stream and brings `bytes` (a multiple of 4) of device memory
+// to dst, and the ints at the device addresses `ints` (up to four) to `out`.
+void fetch(void* dst, const void* src, size_t bytes, std::initializer_list<const int*> ints = {}, int* out = nullptr);
 
 Context& ctx();  // fails with LLMRS_E_NOINIT before llmrs_init
 std::recursive_mutex& api_mutex();

@@ -846,7 +846,7 @@ void enqueue_prefill(llmrs_model* m, Launcher& L, size_t start, int M, bool head
 
 bool prefill_enabled() { return env_int("LLMRS_PREFILL", 1) != 0; }
 
-void set_state(llmrs_model* m, size_t pos, int n_prompt);
+void set_state(llmrs_model* m, size_t pos, int n_prompt, const int* pf_start = nullptr);
 
 // Runs rows [start, start+n) through the prefill kernels in chunks; the last
 // chunk ends with the lm_head and greedy step, leaving the device position
@@ -866,8 +866,7 @@ void run_prefill(llmrs_model* m, size_t start, size_t n, int n_prompt, bool writ
       const int M = (int)std::min<size_t>(m->pf_cap, n - done);
       const bool last = done + M == n;
       const int s0 = (int)(start + done);
-      LLMRS_HIP(hipMemcpyAsync(m->pf_start, &s0, sizeof(int), hipMemcpyHostToDevice, ctx().stream));
-      set_state(m, start + done + M - 1, n_prompt);  // synchronises the stream
+      set_state(m, start + done + M - 1, n_prompt, &s0);
       Launcher L{ctx().stream};
       enqueue_prefill(m, L, start + done, M, last, write_logits && last, tdev, kcs, vcs, exact);
       if (trace) {
@@ -896,10 +895,15 @@ void check_ready(const llmrs_model* m) {
                   "layer " + std::to_string(i) + " weights incomplete");
 }
 
+// The device's error flag: read now, or (e) already brought back.
+void check_err(llmrs_model* m, int e);
 void check_err(llmrs_model* m) {
   int e = 0;
-  LLMRS_HIP(hipMemcpyAsync(&e, m->err, sizeof(int), hipMemcpyDeviceToHost, ctx().stream));
-  LLMRS_HIP(hipStreamSynchronize(ctx().stream));
+  fetch(nullptr, nullptr, 0, {m->err}, &e);
+  check_err(m, e);
+}
+
+void check_err(llmrs_model* m, int e) {
   if (e) {
     int zero = 0;
     LLMRS_HIP(hipMemcpyAsync(m->err, &zero, sizeof(int), hipMemcpyHostToDevice, ctx().stream));
@@ -908,21 +912,35 @@ void check_err(llmrs_model* m) {
   }
 }
 
-void set_state(llmrs_model* m, size_t pos, int n_prompt) {
-  int v[3] = {(int)pos, n_prompt, 0};
-  LLMRS_HIP(hipMemcpyAsync(m->pos, &v[0], sizeof(int), hipMemcpyHostToDevice, ctx().stream));
-  LLMRS_HIP(hipMemcpyAsync(m->n_prompt, &v[1], sizeof(int), hipMemcpyHostToDevice, ctx().stream));
-  LLMRS_HIP(hipMemcpyAsync(m->stopped, &v[2], sizeof(int), hipMemcpyHostToDevice, ctx().stream));
-  LLMRS_HIP(hipStreamSynchronize(ctx().stream));
+void set_state(llmrs_model* m, size_t pos, int n_prompt, const int* pf_start) {
+  StateArgs a{};
+  a.pos = m->pos;
+  a.n_prompt = m->n_prompt;
+  a.stopped = m->stopped;
+  a.v_pos = (int)pos;
+  a.v_n_prompt = n_prompt;
+  if (pf_start) {
+    a.pf_start = m->pf_start;
+    a.v_pf_start = *pf_start;
+  }
+  launch("set_state", dim3(1), dim3(256), 0, ctx().stream, a);
 }
 
 void upload_tokens(llmrs_model* m, size_t pos0, const int32_t* ids, size_t n) {
   for (size_t i = 0; i < n; ++i)
     LLMRS_REQUIRE(ids[i] >= 0 && ids[i] < m->c.vocab, LLMRS_E_RANGE,
                   "token id out of range at index " + std::to_string(i));
-  LLMRS_HIP(hipMemcpyAsync(m->tokens + pos0, ids, n * sizeof(int32_t), hipMemcpyHostToDevice,
-                           ctx().stream));
-  LLMRS_HIP(hipStreamSynchronize(ctx().stream));
+  if (n > (size_t)kStateTokens) {
+    LLMRS_HIP(hipMemcpyAsync(m->tokens + pos0, ids, n * sizeof(int32_t), hipMemcpyHostToDevice,
+                             ctx().stream));
+    LLMRS_HIP(hipStreamSynchronize(ctx().stream));
+    return;
+  }
+  StateArgs a{};
+  a.tokens = m->tokens + pos0;
+  a.n = (int)n;
+  std::memcpy(a.tok, ids, n * sizeof(int32_t));
+  launch("set_state", dim3(1), dim3(256), 0, ctx().stream, a);
 }
 
 // One decode position through the captured graph (captured on first use).
@@ -1344,11 +1362,10 @@ int llmrs_model_forward(llmrs_model* m, const int32_t* tokens, size_t n, size_t 
         LLMRS_HIP(hipStreamSynchronize(s));
       }
     }
-    if (logits)
-      LLMRS_HIP(hipMemcpyAsync(logits, m->logits, m->c.vocab * sizeof(float), hipMemcpyDeviceToHost, s));
-    if (next) LLMRS_HIP(hipMemcpyAsync(next, m->gen + start_pos + n, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    LLMRS_HIP(hipStreamSynchronize(s));
-    check_err(m);
+    int v[2] = {0, 0};
+    fetch(logits, m->logits, logits ? m->c.vocab * sizeof(float) : 0, {m->err, m->gen + start_pos + n}, v);
+    check_err(m, v[0]);
+    if (next) *next = v[1];
     m->host_pos = start_pos + n;
     m->begun = false;
   });
@@ -1361,11 +1378,11 @@ int llmrs_model_begin_at(llmrs_model* m, const int32_t* prompt, size_t n_prompt,
     LLMRS_REQUIRE(start_pos + n_prompt <= (size_t)m->c.max_seq, LLMRS_E_RANGE, "prompt beyond max_seq");
     const size_t end = start_pos + n_prompt;
     upload_tokens(m, start_pos, prompt, n_prompt);
-    set_state(m, start_pos, (int)end);
     m->host_n_prompt = (int)end;
     if (n_prompt > 1 && prefill_enabled()) {
       run_prefill(m, start_pos, n_prompt, (int)end, false, nullptr);
     } else {
+      set_state(m, start_pos, (int)end);
       for (size_t p = start_pos; p < end; ++p) {
         m->host_pos = p;
         replay_step(m);
@@ -1395,9 +1412,9 @@ int llmrs_model_tokens(llmrs_model* m, int32_t* out, size_t count) {
   return guard([&] {
     LLMRS_REQUIRE(m && out, LLMRS_E_INVALID, "null argument");
     LLMRS_REQUIRE(count <= m->host_pos + 1, LLMRS_E_RANGE, "more tokens requested than produced");
-    LLMRS_HIP(hipMemcpyAsync(out, m->tokens, count * sizeof(int32_t), hipMemcpyDeviceToHost, ctx().stream));
-    LLMRS_HIP(hipStreamSynchronize(ctx().stream));
-    check_err(m);
+    int e = 0;
+    fetch(out, m->tokens, count * sizeof(int32_t), {m->err}, &e);
+    check_err(m, e);
   });
 }
 
@@ -1425,9 +1442,7 @@ int llmrs_model_produced(llmrs_model* m, size_t* n, int32_t* stopped) {
   return guard([&] {
     LLMRS_REQUIRE(m && m->begun, LLMRS_E_INVALID, "llmrs_model_begin has not been called");
     int v[2] = {0, 0};
-    LLMRS_HIP(hipMemcpyAsync(&v[0], m->pos, sizeof(int), hipMemcpyDeviceToHost, ctx().stream));
-    LLMRS_HIP(hipMemcpyAsync(&v[1], m->stopped, sizeof(int), hipMemcpyDeviceToHost, ctx().stream));
-    LLMRS_HIP(hipStreamSynchronize(ctx().stream));
+    fetch(nullptr, nullptr, 0, {m->pos, m->stopped}, v);
     // the device position is that of the last token produced (the prompt's
     // last before any)
     if (n) *n = (size_t)std::max(0, v[0] + 1 - m->host_n_prompt);
@@ -1615,8 +1630,7 @@ int llmrs_model_profile_prefill(llmrs_model* m, const int32_t* tokens, size_t n,
     LLMRS_REQUIRE(n <= (size_t)m->pf_cap, LLMRS_E_RANGE, "more rows than one prefill chunk");
     upload_tokens(m, start_pos, tokens, n);
     const int s0 = (int)start_pos;
-    LLMRS_HIP(hipMemcpyAsync(m->pf_start, &s0, sizeof(int), hipMemcpyHostToDevice, ctx().stream));
-    set_state(m, start_pos + n - 1, INT_MAX);
+    set_state(m, start_pos + n - 1, INT_MAX, &s0);
     count = profile_launches(
         [&](Launcher& L) { enqueue_prefill(m, L, start_pos, (int)n, true, false, nullptr, nullptr, nullptr, m->exact); },
         names, ms,
@@ -2194,7 +2208,6 @@ int llmrs_batch_begin(llmrs_batch* b, int32_t slot, const int32_t* prompt, size_
     // the prompt through the prefill kernels into the slot's cache, then the
     // lm_head and greedy step of its last row, on the model's own buffers
     upload_tokens(m, 0, prompt, n_prompt);
-    set_state(m, 0, (int)n_prompt);
     std::vector<void*> kcs(b->kc.size()), vcs(b->vc.size());
     for (size_t li = 0; li < kcs.size(); ++li) {
       kcs[li] = (uint8_t*)b->kc[li] + (size_t)slot * b->kv_bytes;
@@ -2203,14 +2216,10 @@ int llmrs_batch_begin(llmrs_batch* b, int32_t slot, const int32_t* prompt, size_
     run_prefill(m, 0, n_prompt, (int)n_prompt, false, nullptr, kcs.data(), vcs.data());
     m->begun = false;  // the model's own sequence state was used as scratch
     m->host_pos = n_prompt;
-    hipStream_t s = ctx().stream;
-    const int p = (int)n_prompt;
-    LLMRS_HIP(hipMemcpyAsync(b->tokens + (size_t)slot * b->cap, m->tokens, (n_prompt + 1) * sizeof(int32_t),
-                             hipMemcpyDeviceToDevice, s));
-    LLMRS_HIP(hipMemcpyAsync(b->gen + (size_t)slot * b->cap, m->gen, (n_prompt + 1) * sizeof(int32_t),
-                             hipMemcpyDeviceToDevice, s));
-    LLMRS_HIP(hipMemcpyAsync(b->pos + slot, &p, sizeof(int), hipMemcpyHostToDevice, s));
-    LLMRS_HIP(hipStreamSynchronize(s));
+    // the greedy step has left the model's position at the prompt's end
+    const size_t at = (size_t)slot * b->cap;
+    AdoptArgs ad{m->tokens, m->gen, m->pos, b->tokens + at, b->gen + at, b->pos + slot, (int)n_prompt + 1};
+    launch("batch_adopt", dim3(1), dim3(256), 0, ctx().stream, ad);
     check_err(m);
     b->host_pos[slot] = n_prompt;
     b->begun[slot] = 1;
@@ -2235,19 +2244,16 @@ int llmrs_batch_tokens(llmrs_batch* b, int32_t slot, int32_t* out, size_t count)
     LLMRS_REQUIRE(b && out, LLMRS_E_INVALID, "null argument");
     LLMRS_REQUIRE(slot >= 0 && slot < b->B, LLMRS_E_RANGE, "slot out of range");
     LLMRS_REQUIRE(count <= b->host_pos[slot] + 1, LLMRS_E_RANGE, "more tokens requested than produced");
-    LLMRS_HIP(hipMemcpyAsync(out, b->tokens + (size_t)slot * b->cap, count * sizeof(int32_t),
-                             hipMemcpyDeviceToHost, ctx().stream));
-    LLMRS_HIP(hipStreamSynchronize(ctx().stream));
-    check_err(b->m);
+    int e = 0;
+    fetch(out, b->tokens + (size_t)slot * b->cap, count * sizeof(int32_t), {b->m->err}, &e);
+    check_err(b->m, e);
   });
 }
 
 int llmrs_batch_logits(llmrs_batch* b, float* out) {
   return guard([&] {
     LLMRS_REQUIRE(b && out, LLMRS_E_INVALID, "null argument");
-    LLMRS_HIP(hipMemcpyAsync(out, b->logits, (size_t)b->B * b->m->c.vocab * sizeof(float), hipMemcpyDeviceToHost,
-                             ctx().stream));
-    LLMRS_HIP(hipStreamSynchronize(ctx().stream));
+    fetch(out, b->logits, (size_t)b->B * b->m->c.vocab * sizeof(float));
   });
 }
 

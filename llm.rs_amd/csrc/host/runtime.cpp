@@ -7,6 +7,7 @@
 #include <cstring>
 #include <filesystem>
 #include <functional>
+#include <initializer_list>
 #include <thread>
 
 #include "../kernel_args.h"
@@ -51,9 +52,9 @@ hipFunction_t kernel(const std::string& name, dim3 block) {
         it = c.kernels.emplace(name, k).first;
         break;
       }
+      (void)hipGetLastError();  // not in this module
     }
     if (it == c.kernels.end()) {
-      (void)hipGetLastError();
       fail(LLMRS_E_MODULE, "kernel not found in any loaded hsaco: " + name);
     }
   }
@@ -62,6 +63,25 @@ hipFunction_t kernel(const std::string& name, dim3 block) {
                 name + ": " + std::to_string(threads) + " threads per workgroup, compiled for at most " +
                     std::to_string(it->second.max_threads));
   return it->second.f;
+}
+
+void fetch(void* dst, const void* src, size_t bytes, std::initializer_list<const int*> ints, int* out) {
+  Context& c = ctx();
+  if (bytes > kFetchBytes) {
+    LLMRS_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
+    bytes = 0;
+  }
+  int* host_ints = (int*)(c.host_out + kFetchBytes);
+  if (bytes || ints.size()) {
+    PublishArgs a{src, c.host_out, bytes, {}, host_ints};
+    size_t i = 0;
+    for (const int* p : ints) a.ints[i++] = p;
+    const size_t wgs = (bytes / 16 + 255) / 256;
+    launch("publish", dim3((unsigned)std::max<size_t>(1, std::min<size_t>(wgs, 256))), dim3(256), 0, c.stream, a);
+  }
+  LLMRS_HIP(hipStreamSynchronize(c.stream));
+  if (bytes) std::memcpy(dst, c.host_out, bytes);
+  if (ints.size()) std::memcpy(out, host_ints, ints.size() * sizeof(int));
 }
 
 bool xcd_dealt_mod8(unsigned gx, unsigned gy) {
@@ -341,6 +361,7 @@ int llmrs_init(int device_ordinal, const char* hsaco_dir) {
       LLMRS_HIP(hipGetDeviceProperties(&prop, device_ordinal));
       c->num_cus = prop.multiProcessorCount;
       LLMRS_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+      LLMRS_HIP(hipHostMalloc((void**)&c->host_out, kFetchBytes + 64, hipHostMallocDefault));
       // the no-allocation entry point's scratch, resolved with the device
       // current; a failure is reported by that entry point, not by init
       try {
@@ -362,6 +383,7 @@ int llmrs_init(int device_ordinal, const char* hsaco_dir) {
     } catch (...) {
       for (hipModule_t m : c->modules) (void)hipModuleUnload(m);
       if (c->stream) (void)hipStreamDestroy(c->stream);
+      if (c->host_out) (void)hipHostFree(c->host_out);
       delete c;
       throw;
     }
@@ -376,6 +398,7 @@ int llmrs_shutdown(void) {
     g_ctx->alloc.trim();
     for (hipModule_t m : g_ctx->modules) (void)hipModuleUnload(m);
     (void)hipStreamDestroy(g_ctx->stream);
+    (void)hipHostFree(g_ctx->host_out);
     delete g_ctx;
     g_ctx = nullptr;
   });

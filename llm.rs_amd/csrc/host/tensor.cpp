@@ -132,10 +132,7 @@ int llmrs_tensor_download(const llmrs_tensor* t, float* out, size_t count) {
     require_f32(t, "download");
     LLMRS_REQUIRE(count == t->numel(), LLMRS_E_INVALID, "download count != numel");
     LLMRS_REQUIRE(out || !count, LLMRS_E_INVALID, "out is null");
-    if (count)
-      LLMRS_HIP(hipMemcpyAsync(out, t->data, count * sizeof(float), hipMemcpyDeviceToHost,
-                               ctx().stream));
-    LLMRS_HIP(hipStreamSynchronize(ctx().stream));
+    fetch(out, t->data, count * sizeof(float));
   });
 }
 

@@ -212,6 +212,42 @@ struct AttnArgs {
   int ctx_layout;
 };
 
+// Sequence state set from the host (ops.hip: set_state): values and up to
+// kStateTokens ids travel in the launch's own arguments, so the call returns
+// without waiting and nothing of the caller's is read later.
+constexpr int kStateTokens = 512;
+struct StateArgs {
+  int* tokens;      // ids tok[0..n) go here (n may be 0)
+  int* pos;         // null: the four values stay as they are
+  int* n_prompt;
+  int* stopped;
+  int* pf_start;    // null: not set
+  int n, v_pos, v_n_prompt, v_pf_start;
+  int tok[kStateTokens];
+};
+
+// A batch slot takes over the sequence the model has just begun (ops.hip:
+// batch_adopt): ids and produced ids of positions 0 .. n-1, and the position.
+struct AdoptArgs {
+  const int* tokens;
+  const int* gen;
+  const int* pos;
+  int* to_tokens;
+  int* to_gen;
+  int* to_pos;
+  int n;
+};
+
+// Device memory to mapped host memory (ops.hip: publish): `bytes` of src (a
+// multiple of 4; whole 16-byte words where src allows) and up to four ints.
+struct PublishArgs {
+  const void* src;
+  void* dst;
+  size_t bytes;
+  const int* ints[4];  // null: skipped
+  int* out;
+};
+
 // Elementwise trait operators (ops.hip).
 struct EwArgs {
   float* a;          // in/out

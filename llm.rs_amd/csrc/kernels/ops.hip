@@ -220,6 +220,38 @@ extern "C" __global__ __launch_bounds__(kEmbedThreads) void embed_gather(EmbedAr
   }
 }
 
+// Small transfers as kernels.  What bounds them is the runtime's path, not the
+// bytes: copying to or from pageable host memory stages and waits (measured,
+// with the wait for the stream: 4 bytes in 13 us, out 20 us, 8 KB out 26 us,
+// 512 KB out 45 us).  One launch on the same stream with the values in its
+// arguments, or storing straight into mapped host memory (8 KB 12 us, 512 KB
+// 21 us, of which 11 us are the launch and the wait), replaces them.
+extern "C" __global__ __launch_bounds__(256) void set_state(StateArgs a) {
+  for (int i = threadIdx.x; i < a.n; i += 256) a.tokens[i] = a.tok[i];
+  if (threadIdx.x == 0) {
+    if (a.pos) {
+      *a.pos = a.v_pos;
+      *a.n_prompt = a.v_n_prompt;
+      *a.stopped = 0;
+    }
+    if (a.pf_start) *a.pf_start = a.v_pf_start;
+  }
+}
+extern "C" __global__ __launch_bounds__(256) void batch_adopt(AdoptArgs a) {
+  for (int i = threadIdx.x; i < a.n; i += 256) {
+    a.to_tokens[i] = a.tokens[i];
+    a.to_gen[i] = a.gen[i];
+  }
+  if (threadIdx.x == 0) *a.to_pos = *a.pos;
+}
+extern "C" __global__ __launch_bounds__(256) void publish(PublishArgs a) {
+  const size_t t = blockIdx.x * (size_t)256 + threadIdx.x, step = gridDim.x * (size_t)256;
+  const size_t n16 = ((size_t)a.src & 15) == 0 ? a.bytes / 16 : 0;
+  for (size_t i = t; i < n16; i += step) ((uint4*)a.dst)[i] = ((const uint4*)a.src)[i];
+  for (size_t i = 4 * n16 + t; i < a.bytes / 4; i += step) ((unsigned*)a.dst)[i] = ((const unsigned*)a.src)[i];
+  if (blockIdx.x == 0 && threadIdx.x < 4 && a.ints[threadIdx.x]) a.out[threadIdx.x] = *a.ints[threadIdx.x];
+}
+
 // XCD (XCC id) each workgroup of a (gx, gy) grid runs on, at its linear index:
 // lets the host check how workgroups are dealt to the XCDs.
 extern "C" __global__ __launch_bounds__(64) void xcc_ids(int* out) {
