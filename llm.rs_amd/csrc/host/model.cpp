@@ -753,7 +753,7 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
       L(p.name, work, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
     } else {
       PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, gemm_group_m()};
-      L(gemm_kernel(m, epi), work, gemm_grid(M, W.n), blk, glds, g);
+      L(gemm_kernel(m, epi), work, gemm_grid(M, W.n), dim3(llmrs::kGemmThreads), glds, g);
     }
   };
   if (exact) {  // RMSNorm + Q8_0 of each row (layer.rs:378; cpu.rs:90-93)
@@ -2040,7 +2040,7 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
       L(p.name, wb, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
     } else {
       PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, silu ? W.n / 2 : W.n, gemm_group_m()};
-      L(name, wb, gemm_grid(B, W.n), blk, glds, g);
+      L(name, wb, gemm_grid(B, W.n), dim3(llmrs::kGemmThreads), glds, g);
     }
   };
   EmbedArgs e{m->embed, b->tokens, b->pos, b->x, m->err, H, c.vocab, nullptr, nullptr, nullptr, nullptr, nullptr,

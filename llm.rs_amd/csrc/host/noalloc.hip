@@ -110,6 +110,7 @@ extern "C" int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmr
     PrefillGemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)out->data, nullptr,
                       nullptr, nullptr, (int)m, (int)n, (int)k, (int)n, gemm_group_m()};
     launch(std::string("gemm_") + wt_tag(b->wt) + "_store",
-           dim3((unsigned)((n + 127) / 128), (unsigned)((m + 127) / 128)), dim3(256), gemm_lds_bytes(), s, g);
+           dim3((unsigned)((n + 127) / 128), (unsigned)((m + 127) / 128)), dim3(kGemmThreads), gemm_lds_bytes(),
+           s, g);
   });
 }

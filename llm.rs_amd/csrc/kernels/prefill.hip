@@ -17,17 +17,26 @@
 // 32 x 32 MFMA (checked on the device), so no operand is wasted.  The epilogue per element and
 // block is then the reference's own two roundings, total = total + isum * s,
 // in block order, so every output is bit-identical to the reference for
-// identical activation codes.  Three VALU operations per element and block
-// (convert, multiply, add) bound the kernel, not the MFMA.
+// identical activation codes.
 //
-// Workgroup tile 128 tokens x 128 rows, four waves of 64 x 64 (2 x 2 MFMA
-// tiles).  Operands are staged in LDS four blocks at a time, double-buffered:
-// the global loads of stage s+1 are issued before stage s is computed and
-// written to LDS after it, so their latency hides behind a whole stage.
-// LDS layouts make each MFMA operand read conflict-free: 16-byte chunk
-// (c, token) lives at c * 128 + (token ^ c), so the 32 lanes of a half-wave
-// read 32 distinct consecutive chunks.  Q4 codes become (q - 8) bytes with
-// ((q | 0x80) - 8) ^ 0x80.
+// Three VALU operations per element and block (convert, multiply, add) bound
+// the kernel: at the 8B gate|up shape with 2048 tokens the VALU issues on 93 %
+// of its cycles and the matrix cores work on 23 %.  So everything else is kept
+// off the VALU.  Workgroup tile 128 tokens x 128 rows, four waves of 64 x 64
+// (2 x 2 MFMA tiles).  Operands reach LDS four blocks at a time by direct
+// loads (no registers, no LDS writes), double-buffered: a stage's loads are in
+// flight while the one before is computed.  Q4 codes stay packed until the
+// operand is read: lanes 0..31 of a wave take a block's low nibbles, the
+// others the high ones, as 16 (q - 8) in the upper half of a byte - a shift
+// and one three-input operation per dword; the factor 16 leaves sums and
+// totals exact (it only moves their exponent) and is taken out at the end.
+// Within a wave the matrix instructions run one tile ahead of the arithmetic.
+// Measured (8B, 2048 tokens, us; before: codes through registers, unpacked
+// when written to LDS, matrix results read as soon as issued): gate|up 1066 ->
+// 867 (555 TOP/s), down 492 -> 412, O 161 -> 139, Q|K|V 244 -> 186; 1B, 700
+// tokens: gate|up 160 -> 128, down 232 -> 163.  Eight waves of 64 x 32 (four a
+// SIMD) were no faster (down 440, O 137), nor were sums started at 1.5 * 2^23
+// so that a subtraction replaces the convert (gate|up 859).
 #include "attn_core.h"
 #include "exact_math.h"
 #include "gemv_core.h"
@@ -41,29 +50,16 @@ typedef float v32f __attribute__((ext_vector_type(32)));
 
 namespace {
 
-#ifndef LLMRS_GEMM_WAVES
-#define LLMRS_GEMM_WAVES 2    // workgroups per CU the register budget allows
-#endif
 constexpr int kBM = 128, kBN = 128;  // workgroup tile (tokens x rows)
 constexpr int kKB = 4;               // 32-element blocks per pipeline stage
 
-// 16 Q4 codes (low or high nibbles of a 16-byte block) as int8 (q - 8).
-// Branch-free: the half-wave selects its nibble with a per-lane shift.
-__device__ __forceinline__ v4i q4_bytes(u32x4 w, int high) {
-  const unsigned M = 0x0F0F0F0Fu, sh = 4u * (unsigned)high;
-  const u32x4 q = u32x4{(w.x >> sh) & M, (w.y >> sh) & M, (w.z >> sh) & M, (w.w >> sh) & M};
-  // per byte: ((q + 128) - 8) - 128 without borrows between bytes
-  const u32x4 r = ((q | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-  return v4i{(int)r.x, (int)r.y, (int)r.z, (int)r.w};
-}
-
-// LDS of one pipeline stage (bytes): activation codes and weight codes as
-// int8 in 16-byte chunks, chunk (c, i) at c * 128 + (i ^ c) for c = 2 b + h
-// (codes 16 h .. 16 h + 15 of block b) and token / row i, then f32 scales
-// d_w [kKB][SW] and d_a [kKB][SW] (rows padded by 4).  A half-wave's MFMA
-// operand read is a permutation of 32 consecutive chunks, and the XOR and
-// the padding spread the staging writes (8 chunks of one token, 4 scales of
-// one row) over distinct banks.
+// LDS of one pipeline stage (bytes).  Codes in 16-byte chunks as they lie in
+// memory, one row (token) after the other: chunk c of row i at
+// i * C + (c ^ swizzle(i)), C chunks per row.  The lanes of a wave's direct
+// load fill 64 consecutive chunks, whole rows of a stage, so the global reads
+// are runs of 64 or 128 bytes; a half-wave's operand read (one chunk of 32
+// rows) takes 16 rows' chunks from 16 different places of a 256-byte window.
+// Then f32 scales d_w [kKB][SW] and d_a [kKB][SW] (rows padded by 4).
 struct GemmStage {
   static constexpr int A = 0;
   static constexpr int B = A + 2 * kKB * kBM * 16;
@@ -73,21 +69,39 @@ struct GemmStage {
   static constexpr int BYTES = DA + kKB * SW * 4;
 };
 
-template <int WT>
-struct GemmLoads {
-  static constexpr int BCH = WT == WT_Q8H ? 2 : 1;             // 16-byte chunks per weight block
-  static constexpr int A_PER_T = 2 * kKB * kBM / 256;          // activation chunks per thread
-  static constexpr int B_PER_T = kKB * BCH * kBN / 256;        // weight chunks per thread
-  static constexpr int S_PER_T = kKB * kBN / 256;              // scales per thread (d_w and d_a)
-};
+// 128-byte rows (activations, Q8 weights): 8 chunks; 64-byte rows (Q4): 4.
+__device__ __forceinline__ int swz8(int row) { return (row >> 1) & 7; }
+__device__ __forceinline__ int swz4(int row) { return (row >> 2) & 3; }
 
-// MFMA operands of one block for a wave's 2 x 2 tiles: codes, d_a of the
-// lane's token in each token tile, d_w of the lane's row in row tile
-// `half` (the two-block scale MFMA takes row tile blk from lanes 32 blk..).
+// MFMA operands of one block for a wave's 2 x 2 tiles: codes (Q4: the raw
+// 16 bytes of the lane's row until unpack()), d_a of the lane's token in each
+// token tile, d_w of the lane's row in row tile `half` (the two-block scale
+// MFMA takes row tile blk from lanes 32 blk..).
 struct GemmOps {
   v4i A[2], B[2];
   float da[2], dw;
 };
+
+// The lane's 16 Q4 codes as int8 16 (q - 8): q ^ 8 in the upper nibble of a
+// byte.  sh = 4 takes the low nibbles (codes 0..15), 0 the high (16..31).
+__device__ __forceinline__ v4i q4_bytes16(v4i w, int sh) {
+  v4i r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = (int)((((unsigned)w[i] << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
+  return r;
+}
+
+// The value is computed here and read after here.
+template <typename T>
+__device__ __forceinline__ void pin(T& x) {
+  asm volatile("" : "+v"(x));
+}
+
+// 16 bytes per lane from global memory to lds + 16 * lane, without registers.
+__device__ __forceinline__ void load_lds16(const void* src, uint8_t* lds) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
 
 }  // namespace
 
@@ -112,167 +126,175 @@ __device__ __forceinline__ void gemm_tile(const PrefillGemmArgs& a, int& m0, int
 template <int WT, int EPI>
 __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds) {
   typedef GemmStage S;
-  typedef GemmLoads<WT> G;
-  constexpr int BCH = G::BCH;
-  const int lane = lane_id(), wave = wave_id(), tid = threadIdx.x;
+  constexpr int BCH = WT == WT_Q8H ? 2 : 1;  // 16-byte chunks per weight block
+  constexpr int RCH = kKB * BCH;             // chunks of a weight row per stage
+  constexpr int AL = 2 * kKB * kBM / 256, BL = RCH * kBN / 256, SL = kKB * kBN / 256;  // loads per thread
+  const int lane = lane_id(), tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int half = lane >> 5, col = lane & 31;
   int m0, n0;
   gemm_tile(a, m0, n0);
   const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
   const int nb = a.K >> 5;
-  const int nstage = (nb + kKB - 1) / kKB;
+  const int nfull = nb / kKB, rest = nb % kKB;
 
-  // ---- staging: global -> registers -> LDS -------------------------------
-  // activation chunk q: token q / (2 kKB), c = q % (2 kKB); weight chunk q:
-  // row q / (kKB BCH), chunk q % (kKB BCH) of that row's stage bytes;
-  // scales: (token | row) q / kKB, block q % kKB.  Scales stay raw until the
-  // LDS write, so nothing waits on the loads before the stage's compute.
-  i32x4 ra[G::A_PER_T], rb[G::B_PER_T];
-  unsigned rdw[G::S_PER_T];
-  float rda[G::S_PER_T];
-  auto load_stage = [&](int st) {
-    const int b0 = st * kKB;
+  // ---- staging: codes straight to LDS, scales through registers -------------
+  // Load j of a wave fills chunks 256 j + 64 wave + lane: chunk p belongs to
+  // row p / C and holds chunk (p % C) ^ swizzle(row) of it.
+  const int8_t* xbase = a.xq + (size_t)m0 * a.K;
+  const uint8_t* wbase = a.wq + (size_t)n0 * nb * (16 * BCH);
+  const int ac = (lane & 7) ^ swz8(8 * wave + lane / 8);  // independent of j (32 rows further)
+  const int bc = WT == WT_Q8H ? ac : ((lane & 3) ^ swz4(lane / 4));
+  unsigned aoff[AL], boff[BL];  // bytes from the tile's first row, block 0
 #pragma unroll
-    for (int j = 0; j < G::A_PER_T; ++j) {
-      const int q = tid + 256 * j;
-      const int tok = min(m0 + q / (2 * kKB), a.M - 1);
-      const int c = q % (2 * kKB);
-      const int blk = min(b0 + c / 2, nb - 1);
-      ra[j] = *(const i32x4*)(a.xq + (size_t)tok * a.K + (size_t)blk * 32 + 16 * (c & 1));
-    }
+  for (int j = 0; j < AL; ++j)
+    aoff[j] = (unsigned)(min(m0 + 32 * j + 8 * wave + lane / 8, a.M - 1) - m0) * (unsigned)a.K;
 #pragma unroll
-    for (int j = 0; j < G::B_PER_T; ++j) {
-      const int q = tid + 256 * j;
-      const int row = min(n0 + q / (kKB * BCH), a.N - 1);
-      const int c = q % (kKB * BCH);
-      const int blk = min(b0 + c / BCH, nb - 1);
-      rb[j] = *(const i32x4*)(a.wq + ((size_t)row * nb + blk) * (16 * BCH) + 16 * (c % BCH));
-    }
+  for (int j = 0; j < BL; ++j)
+    boff[j] = (unsigned)(min(n0 + (256 * j + 64 * wave + lane) / RCH, a.N - 1) - n0) * (unsigned)(nb * 16 * BCH);
+  const int srow = tid / kKB, sblk = tid % kKB;  // scales: row srow + 64 j, block sblk
+  unsigned rdw[SL];
+  float rda[SL];
+  auto load_stage = [&](int b0, uint8_t* base) {
+    // blocks past the row's end (a last partial stage): its last block again
+    const int ab = min(b0 + ac / 2, nb - 1) * 32 + 16 * (ac & 1);
+    const int bb = min(b0 + bc / BCH, nb - 1) * (16 * BCH) + 16 * (bc % BCH);
 #pragma unroll
-    for (int j = 0; j < G::S_PER_T; ++j) {
-      const int q = tid + 256 * j;
-      const int blk = min(b0 + q % kKB, nb - 1);
-      const int row = min(n0 + q / kKB, a.N - 1);
-      const size_t si = (size_t)row * nb + blk;
+    for (int j = 0; j < AL; ++j) load_lds16(xbase + (aoff[j] + (unsigned)ab), base + S::A + (256 * j + 64 * wave) * 16);
+#pragma unroll
+    for (int j = 0; j < BL; ++j) load_lds16(wbase + (boff[j] + (unsigned)bb), base + S::B + (256 * j + 64 * wave) * 16);
+    const int blk = min(b0 + sblk, nb - 1);
+#pragma unroll
+    for (int j = 0; j < SL; ++j) {
+      const size_t si = (size_t)min(n0 + srow + 64 * j, a.N - 1) * nb + blk;
       rdw[j] = WT == WT_Q4F ? ((const unsigned*)a.ws)[si] : ((const uint16_t*)a.ws)[si];
-      const int tok = min(m0 + q / kKB, a.M - 1);
-      rda[j] = a.xd[(size_t)tok * nb + blk];
+      rda[j] = a.xd[(size_t)min(m0 + srow + 64 * j, a.M - 1) * nb + blk];
     }
   };
-  auto store_stage = [&](int buf) {
-    uint8_t* base = lds + buf * S::BYTES;
+  auto store_scales = [&](uint8_t* base) {
 #pragma unroll
-    for (int j = 0; j < G::A_PER_T; ++j) {
-      const int q = tid + 256 * j;
-      const int tok = q / (2 * kKB), c = q % (2 * kKB);
-      *(i32x4*)(base + S::A + (c * kBM + (tok ^ c)) * 16) = ra[j];
-    }
-#pragma unroll
-    for (int j = 0; j < G::B_PER_T; ++j) {
-      const int q = tid + 256 * j;
-      const int row = q / (kKB * BCH), c = q % (kKB * BCH);
-      if (WT == WT_Q8H) {
-        *(i32x4*)(base + S::B + (c * kBN + (row ^ c)) * 16) = rb[j];
-      } else {  // one Q4 block: low nibbles are codes 0..15, high 16..31
-        const u32x4 w = u32x4{(unsigned)rb[j].x, (unsigned)rb[j].y, (unsigned)rb[j].z, (unsigned)rb[j].w};
-        const v4i lo = q4_bytes(w, 0), hi = q4_bytes(w, 1);
-        *(v4i*)(base + S::B + ((2 * c) * kBN + (row ^ (2 * c))) * 16) = lo;
-        *(v4i*)(base + S::B + ((2 * c + 1) * kBN + (row ^ (2 * c + 1))) * 16) = hi;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < G::S_PER_T; ++j) {
-      const int q = tid + 256 * j;
-      const int b = q % kKB, r = q / kKB;
-      ((float*)(base + S::DW))[b * S::SW + r] = wscale<WT>(rdw[j]);
-      ((float*)(base + S::DA))[b * S::SW + r] = rda[j];
+    for (int j = 0; j < SL; ++j) {
+      ((float*)(base + S::DW))[sblk * S::SW + srow + 64 * j] = wscale<WT>(rdw[j]);
+      ((float*)(base + S::DA))[sblk * S::SW + srow + 64 * j] = rda[j];
     }
   };
 
   // ---- compute -------------------------------------------------------------
-  // Per-lane LDS offsets of the operands (the block adds a constant).
-  int offA[2], offB[2], offDA[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    offA[t] = S::A + (half * kBM + wm + 32 * t) * 16;  // + (col ^ c) per block
-    offB[t] = S::B + (half * kBN + wn + 32 * t) * 16;
-    offDA[t] = S::DA + (wm + 32 * t + col) * 4;
-  }
-  const int offDW = S::DW + (wn + 32 * half + col) * 4;  // row tile `half` (two-block MFMA)
   auto load_ops = [&](const uint8_t* base, int b, GemmOps& o) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const int cx = (col ^ half) ^ (2 * b);  // token / row swizzle of chunk c = 2 b + half
-      const i32x4 va = *(const i32x4*)(base + offA[t] + (b * (2 * kBM) + cx) * 16);
-      o.A[t] = v4i{va.x, va.y, va.z, va.w};
-      const i32x4 vb = *(const i32x4*)(base + offB[t] + (b * (2 * kBN) + cx) * 16);
-      o.B[t] = v4i{vb.x, vb.y, vb.z, vb.w};
-      o.da[t] = *(const float*)(base + offDA[t] + b * (S::SW * 4));
+      const int tok = wm + 32 * t + col, row = wn + 32 * t + col;
+      o.A[t] = *(const v4i*)(base + S::A + (tok * 8 + ((2 * b + half) ^ swz8(tok))) * 16);
+      o.B[t] = WT == WT_Q8H ? *(const v4i*)(base + S::B + (row * 8 + ((2 * b + half) ^ swz8(row))) * 16)
+                            : *(const v4i*)(base + S::B + (row * 4 + (b ^ swz4(row))) * 16);
+      o.da[t] = ((const float*)(base + S::DA))[b * S::SW + tok];
     }
-    o.dw = *(const float*)(base + offDW + b * (S::SW * 4));
+    o.dw = ((const float*)(base + S::DW))[b * S::SW + wn + 32 * half + col];
+  };
+  const int sh = half ? 0 : 4;
+  auto unpack = [&](GemmOps& o) {
+    if (WT != WT_Q8H) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) o.B[t] = q4_bytes16(o.B[t], sh);
+    }
+  };
+  auto scales = [&](const GemmOps& o, int t) {
+    return __builtin_amdgcn_mfma_f32_32x32x1f32(o.da[t], o.dw, v32f{}, 0, 0, 0);
+  };
+  auto sums = [&](const GemmOps& o, int t, int r) {
+    return __builtin_amdgcn_mfma_i32_32x32x32_i8(o.A[t], o.B[r], v16i{}, 0, 0, 0);
   };
 
-  float acc[2][2][16];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[t][r][i] = 0.0f;
-  // sc: both row tiles' scales of token tile t (registers 16 r ..).
-  auto epi = [&](int t, int r, const v16i& p, const v32f& sc) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i)  // cpu.rs:913,932: total += isum * (d_w * d_a)
-      acc[t][r][i] = acc[t][r][i] + (float)p[i] * sc[16 * r + i];
-  };
+  v16f acc[2][2] = {{v16f{}, v16f{}}, {v16f{}, v16f{}}};
 
-  load_stage(0);
-  store_stage(0);
-  __syncthreads();
-  for (int st = 0; st < nstage; ++st) {
-    if (st + 1 < nstage) load_stage(st + 1);
-    const uint8_t* base = lds + (st & 1) * S::BYTES;
-    const int kvalid = min(kKB, nb - st * kKB);
-    if (kvalid == kKB) {
-      // Software pipeline over the stage's 4 kKB tiles k = 4 b + 2 t + r:
-      // the MFMAs of tile k+1 are issued before the VALU work of tile k, and
-      // the operands of block b+1 are read while block b is in flight.
-      GemmOps o[2];
-      v16i P[2];
-      v32f SC;  // scales of the current (block, token tile) pair, both row tiles
-      load_ops(base, 0, o[0]);
-      P[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o[0].A[0], o[0].B[0], v16i{}, 0, 0, 0);
-#pragma unroll
-      for (int k = 0; k < 4 * kKB; ++k) {
-        const int b = k / 4, t = (k / 2) % 2, r = k % 2;
-        // The pair's scale MFMA at its r = 0 tile, then the next tile's
-        // integer MFMA, whose issue covers the scale MFMA's latency.
-        if (r == 0) SC = __builtin_amdgcn_mfma_f32_32x32x1f32(o[b % 2].da[t], o[b % 2].dw, v32f{}, 0, 0, 0);
-        if (k % 4 == 0 && b + 1 < kKB) load_ops(base, b + 1, o[(b + 1) % 2]);
-        if (k + 1 < 4 * kKB) {
-          const int kn = k + 1;
-          const GemmOps& on = o[(kn / 4) % 2];
-          P[kn % 2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(on.A[(kn / 2) % 2], on.B[kn % 2], v16i{}, 0, 0, 0);
-        }
-        epi(t, r, P[k % 2], SC);
-      }
-    } else {
-      for (int b = 0; b < kvalid; ++b) {
-        GemmOps o;
-        load_ops(base, b, o);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const v32f sc = __builtin_amdgcn_mfma_f32_32x32x1f32(o.da[t], o.dw, v32f{}, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            const v16i p = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.A[t], o.B[r], v16i{}, 0, 0, 0);
-            epi(t, r, p, sc);
-          }
-        }
-      }
-    }
-    if (st + 1 < nstage) store_stage((st + 1) & 1);
+  // The next stage's loads are in flight while this one is computed; each
+  // wave waits for its own before the barrier that hands the buffer over.
+  auto hand_over = [&](int st, bool more) {
+    if (more) store_scales(lds + ((st + 1) & 1) * S::BYTES);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+  };
+  load_stage(0, lds);
+  hand_over(-1, true);
+  for (int st = 0; st < nfull; ++st) {
+    const bool more = (st + 1) * kKB < nb;
+    if (more) load_stage((st + 1) * kKB, lds + ((st + 1) & 1) * S::BYTES);
+    const uint8_t* base = lds + (st & 1) * S::BYTES;
+    // The stage's 4 kKB tiles k = 4 b + 2 t + r, pipelined within the wave: the
+    // block sums of tile k + 1 are issued before the arithmetic of tile k, and
+    // the next pair's scales between the last products that read this pair's
+    // and the additions, so no result is waited for.  pin() and the fences keep
+    // this order: left to itself the compiler issues a stage's matrix
+    // instructions together and spills their results.
+    GemmOps o[2];
+    v16i P[2];
+    load_ops(base, 0, o[0]);
+    unpack(o[0]);
+    v32f SC = scales(o[0], 0);  // both row tiles of token tile t
+    P[0] = sums(o[0], 0, 0);
+    pin(SC);
+    pin(P[0]);
+#pragma unroll
+    for (int k = 0; k < 4 * kKB; ++k) {
+      const int t = (k / 2) % 2, r = k % 2, kn = k + 1, tn = (kn / 2) % 2;
+      GemmOps& on = o[(kn / 4) % 2];
+      if (k % 4 == 0 && k + 4 < 4 * kKB) load_ops(base, k / 4 + 1, o[(k / 4 + 1) % 2]);
+      if (kn < 4 * kKB) {
+        pin(on.A[tn]);
+        P[kn % 2] = sums(on, tn, kn % 2);
+        pin(P[kn % 2]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      pin(P[k % 2]);
+      v16f f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) f[i] = (float)P[k % 2][i];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) f[i] = f[i] * SC[16 * r + i];  // cpu.rs:913,932: total += isum * (d_w * d_a)
+      pin(f);
+      __builtin_amdgcn_sched_barrier(0);
+      if (r == 1 && kn < 4 * kKB) {
+        pin(on.da[tn]);
+        SC = scales(on, tn);
+        pin(SC);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[t][r][i] = acc[t][r][i] + f[i];
+      pin(acc[t][r]);
+      if (k % 4 == 2 && k + 2 < 4 * kKB) {
+        GemmOps& ob = o[(k / 4 + 1) % 2];
+        unpack(ob);
+        pin(ob.B[0]);
+        pin(ob.B[1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    hand_over(st, more);
+  }
+  const uint8_t* tail = lds + (nfull & 1) * S::BYTES;
+  for (int b = 0; b < rest; ++b) {
+    GemmOps o;
+    load_ops(tail, b, o);
+    unpack(o);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const v32f sc = scales(o, t);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const v16i p = sums(o, t, r);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][r][i] = acc[t][r][i] + (float)p[i] * sc[16 * r + i];
+      }
+    }
+  }
+  if (WT != WT_Q8H) {  // the Q4 codes were 16 times theirs
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][r][i] = acc[t][r][i] * 0.0625f;
   }
 
   // Epilogues.  Register i of a tile holds token 8 (i / 4) + 4 half + i % 4
@@ -317,7 +339,7 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
 // Dynamic LDS: two pipeline stages, gemm_lds_bytes(weights) at launch.
 static_assert(2 * GemmStage::BYTES == gemm_lds_bytes(), "GEMM LDS size");
 #define LLMRS_GEMM(name, WT, EPI)                                                 \
-  extern "C" __global__ __launch_bounds__(kThreads, LLMRS_GEMM_WAVES) void name(PrefillGemmArgs a) { \
+  extern "C" __global__ __launch_bounds__(kGemmThreads, 2) void name(PrefillGemmArgs a) { \
     extern __shared__ __align__(16) uint8_t gemm_lds[];                            \
     gemm_impl<WT, EPI>(a, gemm_lds);                                              \
   }
