@@ -166,7 +166,15 @@ struct SgemmPlan {
   unsigned grid = 1;
 };
 bool sgemm_serves(size_t m, size_t k);
+bool sgemm_faster(const std::string& epi, int m, int n, int k, int num_cus);
 SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus);
+// A tile GEMM launch (prefill.hip): kernel, grid of tiles, dynamic LDS.
+struct GemmPlan {
+  std::string name;
+  dim3 grid;
+  size_t lds;
+};
+GemmPlan gemm_plan(int wt, const std::string& epi, int m, int n, int num_cus);
 // LDS bytes of a GEMV's activation area (codes, scales, Q4 offsets) for input length k.
 inline size_t gemv_act_lds_host(int k) { return (size_t)k + 8 * (size_t)(k / 32); }
 

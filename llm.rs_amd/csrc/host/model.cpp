@@ -684,19 +684,12 @@ void ensure_prefill(llmrs_model* m) {
   m->pf_cap = cap;
 }
 
-std::string gemm_kernel(const llmrs_model* m, const char* epi) {
-  return std::string("gemm_") + wt_tag(m->wt) + "_" + epi;
+// Operand order of the activation rows of a prefill linear layer: the skinny
+// GEMM's (sgemm.hip) or the tile GEMM's; both are bit-identical to the
+// reference's block loop, and each launch takes the faster.
+int prefill_layout(const char* epi, int M, const DevLinear& W) {
+  return sgemm_faster(epi, M, W.n, W.k, ctx().num_cus) ? llmrs::kActMfma : llmrs::kActNatural;
 }
-
-// Whether M prefill rows run their linear layers on the skinny GEMM (sgemm.hip;
-// the activation codes then in its operand order) rather than the 128 x
-// 128-tile GEMM; both are bit-identical to the reference's block loop.
-bool prefill_skinny(const llmrs_model* m, int M) {
-  const llmrs_model_config& c = m->c;
-  return sgemm_serves(M, c.hidden) && sgemm_serves(M, c.ffn) && sgemm_serves(M, (size_t)c.n_heads * c.head_dim);
-}
-
-dim3 gemm_grid(int M, int N) { return dim3((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128)); }
 
 // Device buffers a test probe adds to one prefill layer: ctx and the SwiGLU
 // product m as f32 (the production path keeps only their Q8_0 codes).
@@ -726,7 +719,6 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
   auto after = [&](int stage) {
     if (probe && probe->after) probe->after(stage);
   };
-  const size_t glds = gemm_lds_bytes();
   const float scale = 1.0f / std::sqrt((float)hd);  // layer.rs:258
   // f16 caches use the matrix-core kernel (LLMRS_PREFILL_ATTN=valu selects the
   // vector kernel, which also serves f32 caches)
@@ -741,29 +733,31 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
     kc = Lb.kc;
     vc = Lb.vc;
   }
-  const bool skinny = prefill_skinny(m, M);
-  const int layout = skinny ? llmrs::kActMfma : llmrs::kActNatural;
-  // One linear layer over the M rows on the tile GEMM or the skinny GEMM.
-  auto linear = [&](const char* epi, const DevLinear& W, const int8_t* xq, const float* xd, float* y,
+  const int lay_qkv = prefill_layout("store", M, Lb.qkv), lay_o = prefill_layout("resid", M, Lb.o);
+  const int lay_gu = prefill_layout("silu", M, Lb.gu), lay_down = prefill_layout("resid", M, Lb.down);
+  // One linear layer over the M rows (operand order `layout`; the SwiGLU's
+  // outputs in the order of the down projection).
+  auto linear = [&](const char* epi, const DevLinear& W, int layout, const int8_t* xq, const float* xd, float* y,
                     const float* res, int8_t* yq, float* yd, int ldy) {
     const double work = flops(M, W.n, W.k);
-    if (skinny) {
-      SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, layout};
+    if (layout == llmrs::kActMfma) {
+      SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, lay_down};
       const SgemmPlan p = sgemm_plan(m->wt, epi, M, W.n, ctx().num_cus);
       L(p.name, work, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
     } else {
-      PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, gemm_group_m()};
-      L(gemm_kernel(m, epi), work, gemm_grid(M, W.n), dim3(llmrs::kGemmThreads), glds, g);
+      PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, gemm_group_m(), lay_down};
+      const GemmPlan p = gemm_plan(m->wt, epi, M, W.n, ctx().num_cus);
+      L(p.name, work, p.grid, dim3(llmrs::kGemmThreads), p.lds, g);
     }
   };
   if (exact) {  // RMSNorm + Q8_0 of each row (layer.rs:378; cpu.rs:90-93)
-    exact_norm(m, L, m->pf_x, Lb.norm[0], m->pf_aq, m->pf_ad, nullptr, M, layout);
+    exact_norm(m, L, m->pf_x, Lb.norm[0], m->pf_aq, m->pf_ad, nullptr, M, lay_qkv);
   } else {
-    PrefillRowArgs r{m->pf_x, Lb.norm[0], m->pf_aq, m->pf_ad, M, H, c.rms_eps, layout};
+    PrefillRowArgs r{m->pf_x, Lb.norm[0], m->pf_aq, m->pf_ad, M, H, c.rms_eps, lay_qkv};
     L("prefill_rows_q8", 5.0 * H * M, dim3((unsigned)M), blk, gemv_act_lds_host(H), r);
   }
   after(0);
-  linear("store", Lb.qkv, m->pf_aq, m->pf_ad, m->pf_qkv, nullptr, nullptr, nullptr, QR);  // Q|K|V
+  linear("store", Lb.qkv, lay_qkv, m->pf_aq, m->pf_ad, m->pf_qkv, nullptr, nullptr, nullptr, QR);  // Q|K|V
   after(1);
   {  // RoPE + K/V append
     PrefillRopeArgs r{m->pf_qkv, m->pf_q, kc, vc, m->rope_cos, m->rope_sin, M, nq, nkv, hd,
@@ -775,7 +769,7 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
   after(2);
   {  // causal attention
     PrefillAttnArgs a{m->pf_q, kc, vc, probe ? probe->ctx : nullptr, m->pf_ctx_q, m->pf_ctx_d, M, nq,
-                      nkv, kv_rows(m), (int)start, scale, layout};
+                      nkv, kv_rows(m), (int)start, scale, lay_o};
     if (exact)  // one workgroup per (query head, row); the scores of up to start + M positions in LDS
       L("exact_attn_prefill_hd" + std::to_string(hd) + (kv16 ? "_f16" : "_f32"), attn_flops,
         dim3((unsigned)nq, (unsigned)M), blk, (start + M) * 4, a);
@@ -785,19 +779,19 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
       L(attn, attn_flops, dim3((unsigned)((M + 31) / 32), (unsigned)nq), blk, 0, a);
   }
   after(3);
-  linear("resid", Lb.o, m->pf_ctx_q, m->pf_ctx_d, m->pf_h, m->pf_x, nullptr, nullptr, H);  // O + residual
+  linear("resid", Lb.o, lay_o, m->pf_ctx_q, m->pf_ctx_d, m->pf_h, m->pf_x, nullptr, nullptr, H);  // O + residual
   after(4);
   if (exact) {  // post-attention RMSNorm + Q8_0
-    exact_norm(m, L, m->pf_h, Lb.norm[1], m->pf_aq, m->pf_ad, nullptr, M, layout);
+    exact_norm(m, L, m->pf_h, Lb.norm[1], m->pf_aq, m->pf_ad, nullptr, M, lay_gu);
   } else {
-    PrefillRowArgs r{m->pf_h, Lb.norm[1], m->pf_aq, m->pf_ad, M, H, c.rms_eps, layout};
+    PrefillRowArgs r{m->pf_h, Lb.norm[1], m->pf_aq, m->pf_ad, M, H, c.rms_eps, lay_gu};
     L("prefill_rows_q8", 5.0 * H * M, dim3((unsigned)M), blk, gemv_act_lds_host(H), r);
   }
   after(5);
   // gate|up + SiLU + Q8_0 of m (layer.rs:40-89)
-  linear("silu", Lb.gu, m->pf_aq, m->pf_ad, probe ? probe->mf : nullptr, nullptr, m->pf_m_q, m->pf_m_d, F);
+  linear("silu", Lb.gu, lay_gu, m->pf_aq, m->pf_ad, probe ? probe->mf : nullptr, nullptr, m->pf_m_q, m->pf_m_d, F);
   after(6);
-  linear("resid", Lb.down, m->pf_m_q, m->pf_m_d, m->pf_x, m->pf_h, nullptr, nullptr, H);  // down + residual
+  linear("resid", Lb.down, lay_down, m->pf_m_q, m->pf_m_d, m->pf_x, m->pf_h, nullptr, nullptr, H);  // down + residual
   after(7);
 }
 
@@ -1885,9 +1879,12 @@ int llmrs_model_probe_prefill_layer(llmrs_model* m, int layer, size_t start_pos,
     p.ctx = pb.get<float>(M * qd);
     p.mf = pb.get<float>(M * F);
     LLMRS_HIP(hipMemcpyAsync(m->pf_x, x, M * H * sizeof(float), hipMemcpyHostToDevice, s));
-    const int layout = prefill_skinny(m, (int)M) ? llmrs::kActMfma : llmrs::kActNatural;
+    const LayerBufs& Lb = m->layers[layer];
     // codes and scales of the M rows, back in element order
-    auto copy_act = [&](int8_t* q, float* d, const int8_t* dev_q, const float* dev_d, size_t K) {
+    auto copy_act = [&](const char* epi, const DevLinear& W, int8_t* q, float* d, const int8_t* dev_q,
+                        const float* dev_d) {
+      const size_t K = W.k;
+      const int layout = prefill_layout(epi, (int)M, W);
       const size_t rows = llmrs::act_rows(M);
       std::vector<int8_t> hq(rows * K);
       std::vector<float> hd(rows * K / 32);
@@ -1904,20 +1901,20 @@ int llmrs_model_probe_prefill_layer(llmrs_model* m, int layer, size_t start_pos,
     p.after = [&](int stage) {
       switch (stage) {
         case 0:
-          copy_act(out->xq, out->xd, m->pf_aq, m->pf_ad, H);
+          copy_act("store", Lb.qkv, out->xq, out->xd, m->pf_aq, m->pf_ad);
           break;
         case 1: probe_copy(out->qkv, m->pf_qkv, M * m->qkv_rows * sizeof(float)); break;
         case 3:
           probe_copy(out->ctx, p.ctx, M * qd * sizeof(float));
-          copy_act(out->ctx_q, out->ctx_d, m->pf_ctx_q, m->pf_ctx_d, qd);
+          copy_act("resid", Lb.o, out->ctx_q, out->ctx_d, m->pf_ctx_q, m->pf_ctx_d);
           break;
         case 4: probe_copy(out->h, m->pf_h, M * H * sizeof(float)); break;
         case 5:
-          copy_act(out->hq, out->hd, m->pf_aq, m->pf_ad, H);
+          copy_act("silu", Lb.gu, out->hq, out->hd, m->pf_aq, m->pf_ad);
           break;
         case 6:
           probe_copy(out->m, p.mf, M * F * sizeof(float));
-          copy_act(out->m_q, out->m_d, m->pf_m_q, m->pf_m_d, F);
+          copy_act("resid", Lb.down, out->m_q, out->m_d, m->pf_m_q, m->pf_m_d);
           break;
         case 7: probe_copy(out->out, m->pf_x, M * H * sizeof(float)); break;
       }
@@ -2001,7 +1998,8 @@ GemvPlan batch_gemv_plan(const llmrs_batch* b, const char* epi, const DevLinear&
 
 std::string batch_linear_kernel(const llmrs_batch* b, const char* epi, const DevLinear& W) {
   if (b->gemv) return batch_gemv_plan(b, epi, W).name;
-  return b->skinny ? sgemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name : gemm_kernel(b->m, epi);
+  return b->skinny ? sgemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name
+                   : gemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name;
 }
 
 // One greedy step of every sequence of the batch.
@@ -2010,7 +2008,6 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
   const llmrs_model_config& c = m->c;
   const int B = b->B, H = c.hidden, hd = c.head_dim, nq = c.n_heads, nkv = c.n_kv_heads;
   const dim3 blk(256);
-  const size_t glds = gemm_lds_bytes();
   // One linear layer over the B rows: Y = X W^T (+ res), or the SwiGLU
   // product's Q8_0 codes; work figure = the weight bytes.
   auto linear = [&](const char* epi, const DevLinear& W, const int8_t* xq, const float* xd, float* y,
@@ -2039,8 +2036,10 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
       const SgemmPlan p = sgemm_plan(m->wt, epi, B, W.n, ctx().num_cus);
       L(p.name, wb, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
     } else {
-      PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, silu ? W.n / 2 : W.n, gemm_group_m()};
-      L(name, wb, gemm_grid(B, W.n), dim3(llmrs::kGemmThreads), glds, g);
+      PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, silu ? W.n / 2 : W.n, gemm_group_m(),
+                        llmrs::kActNatural};
+      const GemmPlan p = gemm_plan(m->wt, epi, B, W.n, ctx().num_cus);
+      L(p.name, wb, p.grid, dim3(llmrs::kGemmThreads), p.lds, g);
     }
   };
   EmbedArgs e{m->embed, b->tokens, b->pos, b->x, m->err, H, c.vocab, nullptr, nullptr, nullptr, nullptr, nullptr,

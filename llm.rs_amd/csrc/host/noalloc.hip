@@ -94,7 +94,8 @@ extern "C" int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmr
     // few rows of whole 128-element runs: the skinny GEMM, where its whole
     // 16-row tiles fit the scratch too
     size_t tile_off = 0;
-    const bool skinny = sgemm_serves(m, k) && scratch_need(act_rows(m), k, &tile_off) <= kNoAllocScratchBytes;
+    const bool skinny = sgemm_faster("store", (int)m, (int)n, (int)k, cx.num_cus) &&
+                        scratch_need(act_rows(m), k, &tile_off) <= kNoAllocScratchBytes;
     if (skinny) scale_off = tile_off;
     int8_t* xq = (int8_t*)cx.noalloc_scratch;
     float* xd = (float*)((uint8_t*)cx.noalloc_scratch + scale_off);
@@ -108,9 +109,8 @@ extern "C" int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmr
       return;
     }
     PrefillGemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)out->data, nullptr,
-                      nullptr, nullptr, (int)m, (int)n, (int)k, (int)n, gemm_group_m()};
-    launch(std::string("gemm_") + wt_tag(b->wt) + "_store",
-           dim3((unsigned)((n + 127) / 128), (unsigned)((m + 127) / 128)), dim3(kGemmThreads), gemm_lds_bytes(),
-           s, g);
+                      nullptr, nullptr, (int)m, (int)n, (int)k, (int)n, gemm_group_m(), llmrs::kActNatural};
+    const GemmPlan p = gemm_plan(b->wt, "store", (int)m, (int)n, cx.num_cus);
+    launch(p.name, p.grid, dim3(kGemmThreads), p.lds, s, g);
   });
 }

@@ -178,12 +178,8 @@ GemvPlan gemv_plan(int wt, const std::string& kind, int n, int k, int num_cus) {
   return p;
 }
 
-// Whether M rows run on the skinny GEMM rather than the 128 x 128-tile GEMM:
-// whole 128-element runs and up to 160 rows, beyond which its 16-row tiles'
-// work passes the time of the few tiles' serial block loops (8B widths at 130
-// rows, skinny / tile us: Q|K|V 36 / 106, O and down 61 / 249, gate|up 142 /
-// 157; its time grows by a ninth of that per 16 rows, the tile GEMM's by a
-// whole pass per 128).  LLMRS_PREFILL_SKINNY=0 keeps every GEMM on the tiles.
+// Whether M rows can run on the skinny GEMM: whole 128-element runs and up to
+// 160 rows.  LLMRS_PREFILL_SKINNY=0 keeps every GEMM on the tiles.
 bool sgemm_serves(size_t m, size_t k) {
   const char* e = std::getenv("LLMRS_PREFILL_SKINNY");
   return m <= 160 && k % 128 == 0 && !(e && *e == '0');
@@ -204,6 +200,61 @@ SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) 
   p.name = std::string("sgemm_") + wt_tag(wt) + "_" + epi + "_r" + std::to_string(R);
   p.grid = (unsigned)(8 * nt * ((rows + 7) / 8));
   return p;
+}
+
+namespace {
+struct GemmTile {
+  int tt, rt;         // 64 tt tokens x 64 rt rows
+  double lone, pair;  // time per block of 32: one workgroup on a CU, two
+};
+constexpr GemmTile kGemmTiles[] = {{2, 2, 2.9, 4.4}, {1, 2, 1.65, 2.5}, {1, 1, 1.0, 1.4}};
+
+// The tile for m tokens x n rows, and its time per block of 32.  It follows
+// from how the tiles fill the CUs: a CU works on two workgroups at once, and a
+// lone one takes more than half the time of a pair (nothing covers its waves'
+// latencies).  In units of a lone 64 x 64 tile's block (0.21 us) the tiles took
+// the times above; the tile with the smallest sum over the fullest CU is
+// taken.  8B down, us for 128 x 128 / 64 x 128 / 64 x 64: 256 rows 269 / 154 /
+// 94, 1024 rows 297 / 237 / 255, 2048 rows 423 / 452 / 492; 1B O at 1500 rows
+// 57 / 43 / 39, gate|up 231 / 245.
+const GemmTile& gemm_tile(const std::string& epi, int m, int n, int num_cus, double* units) {
+  const GemmTile* best = nullptr;
+  for (const GemmTile& t : kGemmTiles) {
+    if (epi == "silu" && t.rt == 1) continue;  // a gate and an up run of 32 per wave
+    const long wgs = (long)((m + 64 * t.tt - 1) / (64 * t.tt)) * ((n + 64 * t.rt - 1) / (64 * t.rt));
+    const long per_cu = (wgs + num_cus - 1) / num_cus;
+    const double u = (double)(per_cu / 2) * t.pair + (double)(per_cu % 2) * t.lone;
+    if (best && u >= *units) continue;
+    best = &t;
+    *units = u;
+  }
+  return *best;
+}
+}  // namespace
+
+GemmPlan gemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
+  double units = 0;
+  const GemmTile& t = gemm_tile(epi, m, n, num_cus, &units);
+  const int bm = 64 * t.tt, bn = 64 * t.rt, bch = wt == WT_Q8H ? 2 : 1;
+  GemmPlan p;
+  p.name = std::string("gemm_") + wt_tag(wt) + "_" + epi + "_" + std::to_string(bm) + "x" + std::to_string(bn);
+  p.grid = dim3((unsigned)((n + bn - 1) / bn), (unsigned)((m + bm - 1) / bm));
+  p.lds = gemm_lds_bytes(t.tt, t.rt, gemm_stage_blocks(t.tt, t.rt, bch), bch);
+  return p;
+}
+
+// Whether the skinny GEMM is the faster one for m rows that it can run: it
+// spreads one row of tiles over the chip, so its time per block grows with
+// n * m / 16, by 0.0061 of gemm_tile's units for 16 tokens x n = the number of
+// CUs; the tiles' time only with the fullest CU.  Skinny / tile, us: 8B gate|up
+// at 32 rows 42 / 52, 48 rows 60 / 53, 128 rows 138 / 76; O at 128 rows 22 /
+// 29, 160 rows 32 / 31; 1B gate|up at 64 rows 26 / 33, 100 rows 42 / 33, O at
+// 160 rows 11 / 18.
+bool sgemm_faster(const std::string& epi, int m, int n, int k, int num_cus) {
+  if (!sgemm_serves((size_t)m, (size_t)k)) return false;
+  double units = 0;
+  (void)gemm_tile(epi, m, n, num_cus, &units);
+  return 0.0061 * n / num_cus * ((m + 15) / 16) < units;
 }
 
 // ---- allocator -------------------------------------------------------------

@@ -316,8 +316,8 @@ struct PrefillGemmArgs {
   const void* ws;        // weight scales [N][nb]
   float* y;              // [M][ldy]: GEMM out (STORE, RESID) or m (SILU, may be null)
   const float* res;      // [M][N] residual (RESID; may alias y)
-  int8_t* yq;            // SILU: [M][N/2] codes of m
-  float* yd;             // SILU: [M][N/64] scales of m
+  int8_t* yq;            // SILU: [M][N/2] codes of m (operand order `layout`)
+  float* yd;             // SILU: [M][N/64] scales of m (operand order `layout`)
   int M, N, K, ldy;
   // Tile order (0 = row-major).  Workgroups reach the 8 XCDs round-robin in
   // dispatch order; with group_m > 0 and a tile count divisible by 8, XCD x
@@ -325,13 +325,18 @@ struct PrefillGemmArgs {
   // at a time, so the workgroups resident on one XCD share operand panels
   // in its L2.
   int group_m;
+  int layout;  // SILU: kActNatural or kActMfma
 };
 
-// Dynamic LDS of the prefill GEMM: two pipeline stages of 4 blocks, each
-// activation and weight codes (int8) 2 x 128 x 128 B, f32 scales 2 x 4 x 132.
 constexpr int kGemmThreads = 256;
-constexpr size_t gemm_lds_bytes() {
-  return 2 * ((size_t)2 * 4 * 128 * 16 * 2 + (size_t)4 * 132 * 4 * 2);
+// 32-element blocks per pipeline stage of a 64 TT tokens x 64 RT rows tile,
+// weight blocks of BCH 16-byte chunks: eight where a wave has one or two tiles
+// per block (a stage has to outlast the next one's loads), four for four and
+// where eight would not leave LDS for two workgroups per CU.
+constexpr int gemm_stage_blocks(int tt, int rt, int bch) { return tt * rt == 4 || (rt == 2 && bch == 2) ? 4 : 8; }
+// Dynamic LDS: two stages of codes and f32 scales (rows padded by 4).
+constexpr size_t gemm_lds_bytes(int tt, int rt, int kb, int bch) {
+  return 2 * ((size_t)kb * 16 * 64 * (2 * tt + bch * rt) + (size_t)kb * 4 * (64 * tt + 4 + 64 * rt + 4));
 }
 
 // Prefill row kernels (prefill.hip).

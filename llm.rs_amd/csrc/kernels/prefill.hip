@@ -37,6 +37,13 @@
 // tokens: gate|up 160 -> 128, down 232 -> 163.  Eight waves of 64 x 32 (four a
 // SIMD) were no faster (down 440, O 137), nor were sums started at 1.5 * 2^23
 // so that a subtraction replaces the convert (gate|up 859).
+//
+// 128 x 128 tiles leave CUs idle when the rows or tokens are few (96 of them
+// for 700 tokens and 2048 rows), and the K blocks of an output cannot be split
+// (their additions have an order).  64 x 128 (a wave: one token tile, two row
+// tiles) and 64 x 64 (one tile, its scales two blocks at a time) give more and
+// shorter chains, in stages of eight blocks; gemm_plan (runtime.cpp) picks one.
+// 1B, 700 tokens, us: down 163 -> 74, O 55 -> 24, Q|K|V 43 -> 18.
 #include "attn_core.h"
 #include "exact_math.h"
 #include "gemv_core.h"
@@ -50,36 +57,41 @@ typedef float v32f __attribute__((ext_vector_type(32)));
 
 namespace {
 
-constexpr int kBM = 128, kBN = 128;  // workgroup tile (tokens x rows)
-constexpr int kKB = 4;               // 32-element blocks per pipeline stage
-
-// LDS of one pipeline stage (bytes).  Codes in 16-byte chunks as they lie in
+// LDS of one pipeline stage (bytes) of a workgroup's 64 TT tokens x 64 RT rows,
+// KB blocks of BCH weight chunks.  Codes in 16-byte chunks as they lie in
 // memory, one row (token) after the other: chunk c of row i at
-// i * C + (c ^ swizzle(i)), C chunks per row.  The lanes of a wave's direct
+// i * C + (c ^ swizzle<C>(i)), C chunks per row.  The lanes of a wave's direct
 // load fill 64 consecutive chunks, whole rows of a stage, so the global reads
-// are runs of 64 or 128 bytes; a half-wave's operand read (one chunk of 32
+// are runs of 64 to 256 bytes; a half-wave's operand read (one chunk of 32
 // rows) takes 16 rows' chunks from 16 different places of a 256-byte window.
-// Then f32 scales d_w [kKB][SW] and d_a [kKB][SW] (rows padded by 4).
+// Then f32 scales d_w [KB][SW] and d_a [KB][SA] (rows padded by 4).
+template <int TT, int RT, int KB, int BCH>
 struct GemmStage {
+  static constexpr int BM = 64 * TT, BN = 64 * RT;
+  static constexpr int AC = 2 * KB, RC = BCH * KB;  // chunks of a token / row
   static constexpr int A = 0;
-  static constexpr int B = A + 2 * kKB * kBM * 16;
-  static constexpr int DW = B + 2 * kKB * kBN * 16;
-  static constexpr int SW = kBN + 4;            // padded scale row (floats)
-  static constexpr int DA = DW + kKB * SW * 4;
-  static constexpr int BYTES = DA + kKB * SW * 4;
+  static constexpr int B = A + AC * BM * 16;
+  static constexpr int DW = B + RC * BN * 16;
+  static constexpr int SW = BN + 4, SA = BM + 4;
+  static constexpr int DA = DW + KB * SW * 4;
+  static constexpr int BYTES = DA + KB * SA * 4;
+  static_assert(2 * BYTES == gemm_lds_bytes(TT, RT, KB, BCH), "GEMM LDS size");
 };
 
-// 128-byte rows (activations, Q8 weights): 8 chunks; 64-byte rows (Q4): 4.
-__device__ __forceinline__ int swz8(int row) { return (row >> 1) & 7; }
-__device__ __forceinline__ int swz4(int row) { return (row >> 2) & 3; }
+template <int C>
+__device__ __forceinline__ int swizzle(int row) {
+  return C == 16 ? row & 15 : C == 8 ? (row >> 1) & 7 : (row >> 2) & 3;
+}
 
-// MFMA operands of one block for a wave's 2 x 2 tiles: codes (Q4: the raw
-// 16 bytes of the lane's row until unpack()), d_a of the lane's token in each
-// token tile, d_w of the lane's row in row tile `half` (the two-block scale
-// MFMA takes row tile blk from lanes 32 blk..).
+// MFMA operands of one block for a wave's TT x RT tiles: codes (Q4: the raw
+// 16 bytes of the lane's row until unpacked) and the operands of the two-block
+// scale MFMA, whose block blk comes from lanes 32 blk..: with two row tiles d_a
+// of the lane's token in each token tile and d_w of its row in row tile `half`;
+// with one, of its token and row in block b + half.
+template <int TT, int RT>
 struct GemmOps {
-  v4i A[2], B[2];
-  float da[2], dw;
+  v4i A[TT], B[RT];
+  float da[TT], dw;
 };
 
 // The lane's 16 Q4 codes as int8 16 (q - 8): q ^ 8 in the upper nibble of a
@@ -108,104 +120,126 @@ __device__ __forceinline__ void load_lds16(const void* src, uint8_t* lds) {
 // First token and row of this workgroup's tile (PrefillGemmArgs::group_m).
 // Both steps are bijections on [0, tiles): the XCD deal when the tile count
 // is a multiple of 8, the grouped walk for any grid.
+template <int BM, int BN>
 __device__ __forceinline__ void gemm_tile(const PrefillGemmArgs& a, int& m0, int& n0) {
   const int gx = gridDim.x, gy = gridDim.y, T = gx * gy;
   if (a.group_m <= 0) {
-    m0 = blockIdx.y * kBM;
-    n0 = blockIdx.x * kBN;
+    m0 = blockIdx.y * BM;
+    n0 = blockIdx.x * BN;
     return;
   }
   int t = blockIdx.x + blockIdx.y * gx;
   if ((T & 7) == 0) t = (t & 7) * (T >> 3) + (t >> 3);
   const int gsz = a.group_m * gx, g = t / gsz, fm = g * a.group_m;
   const int gm = min(gy - fm, a.group_m), r = t - g * gsz;
-  m0 = (fm + r % gm) * kBM;
-  n0 = (r / gm) * kBN;
+  m0 = (fm + r % gm) * BM;
+  n0 = (r / gm) * BN;
 }
 
-template <int WT, int EPI>
+template <int WT, int EPI, int TT, int RT>
 __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds) {
-  typedef GemmStage S;
   constexpr int BCH = WT == WT_Q8H ? 2 : 1;  // 16-byte chunks per weight block
-  constexpr int RCH = kKB * BCH;             // chunks of a weight row per stage
-  constexpr int AL = 2 * kKB * kBM / 256, BL = RCH * kBN / 256, SL = kKB * kBN / 256;  // loads per thread
+  constexpr int KB = gemm_stage_blocks(TT, RT, BCH);
+  typedef GemmStage<TT, RT, KB, BCH> S;
+  typedef GemmOps<TT, RT> Ops;
+  constexpr int T = kGemmThreads;
+  constexpr int AL = S::AC * S::BM / T, BL = S::RC * S::BN / T;  // chunks per thread
+  constexpr int SAL = KB * S::BM / T, SWL = KB * S::BN / T;      // scales per thread
+  constexpr int NTB = TT * RT;                                   // a wave's tiles per block
+  constexpr int AHEAD = NTB == 1 ? 2 : 1;                        // blocks whose operands are read ahead
+  static_assert(EPI != EPI_SILU || RT == 2, "SwiGLU: a gate and an up tile per wave");
+  static_assert(RT == 2 || TT == 1, "scale pairs: two row tiles or two blocks");
   const int lane = lane_id(), tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int half = lane >> 5, col = lane & 31;
   int m0, n0;
-  gemm_tile(a, m0, n0);
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  gemm_tile<S::BM, S::BN>(a, m0, n0);
+  const int wm = (wave >> 1) * 32 * TT, wn = (wave & 1) * 32 * RT;
   const int nb = a.K >> 5;
-  const int nfull = nb / kKB, rest = nb % kKB;
+  const int nfull = nb / KB, rest = nb % KB;
 
   // ---- staging: codes straight to LDS, scales through registers -------------
-  // Load j of a wave fills chunks 256 j + 64 wave + lane: chunk p belongs to
-  // row p / C and holds chunk (p % C) ^ swizzle(row) of it.
+  // Load j of a wave fills chunks T j + 64 wave + lane: chunk p belongs to row
+  // p / C and holds chunk (p % C) ^ swizzle(row) of it (the same for every j).
   const int8_t* xbase = a.xq + (size_t)m0 * a.K;
   const uint8_t* wbase = a.wq + (size_t)n0 * nb * (16 * BCH);
-  const int ac = (lane & 7) ^ swz8(8 * wave + lane / 8);  // independent of j (32 rows further)
-  const int bc = WT == WT_Q8H ? ac : ((lane & 3) ^ swz4(lane / 4));
+  const int ac = (tid % S::AC) ^ swizzle<S::AC>(tid / S::AC);
+  const int bc = (tid % S::RC) ^ swizzle<S::RC>(tid / S::RC);
   unsigned aoff[AL], boff[BL];  // bytes from the tile's first row, block 0
 #pragma unroll
   for (int j = 0; j < AL; ++j)
-    aoff[j] = (unsigned)(min(m0 + 32 * j + 8 * wave + lane / 8, a.M - 1) - m0) * (unsigned)a.K;
+    aoff[j] = (unsigned)(min(m0 + (T * j + tid) / S::AC, a.M - 1) - m0) * (unsigned)a.K;
 #pragma unroll
   for (int j = 0; j < BL; ++j)
-    boff[j] = (unsigned)(min(n0 + (256 * j + 64 * wave + lane) / RCH, a.N - 1) - n0) * (unsigned)(nb * 16 * BCH);
-  const int srow = tid / kKB, sblk = tid % kKB;  // scales: row srow + 64 j, block sblk
-  unsigned rdw[SL];
-  float rda[SL];
+    boff[j] = (unsigned)(min(n0 + (T * j + tid) / S::RC, a.N - 1) - n0) * (unsigned)(nb * 16 * BCH);
+  const int srow = tid / KB, sblk = tid % KB;  // scales: row srow + T / KB j, block sblk
+  unsigned rdw[SWL];
+  float rda[SAL];
   auto load_stage = [&](int b0, uint8_t* base) {
     // blocks past the row's end (a last partial stage): its last block again
     const int ab = min(b0 + ac / 2, nb - 1) * 32 + 16 * (ac & 1);
     const int bb = min(b0 + bc / BCH, nb - 1) * (16 * BCH) + 16 * (bc % BCH);
 #pragma unroll
-    for (int j = 0; j < AL; ++j) load_lds16(xbase + (aoff[j] + (unsigned)ab), base + S::A + (256 * j + 64 * wave) * 16);
+    for (int j = 0; j < AL; ++j) load_lds16(xbase + (aoff[j] + (unsigned)ab), base + S::A + (T * j + 64 * wave) * 16);
 #pragma unroll
-    for (int j = 0; j < BL; ++j) load_lds16(wbase + (boff[j] + (unsigned)bb), base + S::B + (256 * j + 64 * wave) * 16);
+    for (int j = 0; j < BL; ++j) load_lds16(wbase + (boff[j] + (unsigned)bb), base + S::B + (T * j + 64 * wave) * 16);
     const int blk = min(b0 + sblk, nb - 1);
 #pragma unroll
-    for (int j = 0; j < SL; ++j) {
-      const size_t si = (size_t)min(n0 + srow + 64 * j, a.N - 1) * nb + blk;
+    for (int j = 0; j < SWL; ++j) {
+      const size_t si = (size_t)min(n0 + srow + T / KB * j, a.N - 1) * nb + blk;
       rdw[j] = WT == WT_Q4F ? ((const unsigned*)a.ws)[si] : ((const uint16_t*)a.ws)[si];
-      rda[j] = a.xd[(size_t)min(m0 + srow + 64 * j, a.M - 1) * nb + blk];
     }
+#pragma unroll
+    for (int j = 0; j < SAL; ++j) rda[j] = a.xd[(size_t)min(m0 + srow + T / KB * j, a.M - 1) * nb + blk];
   };
   auto store_scales = [&](uint8_t* base) {
 #pragma unroll
-    for (int j = 0; j < SL; ++j) {
-      ((float*)(base + S::DW))[sblk * S::SW + srow + 64 * j] = wscale<WT>(rdw[j]);
-      ((float*)(base + S::DA))[sblk * S::SW + srow + 64 * j] = rda[j];
-    }
+    for (int j = 0; j < SWL; ++j) ((float*)(base + S::DW))[sblk * S::SW + srow + T / KB * j] = wscale<WT>(rdw[j]);
+#pragma unroll
+    for (int j = 0; j < SAL; ++j) ((float*)(base + S::DA))[sblk * S::SA + srow + T / KB * j] = rda[j];
   };
 
   // ---- compute -------------------------------------------------------------
-  auto load_ops = [&](const uint8_t* base, int b, GemmOps& o) {
+  const int tok = wm + col, row = wn + col;  // of tile 0; tile t's swizzles are the same
+  auto load_codes = [&](const uint8_t* base, int b, Ops& o) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int tok = wm + 32 * t + col, row = wn + 32 * t + col;
-      o.A[t] = *(const v4i*)(base + S::A + (tok * 8 + ((2 * b + half) ^ swz8(tok))) * 16);
-      o.B[t] = WT == WT_Q8H ? *(const v4i*)(base + S::B + (row * 8 + ((2 * b + half) ^ swz8(row))) * 16)
-                            : *(const v4i*)(base + S::B + (row * 4 + (b ^ swz4(row))) * 16);
-      o.da[t] = ((const float*)(base + S::DA))[b * S::SW + tok];
+    for (int t = 0; t < TT; ++t)
+      o.A[t] = *(const v4i*)(base + S::A + ((tok + 32 * t) * S::AC + ((2 * b + half) ^ swizzle<S::AC>(tok))) * 16);
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int c = BCH == 2 ? 2 * b + half : b;
+      o.B[r] = *(const v4i*)(base + S::B + ((row + 32 * r) * S::RC + (c ^ swizzle<S::RC>(row))) * 16);
     }
-    o.dw = ((const float*)(base + S::DW))[b * S::SW + wn + 32 * half + col];
+  };
+  auto load_scales = [&](const uint8_t* base, int b, Ops& o) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t) o.da[t] = ((const float*)(base + S::DA))[b * S::SA + tok + 32 * t];
+    o.dw = ((const float*)(base + S::DW))[b * S::SW + row + (RT == 2 ? 32 * half : 0)];
+  };
+  auto load_ops = [&](const uint8_t* base, int b, Ops& o) {
+    load_codes(base, b, o);
+    if (RT == 2) load_scales(base, b, o);
+    else if (b % 2 == 0) load_scales(base, b + half, o);
   };
   const int sh = half ? 0 : 4;
-  auto unpack = [&](GemmOps& o) {
+  auto unpack = [&](Ops& o) {
     if (WT != WT_Q8H) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) o.B[t] = q4_bytes16(o.B[t], sh);
+      for (int r = 0; r < RT; ++r) o.B[r] = q4_bytes16(o.B[r], sh);
     }
   };
-  auto scales = [&](const GemmOps& o, int t) {
+  auto scales = [&](const Ops& o, int t) {
     return __builtin_amdgcn_mfma_f32_32x32x1f32(o.da[t], o.dw, v32f{}, 0, 0, 0);
   };
-  auto sums = [&](const GemmOps& o, int t, int r) {
+  auto sums = [&](const Ops& o, int t, int r) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(o.A[t], o.B[r], v16i{}, 0, 0, 0);
   };
 
-  v16f acc[2][2] = {{v16f{}, v16f{}}, {v16f{}, v16f{}}};
+  v16f acc[TT][RT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[t][r] = v16f{};
 
   // The next stage's loads are in flight while this one is computed; each
   // wave waits for its own before the barrier that hands the buffer over.
@@ -217,31 +251,36 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
   load_stage(0, lds);
   hand_over(-1, true);
   for (int st = 0; st < nfull; ++st) {
-    const bool more = (st + 1) * kKB < nb;
-    if (more) load_stage((st + 1) * kKB, lds + ((st + 1) & 1) * S::BYTES);
+    const bool more = (st + 1) * KB < nb;
+    if (more) load_stage((st + 1) * KB, lds + ((st + 1) & 1) * S::BYTES);
     const uint8_t* base = lds + (st & 1) * S::BYTES;
-    // The stage's 4 kKB tiles k = 4 b + 2 t + r, pipelined within the wave: the
+    // The stage's tiles k = NTB b + RT t + r, pipelined within the wave: the
     // block sums of tile k + 1 are issued before the arithmetic of tile k, and
     // the next pair's scales between the last products that read this pair's
     // and the additions, so no result is waited for.  pin() and the fences keep
     // this order: left to itself the compiler issues a stage's matrix
     // instructions together and spills their results.
-    GemmOps o[2];
+    Ops o[AHEAD + 1];
     v16i P[2];
-    load_ops(base, 0, o[0]);
-    unpack(o[0]);
-    v32f SC = scales(o[0], 0);  // both row tiles of token tile t
+#pragma unroll
+    for (int b = 0; b < AHEAD; ++b) {
+      load_ops(base, b, o[b]);
+      unpack(o[b]);
+    }
+    v32f SC = scales(o[0], 0);  // of tiles k and k + 1, k even
     P[0] = sums(o[0], 0, 0);
     pin(SC);
     pin(P[0]);
 #pragma unroll
-    for (int k = 0; k < 4 * kKB; ++k) {
-      const int t = (k / 2) % 2, r = k % 2, kn = k + 1, tn = (kn / 2) % 2;
-      GemmOps& on = o[(kn / 4) % 2];
-      if (k % 4 == 0 && k + 4 < 4 * kKB) load_ops(base, k / 4 + 1, o[(k / 4 + 1) % 2]);
-      if (kn < 4 * kKB) {
+    for (int k = 0; k < NTB * KB; ++k) {
+      const int b = k / NTB, t = (k % NTB) / RT, r = k % RT, kn = k + 1, tn = (kn % NTB) / RT;
+      const bool next = kn < NTB * KB, ahead = b + AHEAD < KB;
+      Ops& on = o[(kn / NTB) % (AHEAD + 1)];
+      Ops& oa = o[(b + AHEAD) % (AHEAD + 1)];
+      if (k % NTB == 0 && ahead) load_ops(base, b + AHEAD, oa);
+      if (next) {
         pin(on.A[tn]);
-        P[kn % 2] = sums(on, tn, kn % 2);
+        P[kn % 2] = sums(on, tn, kn % RT);
         pin(P[kn % 2]);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -250,10 +289,10 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
 #pragma unroll
       for (int i = 0; i < 16; ++i) f[i] = (float)P[k % 2][i];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) f[i] = f[i] * SC[16 * r + i];  // cpu.rs:913,932: total += isum * (d_w * d_a)
+      for (int i = 0; i < 16; ++i) f[i] = f[i] * SC[16 * (k % 2) + i];  // cpu.rs:913,932: total += isum * (d_w * d_a)
       pin(f);
       __builtin_amdgcn_sched_barrier(0);
-      if (r == 1 && kn < 4 * kKB) {
+      if (k % 2 == 1 && next) {
         pin(on.da[tn]);
         SC = scales(on, tn);
         pin(SC);
@@ -262,11 +301,10 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[t][r][i] = acc[t][r][i] + f[i];
       pin(acc[t][r]);
-      if (k % 4 == 2 && k + 2 < 4 * kKB) {
-        GemmOps& ob = o[(k / 4 + 1) % 2];
-        unpack(ob);
-        pin(ob.B[0]);
-        pin(ob.B[1]);
+      if (k % NTB == NTB / 2 - (NTB == 2) && ahead) {
+        unpack(oa);
+#pragma unroll
+        for (int q = 0; q < RT; ++q) pin(oa.B[q]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -274,14 +312,15 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
   }
   const uint8_t* tail = lds + (nfull & 1) * S::BYTES;
   for (int b = 0; b < rest; ++b) {
-    GemmOps o;
-    load_ops(tail, b, o);
+    Ops o;
+    load_codes(tail, b, o);
+    load_scales(tail, b, o);
     unpack(o);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < TT; ++t) {
       const v32f sc = scales(o, t);
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
+      for (int r = 0; r < RT; ++r) {
         const v16i p = sums(o, t, r);
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[t][r][i] = acc[t][r][i] + (float)p[i] * sc[16 * r + i];
@@ -290,9 +329,9 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
   }
   if (WT != WT_Q8H) {  // the Q4 codes were 16 times theirs
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < TT; ++t)
 #pragma unroll
-      for (int r = 0; r < 2; ++r)
+      for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[t][r][i] = acc[t][r][i] * 0.0625f;
   }
@@ -300,11 +339,11 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
   // Epilogues.  Register i of a tile holds token 8 (i / 4) + 4 half + i % 4
   // and row col.
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
+  for (int t = 0; t < TT; ++t) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int tok = m0 + wm + 32 * t + 8 * (i / 4) + 4 * half + (i % 4);
-      if (EPI == EPI_SILU) {
+      const int m = m0 + wm + 32 * t + 8 * (i / 4) + 4 * half + (i % 4);
+      if constexpr (EPI == EPI_SILU) {
         // rows n0+wn .. +31 are gate, +32 .. +63 the matching up rows
         // (layer.rs:72-79); m index j = (n0+wn)/2 + col.
         const float g = acc[t][0][i], u = acc[t][1][i];
@@ -316,19 +355,21 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
         for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 32));
         const float d = amax / 127.0f;
         const float inv = amax == 0.0f ? 0.0f : 1.0f / d;
-        if (tok < a.M && n0 + wn < a.N) {
-          if (a.y) a.y[(size_t)tok * a.ldy + j] = mv;
-          a.yq[(size_t)tok * (a.N / 2) + j] = amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(mv, inv);
-          if (col == 0) a.yd[(size_t)tok * (a.N / 64) + run] = amax == 0.0f ? 0.0f : d;
+        if (m < a.M && n0 + wn < a.N) {
+          if (a.y) a.y[(size_t)m * a.ldy + j] = mv;
+          a.yq[act_row(m, a.N / 2, a.layout) + act_offset(j, a.layout)] =
+              amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(mv, inv);
+          if (col == 0)
+            a.yd[act_scale_row(m, a.N / 64, a.layout) + act_scale_offset(run, a.layout)] = amax == 0.0f ? 0.0f : d;
         }
       } else {
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-          const int row = n0 + wn + 32 * r + col;
-          if (tok < a.M && row < a.N) {
+        for (int r = 0; r < RT; ++r) {
+          const int n = n0 + row + 32 * r;
+          if (m < a.M && n < a.N) {
             float v = acc[t][r][i];
-            if (EPI == EPI_RESID) v = v + a.res[(size_t)tok * a.N + row];  // layer.rs:386,403
-            a.y[(size_t)tok * a.ldy + row] = v;
+            if (EPI == EPI_RESID) v = v + a.res[(size_t)m * a.N + n];  // layer.rs:386,403
+            a.y[(size_t)m * a.ldy + n] = v;
           }
         }
       }
@@ -336,22 +377,24 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
   }
 }
 
-// Dynamic LDS: two pipeline stages, gemm_lds_bytes(weights) at launch.
-static_assert(2 * GemmStage::BYTES == gemm_lds_bytes(), "GEMM LDS size");
-#define LLMRS_GEMM(name, WT, EPI)                                                 \
+// Kernels: gemm_<weights>_<epilogue>_<tokens>x<rows>; dynamic LDS of two stages.
+#define LLMRS_GEMM(name, WT, EPI, TT, RT)                                         \
   extern "C" __global__ __launch_bounds__(kGemmThreads, 2) void name(PrefillGemmArgs a) { \
     extern __shared__ __align__(16) uint8_t gemm_lds[];                            \
-    gemm_impl<WT, EPI>(a, gemm_lds);                                              \
+    gemm_impl<WT, EPI, TT, RT>(a, gemm_lds);                                      \
   }
-LLMRS_GEMM(gemm_q4h_store, WT_Q4H, EPI_STORE)
-LLMRS_GEMM(gemm_q4h_resid, WT_Q4H, EPI_RESID)
-LLMRS_GEMM(gemm_q4h_silu, WT_Q4H, EPI_SILU)
-LLMRS_GEMM(gemm_q4f_store, WT_Q4F, EPI_STORE)
-LLMRS_GEMM(gemm_q4f_resid, WT_Q4F, EPI_RESID)
-LLMRS_GEMM(gemm_q4f_silu, WT_Q4F, EPI_SILU)
-LLMRS_GEMM(gemm_q8h_store, WT_Q8H, EPI_STORE)
-LLMRS_GEMM(gemm_q8h_resid, WT_Q8H, EPI_RESID)
-LLMRS_GEMM(gemm_q8h_silu, WT_Q8H, EPI_SILU)
+#define LLMRS_GEMM_WT(tag, WT)                                  \
+  LLMRS_GEMM(gemm_##tag##_store_128x128, WT, EPI_STORE, 2, 2)   \
+  LLMRS_GEMM(gemm_##tag##_resid_128x128, WT, EPI_RESID, 2, 2)   \
+  LLMRS_GEMM(gemm_##tag##_silu_128x128, WT, EPI_SILU, 2, 2)     \
+  LLMRS_GEMM(gemm_##tag##_store_64x128, WT, EPI_STORE, 1, 2)    \
+  LLMRS_GEMM(gemm_##tag##_resid_64x128, WT, EPI_RESID, 1, 2)    \
+  LLMRS_GEMM(gemm_##tag##_silu_64x128, WT, EPI_SILU, 1, 2)      \
+  LLMRS_GEMM(gemm_##tag##_store_64x64, WT, EPI_STORE, 1, 1)     \
+  LLMRS_GEMM(gemm_##tag##_resid_64x64, WT, EPI_RESID, 1, 1)
+LLMRS_GEMM_WT(q4h, WT_Q4H)
+LLMRS_GEMM_WT(q4f, WT_Q4F)
+LLMRS_GEMM_WT(q8h, WT_Q8H)
 
 // Per-row RMSNorm + Q8_0 (w != null) or plain Q8_0 (w == null): the GEMV
 // prologue's arithmetic (same summation order), one workgroup per row, so a

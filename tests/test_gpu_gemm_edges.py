@@ -16,9 +16,15 @@ F32 = np.float32
 SKINNY = [(2, 16, 128), (15, 33, 128), (16, 64, 256), (17, 100, 384), (31, 1, 640), (33, 4112, 2176),
           (64, 8200, 512), (65, 130, 4224), (160, 72, 1024), (161, 72, 1024)]
 
+# the tile GEMM: 64 x 64, 64 x 128 and 128 x 128 tiles with ragged tokens and
+# rows, K of less than a stage (4 or 8 blocks), of whole stages and of every
+# kind of remainder
+TILES = [(130, 200, 32), (165, 100, 224), (161, 65, 256), (200, 33, 288), (1000, 4090, 416), (2047, 4095, 288),
+         (96, 6144, 1024), (100, 28672, 128)]
+
 
 @pytest.mark.parametrize("wtype", ["q4_0", "q4_ref", "q8_0"])
-@pytest.mark.parametrize("m,n,k", SKINNY)
+@pytest.mark.parametrize("m,n,k", SKINNY + TILES)
 def test_gemm_edges_bit_exact(hip, orc, rng, wtype, m, n, k):
     a = rng.normal(0, 1, (m, k)).astype(F32)
     a[0, :32] = 0.0

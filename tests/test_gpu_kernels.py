@@ -354,3 +354,13 @@ def test_prefill_layer_kernels_short(hip, orc, index, start, M):
     weights, the 70B widths, after a filled cache."""
     spec = syn.with_sizes(syn.WORKLOADS[index], n_layers=1, vocab=1024, prompt=M, decode=0, prefilled=0)
     check_prefill_layer(hip, orc, spec, start, M)
+
+
+@pytest.mark.timeout(900)
+@pytest.mark.parametrize("index,M", [(2, 100), (1, 100), (2, 48)], ids=["8b-100", "1b_q8-100", "8b-48"])
+def test_prefill_layer_kernels_mixed(hip, orc, index, M):
+    """Rows at which one layer takes the skinny GEMM for some projections and
+    the tile GEMM for others: the activation rows pass between them in the
+    consumer's operand order."""
+    spec = syn.with_sizes(syn.WORKLOADS[index], n_layers=1, vocab=1024, prompt=M, decode=0, prefilled=0)
+    check_prefill_layer(hip, orc, spec, 0, M)
