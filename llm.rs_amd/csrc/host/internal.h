@@ -163,10 +163,11 @@ GemvPlan gemv_plan(int wt, const std::string& kind, int n, int k, int num_cus);
 // Launch plan of one skinny GEMM (sgemm.hip; epi: store, resid, silu).
 struct SgemmPlan {
   std::string name;
-  unsigned grid = 1;
+  unsigned grid = 1, threads = 0;
+  double units = 0;  // estimated time per block of 32 (runtime.cpp)
 };
 bool sgemm_serves(size_t m, size_t k);
-bool sgemm_faster(const std::string& epi, int m, int n, int k, int num_cus);
+bool sgemm_faster(int wt, const std::string& epi, int m, int n, int k, int num_cus);
 SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus);
 // A tile GEMM launch (prefill.hip): kernel, grid of tiles, dynamic LDS.
 struct GemmPlan {

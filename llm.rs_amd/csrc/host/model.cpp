@@ -687,8 +687,8 @@ void ensure_prefill(llmrs_model* m) {
 // Operand order of the activation rows of a prefill linear layer: the skinny
 // GEMM's (sgemm.hip) or the tile GEMM's; both are bit-identical to the
 // reference's block loop, and each launch takes the faster.
-int prefill_layout(const char* epi, int M, const DevLinear& W) {
-  return sgemm_faster(epi, M, W.n, W.k, ctx().num_cus) ? llmrs::kActMfma : llmrs::kActNatural;
+int prefill_layout(const llmrs_model* m, const char* epi, int M, const DevLinear& W) {
+  return sgemm_faster(m->wt, epi, M, W.n, W.k, ctx().num_cus) ? llmrs::kActMfma : llmrs::kActNatural;
 }
 
 // Device buffers a test probe adds to one prefill layer: ctx and the SwiGLU
@@ -733,8 +733,8 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
     kc = Lb.kc;
     vc = Lb.vc;
   }
-  const int lay_qkv = prefill_layout("store", M, Lb.qkv), lay_o = prefill_layout("resid", M, Lb.o);
-  const int lay_gu = prefill_layout("silu", M, Lb.gu), lay_down = prefill_layout("resid", M, Lb.down);
+  const int lay_qkv = prefill_layout(m, "store", M, Lb.qkv), lay_o = prefill_layout(m, "resid", M, Lb.o);
+  const int lay_gu = prefill_layout(m, "silu", M, Lb.gu), lay_down = prefill_layout(m, "resid", M, Lb.down);
   // One linear layer over the M rows (operand order `layout`; the SwiGLU's
   // outputs in the order of the down projection).
   auto linear = [&](const char* epi, const DevLinear& W, int layout, const int8_t* xq, const float* xd, float* y,
@@ -743,7 +743,7 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
     if (layout == llmrs::kActMfma) {
       SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, lay_down};
       const SgemmPlan p = sgemm_plan(m->wt, epi, M, W.n, ctx().num_cus);
-      L(p.name, work, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
+      L(p.name, work, dim3(p.grid), dim3(p.threads), 0, g);
     } else {
       PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, M, W.n, W.k, ldy, gemm_group_m(), lay_down};
       const GemmPlan p = gemm_plan(m->wt, epi, M, W.n, ctx().num_cus);
@@ -1884,7 +1884,7 @@ int llmrs_model_probe_prefill_layer(llmrs_model* m, int layer, size_t start_pos,
     auto copy_act = [&](const char* epi, const DevLinear& W, int8_t* q, float* d, const int8_t* dev_q,
                         const float* dev_d) {
       const size_t K = W.k;
-      const int layout = prefill_layout(epi, (int)M, W);
+      const int layout = prefill_layout(m, epi, (int)M, W);
       const size_t rows = llmrs::act_rows(M);
       std::vector<int8_t> hq(rows * K);
       std::vector<float> hd(rows * K / 32);
@@ -2034,7 +2034,7 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
     } else if (b->skinny) {
       SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, W.n, b->layout};
       const SgemmPlan p = sgemm_plan(m->wt, epi, B, W.n, ctx().num_cus);
-      L(p.name, wb, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, g);
+      L(p.name, wb, dim3(p.grid), dim3(p.threads), 0, g);
     } else {
       PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, silu ? W.n / 2 : W.n, gemm_group_m(),
                         llmrs::kActNatural};

@@ -94,7 +94,7 @@ extern "C" int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmr
     // few rows of whole 128-element runs: the skinny GEMM, where its whole
     // 16-row tiles fit the scratch too
     size_t tile_off = 0;
-    const bool skinny = sgemm_faster("store", (int)m, (int)n, (int)k, cx.num_cus) &&
+    const bool skinny = sgemm_faster(b->wt, "store", (int)m, (int)n, (int)k, cx.num_cus) &&
                         scratch_need(act_rows(m), k, &tile_off) <= kNoAllocScratchBytes;
     if (skinny) scale_off = tile_off;
     int8_t* xq = (int8_t*)cx.noalloc_scratch;
@@ -105,7 +105,7 @@ extern "C" int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmr
       SgemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)out->data, nullptr, nullptr, nullptr,
                   (int)m, (int)n, (int)k, (int)n, kActMfma};
       const SgemmPlan p = sgemm_plan(b->wt, "store", (int)m, (int)n, cx.num_cus);
-      launch(p.name, dim3(p.grid), dim3(kSgemmThreads), 0, s, g);
+      launch(p.name, dim3(p.grid), dim3(p.threads), 0, s, g);
       return;
     }
     PrefillGemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)out->data, nullptr,

@@ -185,23 +185,6 @@ bool sgemm_serves(size_t m, size_t k) {
   return m <= 160 && k % 128 == 0 && !(e && *e == '0');
 }
 
-// Row tiles per workgroup (R = 1, 2 or 4 tiles of 16 rows; eight waves share
-// them): the most that still leave every CU two workgroups, since a
-// workgroup's rows share its activation loads (8B O and down at 23 rows: R = 1
-// 14.7 us, R = 2, 256 workgroups, 16.1); SwiGLU runs always span four.  The
-// grid deals eight row sets at a time, one per XCD, each over its token tiles.
-SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
-  const long nt = (m + 15) / 16;
-  int R = 4;
-  if (epi != "silu")
-    while (R > 1 && (n + 16 * R - 1) / (16 * R) * nt < 2 * num_cus) R /= 2;
-  const long rows = (n + 16 * R - 1) / (16 * R);
-  SgemmPlan p;
-  p.name = std::string("sgemm_") + wt_tag(wt) + "_" + epi + "_r" + std::to_string(R);
-  p.grid = (unsigned)(8 * nt * ((rows + 7) / 8));
-  return p;
-}
-
 namespace {
 struct GemmTile {
   int tt, rt;         // 64 tt tokens x 64 rt rows
@@ -243,18 +226,55 @@ GemmPlan gemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
   return p;
 }
 
-// Whether the skinny GEMM is the faster one for m rows that it can run: it
-// spreads one row of tiles over the chip, so its time per block grows with
-// n * m / 16, by 0.0061 of gemm_tile's units for 16 tokens x n = the number of
-// CUs; the tiles' time only with the fullest CU.  Skinny / tile, us: 8B gate|up
-// at 32 rows 42 / 52, 48 rows 60 / 53, 128 rows 138 / 76; O at 128 rows 22 /
-// 29, 160 rows 32 / 31; 1B gate|up at 64 rows 26 / 33, 100 rows 42 / 33, O at
-// 160 rows 11 / 18.
-bool sgemm_faster(const std::string& epi, int m, int n, int k, int num_cus) {
+// The skinny GEMM's kernel for m rows (16-token tiles) x n weight rows, and its
+// time per block of 32 in gemm_tile's units.  The split kernels spread any
+// shape over the chip: 0.0070 for one token tile and n = the number of CUs.
+// Their row tiles per workgroup (R = 1, 2 or 4 tiles of 16 rows; eight waves
+// share them) are the most that still leave every CU two workgroups, since a
+// workgroup's rows share its activation loads (8B O at 23 rows: R = 1 8.0 us,
+// R = 2, 256 workgroups, 8.9); SwiGLU runs always span four.  The wide kernels
+// (64 rows x 1, 2 or 3 token tiles, a wave's tiles its own) win where that
+// grid fills the chip, by the same sum over the fullest CU as the tile GEMM's.
+// Split / wide, us: 8B gate|up at 16 rows 22.9 / 20.4, 23 rows 41.6 / 29.0, 48
+// rows 61 / 39; 1B gate|up at 64 rows 25.6 / 18.1; 8B O at 16 rows 5.9 / 12.9.
+// Either grid deals eight row sets at a time, one per XCD, each over its token
+// tiles.
+SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
+  const long nt = (m + 15) / 16;
+  long R = 4;
+  if (epi != "silu")
+    while (R > 1 && (n + 16 * R - 1) / (16 * R) * nt < 2 * num_cus) R /= 2;
+  SgemmPlan p;
+  const std::string name = std::string("sgemm_") + wt_tag(wt) + "_" + epi;
+  auto deal = [&](long rows, long tokens) { return (unsigned)(8 * tokens * ((rows + 7) / 8)); };
+  p.name = name + "_r" + std::to_string(R);
+  p.grid = deal((n + 16 * R - 1) / (16 * R), nt);
+  p.threads = kSgemmThreads;
+  p.units = 0.0070 * n / num_cus * nt;
+  static const struct {
+    double lone, pair;
+  } kWide[] = {{0.40, 0.68}, {0.64, 1.0}, {0.95, 1.37}};
+  const long rows = (n + 63) / 64;
+  for (int tt = 1; tt <= (wt == WT_Q8H ? 2 : 3); ++tt) {  // three token tiles of Q8: one workgroup per CU
+    const long tokens = (nt + tt - 1) / tt, per_cu = (rows * tokens + num_cus - 1) / num_cus;
+    const double u = (double)(per_cu / 2) * kWide[tt - 1].pair + (double)(per_cu % 2) * kWide[tt - 1].lone;
+    if (u >= p.units) continue;
+    p.name = name + "_w" + std::to_string(tt);
+    p.grid = deal(rows, tokens);
+    p.threads = kWideThreads;
+    p.units = u;
+  }
+  return p;
+}
+
+// Whether the skinny GEMM is the faster one for m rows that it can run.
+// Skinny / tile, us: 8B gate|up at 48 rows 39 / 55, 96 rows 74 / 76; O at 128
+// rows 22 / 29, 160 rows 32 / 31; 1B gate|up at 64 rows 18 / 33.
+bool sgemm_faster(int wt, const std::string& epi, int m, int n, int k, int num_cus) {
   if (!sgemm_serves((size_t)m, (size_t)k)) return false;
   double units = 0;
   (void)gemm_tile(epi, m, n, num_cus, &units);
-  return 0.0061 * n / num_cus * ((m + 15) / 16) < units;
+  return sgemm_plan(wt, epi, m, n, num_cus).units < units;
 }
 
 // ---- allocator -------------------------------------------------------------

@@ -197,7 +197,7 @@ int llmrs_matmul_transposed(const llmrs_tensor* a, const llmrs_tensor* b, llmrs_
       LLMRS_REQUIRE(k <= 32768, LLMRS_E_INVALID, "matmul_transposed: k is limited to 32768");
       LLMRS_REQUIRE(m <= 65535 * 128, LLMRS_E_INVALID, "matmul_transposed: too many rows");
       hipStream_t s = ctx().stream;
-      const bool skinny = sgemm_faster("store", (int)m, (int)n, (int)k, ctx().num_cus);
+      const bool skinny = sgemm_faster(b->wt, "store", (int)m, (int)n, (int)k, ctx().num_cus);
       int8_t* xq = (int8_t*)ctx().alloc.alloc(llmrs::act_rows(m) * k);
       float* xd = (float*)ctx().alloc.alloc(llmrs::act_rows(m) * (k / 32) * sizeof(float));
       PrefillRowArgs r{(const float*)a->data, nullptr, xq, xd, (int)m, (int)k, 0.0f,
@@ -207,7 +207,7 @@ int llmrs_matmul_transposed(const llmrs_tensor* a, const llmrs_tensor* b, llmrs_
         SgemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)o->data, nullptr, nullptr, nullptr,
                     (int)m, (int)n, (int)k, (int)n, llmrs::kActMfma};
         const SgemmPlan p = sgemm_plan(b->wt, "store", (int)m, (int)n, ctx().num_cus);
-        launch(p.name, dim3(p.grid), dim3(llmrs::kSgemmThreads), 0, s, g);
+        launch(p.name, dim3(p.grid), dim3(p.threads), 0, s, g);
       } else {
         PrefillGemmArgs g{xq, xd, (const uint8_t*)b->data, b->scales, (float*)o->data, nullptr,
                           nullptr, nullptr, (int)m, (int)n, (int)k, (int)n, gemm_group_m(), llmrs::kActNatural};

@@ -99,7 +99,8 @@ constexpr size_t act_rows(size_t M) { return (M + 15) / 16 * 16; }
 // sum_b isum_b(t, n) * (d_w[n,b] * d_a[t,b]) over M rows of Q8_0 activation
 // codes (in the operand order kActMfma) and an [N, K] quantised weight, K a
 // multiple of 128.
-constexpr int kSgemmThreads = 512;
+constexpr int kSgemmThreads = 512;  // the split kernels: eight waves
+constexpr int kWideThreads = 256;   // the wide ones: four
 struct SgemmArgs {
   const int8_t* xq;      // [M][K] activation codes, order kActMfma
   const float* xd;       // [M][K/32] activation scales, order kActMfma

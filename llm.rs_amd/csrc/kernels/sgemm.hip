@@ -47,6 +47,8 @@
 // 15, 62 -> 19, 80 -> 52.  The rounds' phases (loads, products, LDS, adds)
 // overlap only across the two workgroups of a CU.
 
+#include <type_traits>
+
 #include "common.h"
 #include "exact_math.h"
 #include "gemv_core.h"
@@ -317,6 +319,250 @@ __device__ __forceinline__ void sgemm_impl(const SgemmArgs& a) {
   }
 }
 
+// ---- wide layers -------------------------------------------------------------
+// Where 64-row sets fill the chip (gate|up, the head of a batch), a wave keeps
+// 16 rows x 16 TT tokens to itself and adds its terms in block order in
+// registers, with no hand-over through LDS.  A workgroup of four waves (64
+// rows) streams eight blocks a stage: weights, activation codes (shared by the
+// waves) and scales go to LDS by direct loads, two or three stages ahead, so
+// that the loads in flight cover the memory's latency without registers; the
+// matrix instructions run one product ahead of the arithmetic.  The serial
+// chain of a stage (LDS reads, transposes, products, additions: 0.7 us for one
+// token tile) bounds it while a SIMD holds one or two waves.
+// Measured (gate|up, us, split kernel -> wide): 8B 16 rows 22.9 -> 20.4 (66
+// MB: 3.2 TB/s), 23 rows 41.6 -> 29.0, 48 rows 61 (tile GEMM 55) -> 39; 1B 64
+// rows 25.6 -> 18.1.
+template <int WT, int TT>
+struct WideStage {
+  static constexpr int RC = kStep * (WT == WT_Q8H ? 2 : 1);  // 16-byte chunks of a row
+  static constexpr int SD = WT == WT_Q4F ? 8 : 4;            // scale dwords of a row (f16: two scales each)
+  static constexpr int X = 0;                                // codes [TT][4 KB]
+  static constexpr int DA = X + TT * 4096;                   // scales [TT][8 blocks][16 tokens]
+  static constexpr int W = DA + TT * 512;                    // codes [64 rows][RC]
+  static constexpr int DW = W + 64 * RC * 16;                // scales [64 rows][SD]
+  static constexpr int BYTES = DW + 64 * SD * 4;
+  static constexpr int LOADS = TT + 1 + RC / 4 + SD / 4;     // per wave
+  static constexpr int N = WT == WT_Q8H || TT == 3 ? 3 : 4;  // buffers
+  static_assert(N * BYTES <= 80 * 1024, "two workgroups per CU");
+};
+
+// The value is computed here and read after here.
+template <typename T>
+__device__ __forceinline__ void pin(T& x) {
+  asm volatile("" : "+v"(x));
+}
+
+__device__ __forceinline__ void load_lds16(const void* src, uint8_t* lds) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+__device__ __forceinline__ void load_lds4(const void* src, uint8_t* lds) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)lds, 4, 0, 0);
+}
+
+template <int WT, int EPI, int TT>
+__device__ __forceinline__ void wide_impl(const SgemmArgs& a, uint8_t* lds) {
+  typedef WideStage<WT, TT> S;
+  constexpr int BCH = WT == WT_Q8H ? 2 : 1, RC = S::RC, SD = S::SD;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int nb = a.K >> 5, nst = (nb + kStep - 1) / kStep;
+  const int nt = (a.M + 16 * TT - 1) / (16 * TT), nrow = (a.N + 63) / 64;
+  const int slot = blockIdx.x >> 3, ty = slot % nt, tx = (slot / nt) * 8 + (blockIdx.x & 7);
+  if (tx >= nrow) return;
+  const int tile0 = ty * TT, tiles = (a.M + 15) >> 4, n0 = tx * 64;
+
+  // Stage st into its buffer.  Rows past N and token tiles past M are the last
+  // one again, blocks past the row's end (nb is a multiple of 4) a valid run;
+  // none of them is added or stored.
+  const uint8_t* wbase = a.wq + (size_t)n0 * nb * (16 * BCH);
+  const uint8_t* dbase = (const uint8_t*)a.ws + (size_t)n0 * nb * (SD / 2);
+  unsigned woff[RC / 4], doff[SD / 4];  // of the lane's chunk c of row i, at c ^ (i & 7), and its scales
+  int wblk[RC / 4], dblk[SD / 4];       // their first block in a stage
+#pragma unroll
+  for (int j = 0; j < RC / 4; ++j) {
+    const int p = 64 * j + lane, i = p / RC, c = (p % RC) ^ (i & 7);
+    woff[j] = (unsigned)(min(n0 + 16 * w + i, a.N - 1) - n0) * (unsigned)(nb * 16 * BCH) + 16 * c;
+    wblk[j] = c / BCH;
+  }
+#pragma unroll
+  for (int j = 0; j < SD / 4; ++j) {
+    const int p = 64 * j + lane;
+    doff[j] = (unsigned)(min(n0 + 16 * w + p / SD, a.N - 1) - n0) * (unsigned)(nb * SD / 2) + 4 * (p % SD);
+    dblk[j] = (p % SD) * (8 / SD);
+  }
+  constexpr int DV = (TT + 1) / 2;  // waves that cover the 32 TT chunks of d_a; the others repeat them
+  const int dq = 64 * (w % DV) + lane;
+  auto load_stage = [&](int st) {
+    uint8_t* base = lds + (st % S::N) * S::BYTES;
+    const int b0 = st * kStep;
+    auto load = [&](bool part) {
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const size_t tile = min(tile0 + t, tiles - 1);
+        load_lds16(a.xq + (tile * 16 * a.K + (size_t)b0 * 512) + (unsigned)(16 * (part ? tid & 127 : tid)),
+                   base + S::X + t * 4096 + 1024 * w);
+      }
+      if (dq / 32 < TT) {
+        const size_t tile = min(tile0 + dq / 32, tiles - 1);
+        load_lds16(a.xd + (size_t)b0 * 16 + tile * 16 * nb + 4 * (dq & (part ? 15 : 31)),
+                   base + S::DA + 1024 * (w % DV));
+      }
+#pragma unroll
+      for (int j = 0; j < RC / 4; ++j) {
+        const int back = part ? max(b0 + wblk[j] - (nb - 1), 0) : 0;
+        load_lds16(wbase + (size_t)b0 * (16 * BCH) + (woff[j] - (unsigned)(16 * BCH * back)),
+                   base + S::W + (16 * w * RC + 64 * j) * 16);
+      }
+#pragma unroll
+      for (int j = 0; j < SD / 4; ++j) {
+        const int back = part ? max(b0 + dblk[j] - (nb - 8 / SD), 0) : 0;
+        load_lds4(dbase + (size_t)b0 * (SD / 2) + (doff[j] - (unsigned)(SD / 2 * back)),
+                  base + S::DW + (16 * w * SD + 64 * j) * 4);
+      }
+    };
+    if (b0 + kStep <= nb) load(false);
+    else load(true);
+  };
+
+  float acc[TT][4];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[t][i] = 0.0f;
+
+  // The first 4 NU blocks of a stage: products q = TT u + t, token tile t of
+  // blocks 4 u .. 4 u + 3.  The matrix instructions of product q + 1 are issued
+  // before the arithmetic of q, and its operands read another one before.
+  auto compute = [&](const uint8_t* base, auto nu) {
+    constexpr int NU = decltype(nu)::value, Q = NU * TT;
+    const u32x4* sw = (const u32x4*)(base + S::W) + (16 * w + r) * RC;
+    const uint8_t* sd = base + S::DW + (16 * w + r) * SD * 4;
+    SgOperands op[NU];
+    SgTokens X[3];
+    auto tokens = [&](int q) {
+      const u32x4* sx = (const u32x4*)(base + S::X + (q % TT) * 4096 + (q / TT) * 2048);
+      X[q % 3].x[0][0] = sx[lane];
+      X[q % 3].x[0][1] = sx[64 + lane];
+      X[q % 3].da[0] = ((const float*)(base + S::DA + (q % TT) * 512))[64 * (q / TT) + lane];
+    };
+    tokens(0);
+    if (Q > 1) tokens(1);
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const u32x4 w0 = sw[((4 * u + g) * BCH) ^ (r & 7)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) op[u].lo[j] = w0[j];
+      transpose4(op[u].lo);
+      if constexpr (WT == WT_Q8H) {
+        const u32x4 w1 = sw[((4 * u + g) * BCH + 1) ^ (r & 7)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) op[u].hi[j] = w1[j];
+        transpose4(op[u].hi);
+      } else {  // 16 (q - 8) in a byte's upper half
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          op[u].hi[j] = (op[u].lo[j] & 0xF0F0F0F0u) ^ 0x80808080u;
+          op[u].lo[j] = ((op[u].lo[j] << 4) & 0xF0F0F0F0u) ^ 0x80808080u;
+        }
+      }
+      op[u].dw = wscale<WT>(WT == WT_Q4F ? ((const unsigned*)sd)[4 * u + g] : ((const uint16_t*)sd)[4 * u + g]);
+    }
+    v16f sc[2];
+    i32x4 isum[2][4];
+    auto issue = [&](int q) {
+      const SgTokens& x = X[q % 3];
+      const SgOperands& o = op[q / TT];
+      sc[q % 2] = __builtin_amdgcn_mfma_f32_16x16x1f32(o.dw, x.da[0], v16f{}, 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const long oa = (long)((unsigned long long)o.lo[j] | ((unsigned long long)o.hi[j] << 32));
+        const long ob = (long)((unsigned long long)x.x[0][j >> 1][2 * (j & 1)] |
+                               ((unsigned long long)x.x[0][j >> 1][2 * (j & 1) + 1] << 32));
+        isum[q % 2][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(oa, ob, i32x4{0, 0, 0, 0}, 0, 0, 0);
+      }
+      pin(sc[q % 2]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pin(isum[q % 2][j]);
+    };
+    issue(0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      if (q + 2 < Q) tokens(q + 2);
+      if (q + 1 < Q) {
+        pin(X[(q + 1) % 3].da[0]);
+        pin(X[(q + 1) % 3].x[0][0]);
+        pin(X[(q + 1) % 3].x[0][1]);
+        issue(q + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      float (&s)[4] = acc[q % TT];
+      pin(sc[q % 2]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        pin(isum[q % 2][j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] = s[i] + (float)isum[q % 2][j][i] * sc[q % 2][4 * j + i];  // cpu.rs:930-935
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pin(s[i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  for (int st = 0; st < S::N - 1 && st < nst; ++st) load_stage(st);
+  for (int st = 0; st < nst; ++st) {
+    // This wave's loads of stage st, then everyone's; the barrier also ends the
+    // reads of stage st - 1, whose buffer the next loads take.
+    if (st + S::N - 1 <= nst) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S::N - 2) * S::LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (st + S::N - 1 < nst) load_stage(st + S::N - 1);
+    const uint8_t* base = lds + (st % S::N) * S::BYTES;
+    if ((st + 1) * kStep <= nb) compute(base, std::integral_constant<int, 2>{});
+    else compute(base, std::integral_constant<int, 1>{});
+  }
+  if (WT != WT_Q8H) {  // the Q4 codes were 16 times theirs
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[t][i] = acc[t][i] * 0.0625f;
+  }
+
+  // token t's 64 rows side by side
+  constexpr int LD = 65;
+  float* s_o = (float*)lds;
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_o[(16 * t + r) * LD + 16 * w + 4 * g + i] = acc[t][i];
+  __syncthreads();
+  if constexpr (EPI == EPI_SILU) {
+    // 32 gate rows, then their up rows (layer.rs:72-79)
+#pragma unroll
+    for (int p = 0; p < 2 * TT; ++p) {
+      const int t = 8 * p + (tid >> 5), j = tid & 31;
+      const float gv = s_o[t * LD + j], uv = s_o[t * LD + 32 + j];
+      const float mv = (gv / (1.0f + exact_expf(-gv))) * uv;  // glibc expf (exact_math.h)
+      swiglu_out(a, 16 * tile0 + t, tx, j, mv);
+    }
+  } else {
+#pragma unroll
+    for (int p = 0; p < 4 * TT; ++p) {
+      const int lt = 4 * p + w, t = 16 * tile0 + lt, n = n0 + lane;
+      if (t < a.M && n < a.N) {
+        float v = s_o[lt * LD + lane];
+        if (EPI == EPI_RESID) v = v + a.res[(size_t)t * a.N + n];  // layer.rs:386,403
+        a.y[(size_t)t * a.ldy + n] = v;
+      }
+    }
+  }
+}
+
 }  // namespace
 
 // Kernels: sgemm_<weights>_<epilogue>_r<row tiles per workgroup>.
@@ -333,3 +579,22 @@ __device__ __forceinline__ void sgemm_impl(const SgemmArgs& a) {
 LLMRS_SGEMM_WT(q4h, WT_Q4H)
 LLMRS_SGEMM_WT(q4f, WT_Q4F)
 LLMRS_SGEMM_WT(q8h, WT_Q8H)
+
+// Kernels: sgemm_<weights>_<epilogue>_w<token tiles per workgroup>.
+#define LLMRS_WIDE(name, WT, EPI, TT)                                                  \
+  extern "C" __global__ __launch_bounds__(kWideThreads, 2) void name(SgemmArgs a) {    \
+    __shared__ __align__(16) uint8_t wide_lds[WideStage<WT, TT>::N * WideStage<WT, TT>::BYTES]; \
+    wide_impl<WT, EPI, TT>(a, wide_lds);                                               \
+  }
+#define LLMRS_WIDE_TT(tag, WT, TT)                            \
+  LLMRS_WIDE(sgemm_##tag##_store_w##TT, WT, EPI_STORE, TT)    \
+  LLMRS_WIDE(sgemm_##tag##_resid_w##TT, WT, EPI_RESID, TT)    \
+  LLMRS_WIDE(sgemm_##tag##_silu_w##TT, WT, EPI_SILU, TT)
+LLMRS_WIDE_TT(q4h, WT_Q4H, 1)
+LLMRS_WIDE_TT(q4h, WT_Q4H, 2)
+LLMRS_WIDE_TT(q4h, WT_Q4H, 3)
+LLMRS_WIDE_TT(q4f, WT_Q4F, 1)
+LLMRS_WIDE_TT(q4f, WT_Q4F, 2)
+LLMRS_WIDE_TT(q4f, WT_Q4F, 3)
+LLMRS_WIDE_TT(q8h, WT_Q8H, 1)
+LLMRS_WIDE_TT(q8h, WT_Q8H, 2)

@@ -21,10 +21,14 @@ SKINNY = [(2, 16, 128), (15, 33, 128), (16, 64, 256), (17, 100, 384), (31, 1, 64
 # kind of remainder
 TILES = [(130, 200, 32), (165, 100, 224), (161, 65, 256), (200, 33, 288), (1000, 4090, 416), (2047, 4095, 288),
          (96, 6144, 1024), (100, 28672, 128)]
+# the skinny GEMM's wide kernels: one, two and three token tiles with ragged
+# last ones, rows past a 64-row set, less than a stage of eight blocks, half
+# stages at the end, fewer stages than buffers and more
+WIDE = [(2, 32770, 128), (16, 32000, 384), (23, 28700, 640), (32, 28672, 256), (48, 28700, 1152), (64, 16400, 896)]
 
 
 @pytest.mark.parametrize("wtype", ["q4_0", "q4_ref", "q8_0"])
-@pytest.mark.parametrize("m,n,k", SKINNY + TILES)
+@pytest.mark.parametrize("m,n,k", SKINNY + TILES + WIDE)
 def test_gemm_edges_bit_exact(hip, orc, rng, wtype, m, n, k):
     a = rng.normal(0, 1, (m, k)).astype(F32)
     a[0, :32] = 0.0
