@@ -720,11 +720,10 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
     if (probe && probe->after) probe->after(stage);
   };
   const float scale = 1.0f / std::sqrt((float)hd);  // layer.rs:258
-  // f16 caches use the matrix-core kernel (LLMRS_PREFILL_ATTN=valu selects the
-  // vector kernel, which also serves f32 caches)
+  // LLMRS_PREFILL_ATTN=valu selects the vector kernels
   const char* pa = std::getenv("LLMRS_PREFILL_ATTN");
-  const bool mfma_attn = kv16 && !(pa && std::string(pa) == "valu");
-  const std::string attn = mfma_attn ? "attn_prefill_mfma_hd" + std::to_string(hd)
+  const bool mfma_attn = !(pa && std::string(pa) == "valu");
+  const std::string attn = mfma_attn ? "attn_prefill_mfma_hd" + std::to_string(hd) + (kv16 ? "" : "_f32")
                                      : "attn_prefill_hd" + std::to_string(hd) + (kv16 ? "_f16" : "_f32");
   // causal score and P.V products over the chunk
   const double attn_flops = 4.0 * nq * hd * ((double)M * start + (double)M * (M + 1) / 2.0);
@@ -773,7 +772,7 @@ void enqueue_prefill_layer(llmrs_model* m, Launcher& L, int li, size_t start, in
     if (exact)  // one workgroup per (query head, row); the scores of up to start + M positions in LDS
       L("exact_attn_prefill_hd" + std::to_string(hd) + (kv16 ? "_f16" : "_f32"), attn_flops,
         dim3((unsigned)nq, (unsigned)M), blk, (start + M) * 4, a);
-    else if (mfma_attn)
+    else if (mfma_attn && kv16)
       L(attn, attn_flops, dim3((unsigned)((M + 31) / 32), (unsigned)nkv), dim3(512), 0, a);
     else
       L(attn, attn_flops, dim3((unsigned)((M + 31) / 32), (unsigned)nq), blk, 0, a);

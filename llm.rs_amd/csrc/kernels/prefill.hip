@@ -43,7 +43,7 @@
 // (their additions have an order).  64 x 128 (a wave: one token tile, two row
 // tiles) and 64 x 64 (one tile, its scales two blocks at a time) give more and
 // shorter chains, in stages of eight blocks; gemm_plan (runtime.cpp) picks one.
-// 1B, 700 tokens, us: down 163 -> 74, O 55 -> 24, Q|K|V 43 -> 18.
+// 1B, 700 tokens, us: down 163 -> 74, O 55 -> 24, Q|K|V 43 -> 33.
 #include "attn_core.h"
 #include "exact_math.h"
 #include "gemv_core.h"
@@ -862,6 +862,150 @@ __device__ __forceinline__ void attn_prefill_mfma_impl(const PrefillAttnArgs& a)
       }
     }
   }
+}
+
+// Causal prefill attention on the matrix cores, f32 K/V cache: one workgroup of
+// four waves per (32-query tile, query head), wave w taking key tiles w, w + 4,
+// ... of 32 keys, so a wave works without barriers until the four streams'
+// (max, sum, O) are merged through LDS.  Everything stays f32:
+//   S^T = K Q^T        v_mfma_f32_32x32x2f32: lane (col, half) holds dims
+//                       half * HD/2 .. of key / query col, so step s takes dims
+//                       s and HD/2 + s
+//   online softmax      one query per lane column, as in the f16 kernel
+//   O^T += V^T P^T      register i of S^T holds keys 8 (i/4) + i%4 (lower half)
+//                       and + 4 (upper half): step i takes those two
+// K rows are read as 16-byte pieces of a lane's own row and V as whole lines; V
+// is requested before the scores and the next K after them, so a tile's 2 HD/2
+// matrix instructions (64 cycles each) cover the reads.  They bound it: 700 rows
+// of the 1B shape need 14 us at the f32 matrix rate and take 51, 2048 rows 319
+// (the longest query tile's streams end last); the vector kernel's dots
+// and P.V (four multiply-adds per LDS read) took 104 and 655.
+template <int HD>
+__device__ __forceinline__ void attn_prefill_f32_impl(const PrefillAttnArgs& a) {
+  constexpr int ND = HD / 32, HH = HD / 2, KT = 32, NSTR = 4;
+  __shared__ float s_o[NSTR][16 * ND][LLMRS_WAVE];
+  __shared__ float s_ml[NSTR][2][LLMRS_WAVE];
+  const int lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int h2 = lane >> 5, col = lane & 31;
+  const int q0 = (gridDim.x - 1 - blockIdx.x) * 32, h = blockIdx.y;  // longest tiles first
+  const int g = h / (a.nq / a.nkv), qdim = a.nq * HD;
+  const float* kc = (const float*)a.kc + (size_t)g * a.max_seq * HD;
+  const float* vc = (const float*)a.vc + (size_t)g * a.max_seq * HD;
+  const int kend = a.start_pos + min(q0 + 32, a.M);  // keys [0, kend)
+  const int ntile = (kend + KT - 1) / KT;
+  const int myq = q0 + col, qpos = a.start_pos + myq;
+
+  float q[HH], k[HH], v[ND][16];
+  auto load_row = [&](const float* row, float (&x)[HH]) {
+#pragma unroll
+    for (int j = 0; j < HH / 4; ++j) {
+      const f32x4 t = *(const f32x4*)(row + HH * h2 + 4 * j);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[4 * j + c] = t[c];
+    }
+  };
+  auto load_k = [&](int kt) { load_row(kc + (size_t)min(kt * KT + col, kend - 1) * HD, k); };
+  load_row(a.q + (size_t)min(myq, a.M - 1) * qdim + (size_t)h * HD, q);
+  if (w < ntile) load_k(w);
+  v16f o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) o[d] = v16f{};
+  float m = -INFINITY, l = 0.0f;
+  for (int kt = w; kt < ntile; kt += NSTR) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int key = min(kt * KT + 8 * (i / 4) + 4 * h2 + (i % 4), kend - 1);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) v[d][i] = vc[(size_t)key * HD + 32 * d + col];
+    }
+    v16f st = v16f{};
+#pragma unroll
+    for (int s = 0; s < HH; ++s) st = __builtin_amdgcn_mfma_f32_32x32x2f32(k[s], q[s], st, 0, 0, 0);
+    if (kt + NSTR < ntile) load_k(kt + NSTR);
+    float p[16];
+    float mloc = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int key = kt * KT + 8 * (i / 4) + 4 * h2 + (i % 4);
+      p[i] = key <= qpos && key < kend ? st[i] * a.scale : -INFINITY;
+      mloc = fmaxf(mloc, p[i]);
+    }
+    mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
+    const float mn = fmaxf(m, mloc);  // -inf while every key so far is masked
+    const float corr = m == -INFINITY ? 0.0f : expf(m - mn);
+    float lsum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      p[i] = p[i] == -INFINITY ? 0.0f : expf(p[i] - mn);
+      lsum += p[i];
+    }
+    lsum += __shfl_xor(lsum, 32);
+    l = l * corr + lsum;
+    m = mn;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[d][i] *= corr;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[d][i], p[i], o[d], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s_o[w][16 * d + i][lane] = o[d][i];
+  s_ml[w][0][lane] = m;
+  s_ml[w][1][lane] = l;
+  __syncthreads();
+  // Wave d merges and writes dims 32 d ..: register i is dim 8 (i/4) + 4 h2 + i%4.
+  if (w >= ND) return;
+  float mm = -INFINITY, c[NSTR];
+#pragma unroll
+  for (int s = 0; s < NSTR; ++s) mm = fmaxf(mm, s_ml[s][0][lane]);  // finite: key 0 is seen
+  l = 0.0f;
+#pragma unroll
+  for (int s = 0; s < NSTR; ++s) {
+    const float ms = s_ml[s][0][lane];
+    c[s] = ms == -INFINITY ? 0.0f : expf(ms - mm);
+    l += s_ml[s][1][lane] * c[s];
+  }
+  float x[16], amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    float t = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NSTR; ++s) t += s_o[s][16 * w + i][lane] * c[s];
+    x[i] = t / l;
+    amax = fmaxf(amax, fabsf(x[i]));
+  }
+  amax = fmaxf(amax, __shfl_xor(amax, 32));
+  const float dq = amax / 127.0f;
+  const float inv = amax == 0.0f ? 0.0f : 1.0f / dq;
+  if (myq >= a.M) return;
+#pragma unroll
+  for (int gq = 0; gq < 4; ++gq) {
+    const int e = h * HD + 32 * w + 8 * gq + 4 * h2;
+    unsigned word = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int q8 = amax == 0.0f ? 0 : q8_code(x[4 * gq + b], inv);
+      word |= ((unsigned)q8 & 0xFFu) << (8 * b);
+    }
+    *(unsigned*)(a.ctx_q + act_row(myq, qdim, a.ctx_layout) + act_offset(e, a.ctx_layout)) = word;
+    if (a.ctx)
+      *(f32x4*)(a.ctx + (size_t)myq * qdim + e) = f32x4{x[4 * gq], x[4 * gq + 1], x[4 * gq + 2], x[4 * gq + 3]};
+  }
+  if (h2 == 0)
+    a.ctx_d[act_scale_row(myq, qdim / 32, a.ctx_layout) + act_scale_offset(h * HD / 32 + w, a.ctx_layout)] =
+        amax == 0.0f ? 0.0f : dq;
+}
+
+extern "C" __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_hd64_f32(PrefillAttnArgs a) {
+  attn_prefill_f32_impl<64>(a);
+}
+extern "C" __global__ __launch_bounds__(256, 1) void attn_prefill_mfma_hd128_f32(PrefillAttnArgs a) {
+  attn_prefill_f32_impl<128>(a);
 }
 
 extern "C" __global__ __launch_bounds__(512) void attn_prefill_mfma_hd64(PrefillAttnArgs a) {

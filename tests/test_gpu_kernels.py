@@ -364,3 +364,12 @@ def test_prefill_layer_kernels_mixed(hip, orc, index, M):
     consumer's operand order."""
     spec = syn.with_sizes(syn.WORKLOADS[index], n_layers=1, vocab=1024, prompt=M, decode=0, prefilled=0)
     check_prefill_layer(hip, orc, spec, 0, M)
+
+
+@pytest.mark.parametrize("head_dim,start,M", [(64, 0, 2), (64, 31, 33), (64, 0, 129), (128, 300, 70), (128, 0, 97)])
+def test_prefill_attention_f32_cache(hip, orc, head_dim, start, M):
+    """The f32-cache prefill attention at the edges of its 32-query and 32-key
+    tiles and its four key streams: fewer tiles than streams, ragged last
+    tiles, after a filled cache."""
+    spec = syn.tiny(DType.Q4_0, DType.F32, head_dim=head_dim, n_heads=8, n_kv_heads=2, ffn=1024, prompt=M, decode=0)
+    check_prefill_layer(hip, orc, syn.with_sizes(spec, n_layers=1), start, M)
