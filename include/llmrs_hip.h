@@ -156,6 +156,23 @@ int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmrs_tensor* b
  * host libm (glibc) computes it, bit for bit. */
 int llmrs_probe_expf(const float* x, size_t n, float* out);
 
+/* Test probes (no reference counterpart) of the several-row GEMMs.  A kernel is
+ * a weight type (q4h, q4f: 4-bit codes with f16 / f32 scales; q8h), an
+ * epilogue (store, resid, silu) and a variant: r1, r2, r4 or w1, w2, w3 of the
+ * skinny GEMM, 128x128, 64x128 or 64x64 tiles.
+ * llmrs_probe_gemm_plan: the kernel name (up to 64 bytes) and the grid that m
+ * rows through an [n, k] weight take on a device of num_cus compute units; needs
+ * no device.
+ * llmrs_probe_gemm: one launch of a given kernel on the rows of the f32 tensor
+ * a [m, k], for shapes it accepts: y [m, n] (store; resid: plus `res` [m, n],
+ * in place), or for silu (rows of w in runs of 32 gate rows, then their 32 up
+ * rows) y [m, n/2] with its Q8_0 codes yq and scales yd [m, n/64], stored in the
+ * skinny GEMM's operand order (order 1) or as rows (0) and returned as rows. */
+int llmrs_probe_gemm_plan(const char* weight, const char* epi, size_t m, size_t n, size_t k, int num_cus,
+                          char* name, uint32_t grid[2]);
+int llmrs_probe_gemm(const llmrs_tensor* a, const llmrs_tensor* w, const llmrs_tensor* res, const char* epi,
+                     const char* variant, int order, float* y, int8_t* yq, float* yd);
+
 /* ---- resident decode model (no trait counterpart) ----------------------- */
 /* Mirrors LlamaConfig (src/core/config.rs:3-17) plus what the reference
  * hard-codes: head_dim (loader.rs:164 derives hidden/num_heads), max_seq

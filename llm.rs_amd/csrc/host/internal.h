@@ -169,6 +169,10 @@ struct SgemmPlan {
 bool sgemm_serves(size_t m, size_t k);
 bool sgemm_faster(int wt, const std::string& epi, int m, int n, int k, int num_cus);
 SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus);
+// One of its kernels whatever the rule says: R row tiles shared by a workgroup's
+// waves, or tt token tiles per wave.
+SgemmPlan sgemm_split_plan(int wt, const std::string& epi, int m, int n, int R);
+SgemmPlan sgemm_wide_plan(int wt, const std::string& epi, int m, int n, int tt);
 // A tile GEMM launch (prefill.hip): kernel, grid of tiles, dynamic LDS.
 struct GemmPlan {
   std::string name;
@@ -176,6 +180,8 @@ struct GemmPlan {
   size_t lds;
 };
 GemmPlan gemm_plan(int wt, const std::string& epi, int m, int n, int num_cus);
+// One tile whatever the rule says: 64 tt tokens x 64 rt rows.
+GemmPlan gemm_tile_plan(int wt, const std::string& epi, int m, int n, int tt, int rt);
 // LDS bytes of a GEMV's activation area (codes, scales, Q4 offsets) for input length k.
 inline size_t gemv_act_lds_host(int k) { return (size_t)k + 8 * (size_t)(k / 32); }
 

@@ -215,14 +215,38 @@ const GemmTile& gemm_tile(const std::string& epi, int m, int n, int num_cus, dou
 }
 }  // namespace
 
-GemmPlan gemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
-  double units = 0;
-  const GemmTile& t = gemm_tile(epi, m, n, num_cus, &units);
-  const int bm = 64 * t.tt, bn = 64 * t.rt, bch = wt == WT_Q8H ? 2 : 1;
+GemmPlan gemm_tile_plan(int wt, const std::string& epi, int m, int n, int tt, int rt) {
+  const int bm = 64 * tt, bn = 64 * rt, bch = wt == WT_Q8H ? 2 : 1;
   GemmPlan p;
   p.name = std::string("gemm_") + wt_tag(wt) + "_" + epi + "_" + std::to_string(bm) + "x" + std::to_string(bn);
   p.grid = dim3((unsigned)((n + bn - 1) / bn), (unsigned)((m + bm - 1) / bm));
-  p.lds = gemm_lds_bytes(t.tt, t.rt, gemm_stage_blocks(t.tt, t.rt, bch), bch);
+  p.lds = gemm_lds_bytes(tt, rt, gemm_stage_blocks(tt, rt, bch), bch);
+  return p;
+}
+
+GemmPlan gemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
+  double units = 0;
+  const GemmTile& t = gemm_tile(epi, m, n, num_cus, &units);
+  return gemm_tile_plan(wt, epi, m, n, t.tt, t.rt);
+}
+
+// Either grid of the skinny GEMM deals eight row sets at a time, one per XCD,
+// each over its token tiles.
+static unsigned sgemm_deal(long rows, long tokens) { return (unsigned)(8 * tokens * ((rows + 7) / 8)); }
+
+SgemmPlan sgemm_split_plan(int wt, const std::string& epi, int m, int n, int R) {
+  SgemmPlan p;
+  p.name = std::string("sgemm_") + wt_tag(wt) + "_" + epi + "_r" + std::to_string(R);
+  p.grid = sgemm_deal(((long)n + 16 * R - 1) / (16 * R), (m + 15) / 16);
+  p.threads = kSgemmThreads;
+  return p;
+}
+
+SgemmPlan sgemm_wide_plan(int wt, const std::string& epi, int m, int n, int tt) {
+  SgemmPlan p;
+  p.name = std::string("sgemm_") + wt_tag(wt) + "_" + epi + "_w" + std::to_string(tt);
+  p.grid = sgemm_deal(((long)n + 63) / 64, (m + 16 * tt - 1) / (16 * tt));
+  p.threads = kWideThreads;
   return p;
 }
 
@@ -237,19 +261,12 @@ GemmPlan gemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
 // grid fills the chip, by the same sum over the fullest CU as the tile GEMM's.
 // Split / wide, us: 8B gate|up at 16 rows 22.9 / 20.4, 23 rows 41.6 / 29.0, 48
 // rows 61 / 39; 1B gate|up at 64 rows 25.6 / 18.1; 8B O at 16 rows 5.9 / 12.9.
-// Either grid deals eight row sets at a time, one per XCD, each over its token
-// tiles.
 SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
   const long nt = (m + 15) / 16;
-  long R = 4;
+  int R = 4;
   if (epi != "silu")
-    while (R > 1 && (n + 16 * R - 1) / (16 * R) * nt < 2 * num_cus) R /= 2;
-  SgemmPlan p;
-  const std::string name = std::string("sgemm_") + wt_tag(wt) + "_" + epi;
-  auto deal = [&](long rows, long tokens) { return (unsigned)(8 * tokens * ((rows + 7) / 8)); };
-  p.name = name + "_r" + std::to_string(R);
-  p.grid = deal((n + 16 * R - 1) / (16 * R), nt);
-  p.threads = kSgemmThreads;
+    while (R > 1 && ((long)n + 16 * R - 1) / (16 * R) * nt < 2 * num_cus) R /= 2;
+  SgemmPlan p = sgemm_split_plan(wt, epi, m, n, R);
   p.units = 0.0070 * n / num_cus * nt;
   static const struct {
     double lone, pair;
@@ -259,9 +276,7 @@ SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) 
     const long tokens = (nt + tt - 1) / tt, per_cu = (rows * tokens + num_cus - 1) / num_cus;
     const double u = (double)(per_cu / 2) * kWide[tt - 1].pair + (double)(per_cu % 2) * kWide[tt - 1].lone;
     if (u >= p.units) continue;
-    p.name = name + "_w" + std::to_string(tt);
-    p.grid = deal(rows, tokens);
-    p.threads = kWideThreads;
+    p = sgemm_wide_plan(wt, epi, m, n, tt);
     p.units = u;
   }
   return p;

@@ -28,8 +28,11 @@
 // flight while the one before is computed.  Q4 codes stay packed until the
 // operand is read: lanes 0..31 of a wave take a block's low nibbles, the
 // others the high ones, as 16 (q - 8) in the upper half of a byte - a shift
-// and one three-input operation per dword; the factor 16 leaves sums and
-// totals exact (it only moves their exponent) and is taken out at the end.
+// and one three-input operation per dword.  The factor 16 only moves the
+// exponent of sums and totals and is taken out at the end; a wave in which it
+// may have carried one past the largest float redoes those outputs without it
+// (gemm_common.h).  The check is one FMA per output (8B, 2048 tokens, without /
+// with it in turn: gate|up 919 - 927 / 892 - 913 us, down 430 - 434 / 421 - 428).
 // Within a wave the matrix instructions run one tile ahead of the arithmetic.
 // Measured (8B, 2048 tokens, us; before: codes through registers, unpacked
 // when written to LDS, matrix results read as soon as issued): gate|up 1066 ->
@@ -46,6 +49,7 @@
 // 1B, 700 tokens, us: down 163 -> 74, O 55 -> 24, Q|K|V 43 -> 33.
 #include "attn_core.h"
 #include "exact_math.h"
+#include "gemm_common.h"
 #include "gemv_core.h"
 
 using namespace llmrs;
@@ -101,18 +105,6 @@ __device__ __forceinline__ v4i q4_bytes16(v4i w, int sh) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) r[i] = (int)((((unsigned)w[i] << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
   return r;
-}
-
-// The value is computed here and read after here.
-template <typename T>
-__device__ __forceinline__ void pin(T& x) {
-  asm volatile("" : "+v"(x));
-}
-
-// 16 bytes per lane from global memory to lds + 16 * lane, without registers.
-__device__ __forceinline__ void load_lds16(const void* src, uint8_t* lds) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
 
 }  // namespace
@@ -337,41 +329,88 @@ __device__ __forceinline__ void gemm_impl(const PrefillGemmArgs& a, uint8_t* lds
   }
 
   // Epilogues.  Register i of a tile holds token 8 (i / 4) + 4 half + i % 4
-  // and row col.
+  // and row col.  Where a wave holds totals that are not finite (gemm_common.h),
+  // those outputs take the plain block loop.
+  bool redo_any = false;
+  if constexpr (WT != WT_Q8H) {
+    float z = 0.0f;  // stays 0 while every total is finite
 #pragma unroll
-  for (int t = 0; t < TT; ++t) {
+    for (int t = 0; t < TT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = m0 + wm + 32 * t + 8 * (i / 4) + 4 * half + (i % 4);
-      if constexpr (EPI == EPI_SILU) {
-        // rows n0+wn .. +31 are gate, +32 .. +63 the matching up rows
-        // (layer.rs:72-79); m index j = (n0+wn)/2 + col.
-        const float g = acc[t][0][i], u = acc[t][1][i];
-        const float mv = (g / (1.0f + exact_expf(-g))) * u;  // glibc expf (exact_math.h)
-        const int run = (n0 + wn) / 64;
-        const int j = run * 32 + col;
-        float amax = fabsf(mv);
+      for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 32));
-        const float d = amax / 127.0f;
-        const float inv = amax == 0.0f ? 0.0f : 1.0f / d;
-        if (m < a.M && n0 + wn < a.N) {
-          if (a.y) a.y[(size_t)m * a.ldy + j] = mv;
-          a.yq[act_row(m, a.N / 2, a.layout) + act_offset(j, a.layout)] =
-              amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(mv, inv);
-          if (col == 0)
-            a.yd[act_scale_row(m, a.N / 64, a.layout) + act_scale_offset(run, a.layout)] = amax == 0.0f ? 0.0f : d;
+        for (int i = 0; i < 16; ++i) z = __builtin_fmaf(acc[t][r][i], 0.0f, z);
+    redo_any = __any(z != 0.0f);
+  }
+  auto token = [&](int t, int i) { return m0 + wm + 32 * t + 8 * (i / 4) + 4 * half + (i % 4); };
+  if constexpr (EPI == EPI_SILU) {
+    // rows n0+wn .. +31 are gate, +32 .. +63 the matching up rows
+    // (layer.rs:72-79); m index j = (n0+wn)/2 + col.
+    const int run = (n0 + wn) / 64, j = run * 32 + col;
+    auto out = [&](int m, float g, float u) {
+      const float mv = (g / (1.0f + exact_expf(-g))) * u;  // glibc expf (exact_math.h)
+      float amax = fabsf(mv);
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 32));
+      const float d = amax / 127.0f;
+      const float inv = amax == 0.0f ? 0.0f : 1.0f / d;
+      if (m < a.M && n0 + wn < a.N) {
+        if (a.y) a.y[(size_t)m * a.ldy + j] = mv;
+        a.yq[act_row(m, a.N / 2, a.layout) + act_offset(j, a.layout)] =
+            amax == 0.0f ? (int8_t)0 : (int8_t)q8_code(mv, inv);
+        if (col == 0)
+          a.yd[act_scale_row(m, a.N / 64, a.layout) + act_scale_offset(run, a.layout)] = amax == 0.0f ? 0.0f : d;
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) out(token(t, i), acc[t][0][i], acc[t][1][i]);
+    if constexpr (WT != WT_Q8H) {
+      if (redo_any) {  // over what was written: the tokens of register 16 t + i
+        unsigned redo = 0;
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (__any(!(is_finite(acc[t][0][i]) && is_finite(acc[t][1][i])))) redo |= 1u << (16 * t + i);
+        const int gr = min(n0 + wn + col, a.N - 1), ur = min(n0 + wn + 32 + col, a.N - 1);
+#pragma unroll 1
+        for (; redo; redo &= redo - 1) {
+          const int k = __builtin_ctz(redo), m = token(k >> 4, k & 15), mc = min(m, a.M - 1);
+          out(m, q4_block_loop<WT, kActNatural>(a, mc, gr), q4_block_loop<WT, kActNatural>(a, mc, ur));
         }
-      } else {
+      }
+    }
+  } else {
+    auto out = [&](int m, int n, float v) {
+      if (EPI == EPI_RESID) v = v + a.res[(size_t)m * a.N + n];  // layer.rs:386,403
+      a.y[(size_t)m * a.ldy + n] = v;
+    };
+    if (!redo_any) {
 #pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          const int n = n0 + row + 32 * r;
-          if (m < a.M && n < a.N) {
-            float v = acc[t][r][i];
-            if (EPI == EPI_RESID) v = v + a.res[(size_t)m * a.N + n];  // layer.rs:386,403
-            a.y[(size_t)m * a.ldy + n] = v;
-          }
-        }
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            if (token(t, i) < a.M && n0 + row + 32 * r < a.N) out(token(t, i), n0 + row + 32 * r, acc[t][r][i]);
+    } else if constexpr (WT != WT_Q8H) {
+      unsigned long long redo = 0;  // this lane's: bit RT (16 t + i) + r
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            if (token(t, i) < a.M && n0 + row + 32 * r < a.N) {
+              if (is_finite(acc[t][r][i])) out(token(t, i), n0 + row + 32 * r, acc[t][r][i]);
+              else redo |= 1ull << (RT * (16 * t + i) + r);
+            }
+#pragma unroll 1
+      for (; redo; redo &= redo - 1) {
+        const int k = __builtin_ctzll(redo), i = k / RT, m = token(i >> 4, i & 15), n = n0 + row + 32 * (k % RT);
+        out(m, n, q4_block_loop<WT, kActNatural>(a, m, n));
       }
     }
   }

@@ -51,6 +51,7 @@
 
 #include "common.h"
 #include "exact_math.h"
+#include "gemm_common.h"
 #include "gemv_core.h"
 #include "../kernel_args.h"
 
@@ -63,15 +64,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int kSgThreads = kSgemmThreads;   // eight waves
 constexpr int kSgWaves = kSgThreads / LLMRS_WAVE;
 constexpr int kStep = 8;                    // blocks of one wave per round
-
-template <int WT>
-__device__ __forceinline__ unsigned load_scale(const void* ws, size_t i) {
-  return WT == WT_Q4F ? ((const unsigned*)ws)[i] : ((const uint16_t*)ws)[i];
-}
-
-// q - 8 for four nibbles held one per byte (0..15): (v + 0x78) ^ 0x80 per
-// byte, no carry between bytes.
-__device__ __forceinline__ unsigned nib_s8(unsigned v) { return (v + 0x78787878u) ^ 0x80808080u; }
 
 // In: lane group g holds the four dwords of its block g.  Out: x[j] = dword
 // g of block j.  v_permlane32_swap(a, b) exchanges the upper half of a with
@@ -346,21 +338,6 @@ struct WideStage {
   static_assert(N * BYTES <= 80 * 1024, "two workgroups per CU");
 };
 
-// The value is computed here and read after here.
-template <typename T>
-__device__ __forceinline__ void pin(T& x) {
-  asm volatile("" : "+v"(x));
-}
-
-__device__ __forceinline__ void load_lds16(const void* src, uint8_t* lds) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
-}
-__device__ __forceinline__ void load_lds4(const void* src, uint8_t* lds) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)lds, 4, 0, 0);
-}
-
 template <int WT, int EPI, int TT>
 __device__ __forceinline__ void wide_impl(const SgemmArgs& a, uint8_t* lds) {
   typedef WideStage<WT, TT> S;
@@ -461,7 +438,7 @@ __device__ __forceinline__ void wide_impl(const SgemmArgs& a, uint8_t* lds) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) op[u].hi[j] = w1[j];
         transpose4(op[u].hi);
-      } else {  // 16 (q - 8) in a byte's upper half
+      } else {  // 16 (q - 8) in a byte's upper half (gemm_common.h)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           op[u].hi[j] = (op[u].lo[j] & 0xF0F0F0F0u) ^ 0x80808080u;
@@ -540,6 +517,22 @@ __device__ __forceinline__ void wide_impl(const SgemmArgs& a, uint8_t* lds) {
   for (int t = 0; t < TT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) s_o[(16 * t + r) * LD + 16 * w + 4 * g + i] = acc[t][i];
+  if constexpr (WT != WT_Q8H) {
+    // totals that are not finite: the plain block loop (gemm_common.h); tokens
+    // past M hold whatever the buffer did
+    unsigned redo = 0;  // bit 4 t + i
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (!is_finite(acc[t][i]) && 16 * (tile0 + t) + r < a.M && n0 + 16 * w + 4 * g + i < a.N) redo |= 1u << (4 * t + i);
+#pragma unroll 1
+    while (redo) {
+      const int k = __builtin_ctz(redo), lt = 16 * (k >> 2) + r, ln = 16 * w + 4 * g + (k & 3);
+      redo &= redo - 1;
+      s_o[lt * LD + ln] = q4_block_loop<WT, kActMfma>(a, 16 * tile0 + lt, n0 + ln);
+    }
+  }
   __syncthreads();
   if constexpr (EPI == EPI_SILU) {
     // 32 gate rows, then their up rows (layer.rs:72-79)

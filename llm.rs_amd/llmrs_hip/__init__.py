@@ -101,6 +101,10 @@ _SIGS = {
     "llmrs_model_set_sampling": (C.c_int, [C.c_void_p, C.c_void_p]),
     "llmrs_model_set_exact": (C.c_int, [C.c_void_p, C.c_int]),
     "llmrs_probe_expf": (C.c_int, [C.c_void_p, C.c_size_t, C.c_void_p]),
+    "llmrs_probe_gemm_plan": (C.c_int, [C.c_char_p, C.c_char_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_int, C.c_char_p,
+                                        C.POINTER(C.c_uint32)]),
+    "llmrs_probe_gemm": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_char_p, C.c_char_p, C.c_int, C.c_void_p,
+                                   C.c_void_p, C.c_void_p]),
     "llmrs_batch_create": (C.c_int, [C.c_void_p, C.c_int32, C.POINTER(C.c_void_p)]),
     "llmrs_batch_free": (C.c_int, [C.c_void_p]),
     "llmrs_batch_begin": (C.c_int, [C.c_void_p, C.c_int32, C.c_void_p, C.c_size_t]),
@@ -180,6 +184,27 @@ def probe_expf(x) -> np.ndarray:
     out = np.empty_like(x)
     _check(lib().llmrs_probe_expf(_ptr(x), x.size, _ptr(out)))
     return out
+
+
+def probe_gemm_plan(weight: str, epi: str, m: int, n: int, k: int, cus: int = 256) -> tuple[str, tuple[int, int]]:
+    """The GEMM kernel and grid that m rows take through an [n, k] weight
+    (llmrs_probe_gemm_plan); needs no device."""
+    name, grid = C.create_string_buffer(64), (C.c_uint32 * 2)()
+    _check(lib().llmrs_probe_gemm_plan(weight.encode(), epi.encode(), m, n, k, cus, name, grid))
+    return name.value.decode(), (grid[0], grid[1])
+
+
+def probe_gemm(a: Tensor, w: Tensor, epi: str, variant: str, res: Tensor | None = None, order: int = 0):
+    """One launch of a given GEMM kernel (llmrs_probe_gemm): y, or for silu
+    (m, codes, scales)."""
+    m, n = a.shape[0], w.shape[0]
+    silu = epi == "silu"
+    y = np.empty((m, n // 2 if silu else n), np.float32)
+    q = np.empty(y.shape, np.int8) if silu else None
+    d = np.empty((m, n // 64), np.float32) if silu else None
+    _check(lib().llmrs_probe_gemm(a.handle, w.handle, res.handle if res else None, epi.encode(), variant.encode(),
+                                  order, _ptr(y), _ptr(q), _ptr(d)))
+    return (y, q, d) if silu else y
 
 
 def num_cus() -> int:

@@ -45,3 +45,58 @@ def test_gemm_edges_bit_exact(hip, orc, rng, wtype, m, n, k):
         want = orc.matmul_transposed_q4(a, qs, sc, n)
     got = hip.HipBackend().matmul_transposed(hip.Tensor.from_numpy(a), w).data()
     assert np.array_equal(got.view(np.uint32), np.asarray(want, F32).reshape(m, n).view(np.uint32))
+
+
+def same_bits(got, want, what):
+    """Equal in every bit, any NaN equal to any other."""
+    got, want = np.asarray(got, F32), np.asarray(want, F32)
+    bad = (got.view(np.uint32) != want.view(np.uint32)) & ~(np.isnan(got) & np.isnan(want))
+    assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.size} differ, first {got[bad][0]!r} for {want[bad][0]!r}"
+
+
+def check_variant(hip, orc, epi, variant, a, w, y, res, order):
+    """One launch of a GEMM kernel against the oracle's products y [m, n] of
+    the same rows: stored, added to `res`, or as the SwiGLU product (runs of 32
+    gate rows, then their up rows) with its Q8_0 codes."""
+    ta = hip.Tensor.from_numpy(a)
+    if epi == "store":
+        same_bits(hip.probe_gemm(ta, w, epi, variant), y, variant)
+    elif epi == "resid":
+        with np.errstate(all="ignore"):
+            same_bits(hip.probe_gemm(ta, w, epi, variant, hip.Tensor.from_numpy(res)), y + res, variant)
+    else:
+        m, n = y.shape
+        runs = y.reshape(m, n // 64, 2, 32)
+        want = orc.silu_mul(runs[:, :, 0].reshape(m, n // 2), runs[:, :, 1].reshape(m, n // 2)).reshape(m, n // 2)
+        got, q, d = hip.probe_gemm(ta, w, epi, variant, order=order)
+        same_bits(got, want, variant)
+        for t in range(m):
+            oq, od = orc.quantize_row_q8_0(want[t])
+            some = ~np.isnan(want[t]).reshape(-1, 32).all(1)  # a block of nothing but NaN has no scale
+            assert np.array_equal(q[t].reshape(-1, 32)[some], oq.reshape(-1, 32)[some]), f"{variant}: codes of row {t}"
+            same_bits(d[t][some], od[some], f"{variant}: scales of row {t}")
+
+
+Q4_VARIANTS = [(v, e) for v in ("r1", "r2", "r4", "w1", "w2", "w3", "128x128", "64x128", "64x64")
+               for e in ("store", "resid", "silu") if e != "silu" or v not in ("r1", "r2", "64x64")]
+
+
+@pytest.mark.parametrize("wtype", ["q4_0", "q4_ref"])
+@pytest.mark.parametrize("variant,epi", Q4_VARIANTS, ids=["-".join(v) for v in Q4_VARIANTS])
+def test_gemm_near_overflow(hip, orc, rng, wtype, variant, epi):
+    """Rows whose terms and sums lie from far below the largest float to beyond
+    it: what the block loop keeps finite stays finite, and what overflows there
+    overflows the same way, whatever factor a kernel carries its codes with."""
+    m, n, k = 70, 256, 640
+    a = (rng.normal(0, 1, (m, k)) * 10.0 ** rng.uniform(34.0, 37.5, (m, 1))).astype(F32)
+    qs = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    sc = rng.uniform(0.1, 1.0, (n, k // 32)).astype(F32)
+    if wtype == "q4_0":
+        sc = sc.astype(np.float16).astype(F32)
+    elif epi == "silu":
+        sc.reshape(n // 64, 2, 32, -1)[:, 1] *= F32(1e-37)  # up rows that bring the product back into range
+    with np.errstate(all="ignore"):
+        y = np.asarray(orc.matmul_transposed_q4(a, qs, sc, n), F32).reshape(m, n)
+    assert np.any(np.isfinite(y) & (np.abs(y) > 2.0 ** 124)) and np.any(np.isinf(y))
+    res = (rng.normal(0, 1, (m, n)) * 1e37).astype(F32)
+    check_variant(hip, orc, epi, variant, a, hip.Tensor.from_q4(qs, sc, n, k), y, res, order=1)
