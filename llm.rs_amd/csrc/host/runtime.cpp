@@ -204,7 +204,9 @@ const GemmTile& gemm_tile(const std::string& epi, int m, int n, int num_cus, dou
   const GemmTile* best = nullptr;
   for (const GemmTile& t : kGemmTiles) {
     if (epi == "silu" && t.rt == 1) continue;  // a gate and an up run of 32 per wave
-    const long wgs = (long)((m + 64 * t.tt - 1) / (64 * t.tt)) * ((n + 64 * t.rt - 1) / (64 * t.rt));
+    const long token_tiles = (m + 64 * t.tt - 1) / (64 * t.tt);
+    if (t.tt == 1 && token_tiles > 65535) continue;  // past a grid's second dimension
+    const long wgs = token_tiles * ((n + 64 * t.rt - 1) / (64 * t.rt));
     const long per_cu = (wgs + num_cus - 1) / num_cus;
     const double u = (double)(per_cu / 2) * t.pair + (double)(per_cu % 2) * t.lone;
     if (best && u >= *units) continue;
