@@ -909,7 +909,8 @@ __device__ __forceinline__ void attn_prefill_mfma_impl(const PrefillAttnArgs& a)
 // (max, sum, O) are merged through LDS.  Everything stays f32:
 //   S^T = K Q^T        v_mfma_f32_32x32x2f32: lane (col, half) holds dims
 //                       half * HD/2 .. of key / query col, so step s takes dims
-//                       s and HD/2 + s
+//                       s and HD/2 + s; two sums of half the steps each, which
+//                       rounds less than one long one
 //   online softmax      one query per lane column, as in the f16 kernel
 //   O^T += V^T P^T      register i of S^T holds keys 8 (i/4) + i%4 (lower half)
 //                       and + 4 (upper half): step i takes those two
@@ -918,7 +919,11 @@ __device__ __forceinline__ void attn_prefill_mfma_impl(const PrefillAttnArgs& a)
 // matrix instructions (64 cycles each) cover the reads.  They bound it: 700 rows
 // of the 1B shape need 14 us at the f32 matrix rate and take 51, 2048 rows 319
 // (the longest query tile's streams end last); the vector kernel's dots
-// and P.V (four multiply-adds per LDS read) took 104 and 655.
+// and P.V (four multiply-adds per LDS read) took 104 and 655.  Distance from
+// 64-bit sums as a share of the vector kernel's (30 seeds a shape), with one
+// sum / two: 16 rows after 17 1.03 / 0.94 (head_dim 64), 1.01 / 0.80 (128); 32
+// rows 1.01 / 0.99, 1.01 / 0.87; 64 rows 0.97 / 0.94, 0.99 / 0.85; 700 rows (3
+// seeds) 0.66 / 0.65, 0.71 / 0.63.  Times are the same.
 template <int HD>
 __device__ __forceinline__ void attn_prefill_f32_impl(const PrefillAttnArgs& a) {
   constexpr int ND = HD / 32, HH = HD / 2, KT = 32, NSTR = 4;
@@ -958,9 +963,14 @@ __device__ __forceinline__ void attn_prefill_f32_impl(const PrefillAttnArgs& a) 
 #pragma unroll
       for (int d = 0; d < ND; ++d) v[d][i] = vc[(size_t)key * HD + 32 * d + col];
     }
-    v16f st = v16f{};
+    v16f st = v16f{}, st1 = v16f{};
 #pragma unroll
-    for (int s = 0; s < HH; ++s) st = __builtin_amdgcn_mfma_f32_32x32x2f32(k[s], q[s], st, 0, 0, 0);
+    for (int s = 0; s < HH / 2; ++s) {
+      st = __builtin_amdgcn_mfma_f32_32x32x2f32(k[s], q[s], st, 0, 0, 0);
+      st1 = __builtin_amdgcn_mfma_f32_32x32x2f32(k[HH / 2 + s], q[HH / 2 + s], st1, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) st[i] = st[i] + st1[i];
     if (kt + NSTR < ntile) load_k(kt + NSTR);
     float p[16];
     float mloc = -INFINITY;

@@ -373,3 +373,29 @@ def test_prefill_attention_f32_cache(hip, orc, head_dim, start, M):
     tiles, after a filled cache."""
     spec = syn.tiny(DType.Q4_0, DType.F32, head_dim=head_dim, n_heads=8, n_kv_heads=2, ffn=1024, prompt=M, decode=0)
     check_prefill_layer(hip, orc, syn.with_sizes(spec, n_layers=1), start, M)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_prefill_attention_f32_no_further_than_vector(hip, orc, head_dim, monkeypatch):
+    """The matrix-core kernel's ctx is no further from float64 sums than the
+    vector kernel's on few keys, where its sums are no shorter (one or two key
+    tiles; more keys favour it).  Single shapes scatter by several percent, so
+    the distances of ten inputs a shape are compared together."""
+    total = {"valu": 0.0, "mfma": 0.0}
+    for start, M in [(0, 17), (0, 32), (17, 16)]:
+        for seed in range(100, 110):
+            spec = syn.with_sizes(syn.tiny(DType.Q4_0, DType.F32, head_dim=head_dim, n_heads=8, n_kv_heads=2, prompt=M,
+                                           decode=0, seed=seed), n_layers=1)
+            gm, om, _ = layer_models(hip, orc, spec, start + M)
+            if start:
+                fill_cache(gm, om, spec, start)
+            x = synth_normal(seed, 96, M * spec.hidden, 0.0, 1.0).reshape(M, spec.hidden)
+            for mode in total:
+                monkeypatch.setenv("LLMRS_PREFILL_ATTN", mode)
+                pr = gm.probe_prefill_layer(0, start, x)
+                exact = exact_attention(om, orc, pr["qkv"], start).astype(np.float64)
+                total[mode] += float(np.linalg.norm(pr["ctx"] - exact) / np.linalg.norm(exact))
+            gm.close()
+    print(f"\nf32 prefill attention, head_dim {head_dim}: distance / the vector kernel's "
+          f"{total['mfma'] / total['valu']:.4f}", flush=True)
+    assert total["mfma"] <= total["valu"]
