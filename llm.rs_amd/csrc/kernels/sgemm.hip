@@ -517,29 +517,15 @@ __device__ __forceinline__ void wide_impl(const SgemmArgs& a, uint8_t* lds) {
   for (int t = 0; t < TT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) s_o[(16 * t + r) * LD + 16 * w + 4 * g + i] = acc[t][i];
-  if constexpr (WT != WT_Q8H) {
-    // totals that are not finite: the plain block loop (gemm_common.h); tokens
-    // past M hold whatever the buffer did
-    unsigned redo = 0;  // bit 4 t + i
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (!is_finite(acc[t][i]) && 16 * (tile0 + t) + r < a.M && n0 + 16 * w + 4 * g + i < a.N) redo |= 1u << (4 * t + i);
-#pragma unroll 1
-    while (redo) {
-      const int k = __builtin_ctz(redo), lt = 16 * (k >> 2) + r, ln = 16 * w + 4 * g + (k & 3);
-      redo &= redo - 1;
-      s_o[lt * LD + ln] = q4_block_loop<WT, kActMfma>(a, 16 * tile0 + lt, n0 + ln);
-    }
-  }
   __syncthreads();
+  bool redo = false;  // this lane met a total that is not finite
   if constexpr (EPI == EPI_SILU) {
     // 32 gate rows, then their up rows (layer.rs:72-79)
 #pragma unroll
     for (int p = 0; p < 2 * TT; ++p) {
       const int t = 8 * p + (tid >> 5), j = tid & 31;
       const float gv = s_o[t * LD + j], uv = s_o[t * LD + 32 + j];
+      if (WT != WT_Q8H) redo |= !is_finite(gv) || !is_finite(uv);
       const float mv = (gv / (1.0f + exact_expf(-gv))) * uv;  // glibc expf (exact_math.h)
       swiglu_out(a, 16 * tile0 + t, tx, j, mv);
     }
@@ -549,8 +535,35 @@ __device__ __forceinline__ void wide_impl(const SgemmArgs& a, uint8_t* lds) {
       const int lt = 4 * p + w, t = 16 * tile0 + lt, n = n0 + lane;
       if (t < a.M && n < a.N) {
         float v = s_o[lt * LD + lane];
-        if (EPI == EPI_RESID) v = v + a.res[(size_t)t * a.N + n];  // layer.rs:386,403
-        a.y[(size_t)t * a.ldy + n] = v;
+        const bool ok = WT == WT_Q8H || is_finite(v);
+        redo |= !ok;
+        if (EPI == EPI_RESID && ok) v = v + a.res[(size_t)t * a.N + n];  // layer.rs:386,403
+        if (EPI != EPI_RESID || ok) a.y[(size_t)t * a.ldy + n] = v;     // may be the residual's place
+      }
+    }
+  }
+  if constexpr (WT != WT_Q8H) {
+    // Those outputs again by the plain block loop (gemm_common.h).  The
+    // arguments are read anew, so that the loops above need not hold them.
+    if (__any(redo)) {
+      const SgemmArgs* ka = (const SgemmArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+      asm volatile("" : "+s"(ka));
+#pragma unroll 1
+      for (int p = 0; p < (EPI == EPI_SILU ? 2 : 4) * TT; ++p) {
+        if constexpr (EPI == EPI_SILU) {
+          const int lt = 8 * p + (tid >> 5), j = tid & 31, t = 16 * tile0 + lt;
+          float gv = s_o[lt * LD + j], uv = s_o[lt * LD + 32 + j];
+          if (t < ka->M && !is_finite(gv)) gv = q4_block_loop<WT, kActMfma>(*ka, t, n0 + j);
+          if (t < ka->M && !is_finite(uv)) uv = q4_block_loop<WT, kActMfma>(*ka, t, n0 + 32 + j);
+          swiglu_out(*ka, t, tx, j, (gv / (1.0f + exact_expf(-gv))) * uv);
+        } else {
+          const int lt = 4 * p + w, t = 16 * tile0 + lt, n = n0 + lane;
+          if (t < ka->M && n < ka->N && !is_finite(s_o[lt * LD + lane])) {
+            float v = q4_block_loop<WT, kActMfma>(*ka, t, n);
+            if (EPI == EPI_RESID) v = v + ka->res[(size_t)t * ka->N + n];
+            ka->y[(size_t)t * ka->ldy + n] = v;
+          }
+        }
       }
     }
   }
