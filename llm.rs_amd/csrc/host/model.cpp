@@ -1952,13 +1952,12 @@ struct llmrs_batch {
   // linear layers on the decode GEMV over all rows (gemv_*_q8b_*: one
   // workgroup per row and weight slice, the rows' workgroups of a slice on
   // one XCD so that the weights stream from HBM about once and the other rows
-  // read them from its L2; up to kBatchGemvMax sequences), on the skinny GEMM
-  // (sgemm.hip; token tiles of 16, the activation codes in its operand order)
-  // or, beyond its rows or for widths not a multiple of 128, on the prefill
-  // GEMM
+  // read them from its L2; up to kBatchGemvMax sequences), or each on the
+  // skinny GEMM (sgemm.hip; activation rows in its operand order) or the
+  // prefill GEMM (rows as they are), whichever is the faster for it
   bool gemv = false;
-  bool skinny = false;
-  int layout = llmrs::kActNatural;
+  int lay_qkv = llmrs::kActNatural, lay_o = llmrs::kActNatural, lay_gu = llmrs::kActNatural;
+  int lay_down = llmrs::kActNatural, lay_head = llmrs::kActNatural;
   // attention splits per sequence: the model's (planned for one sequence)
   // cut so that the B sequences' workgroups fill the GPU about twice
   int nsplit = 1;
@@ -1995,10 +1994,20 @@ GemvPlan batch_gemv_plan(const llmrs_batch* b, const char* epi, const DevLinear&
   return gemv_plan(b->m->wt, std::string("q8b_") + epi, W.n, W.k, ctx().num_cus);
 }
 
-std::string batch_linear_kernel(const llmrs_batch* b, const char* epi, const DevLinear& W) {
+std::string batch_linear_kernel(const llmrs_batch* b, const char* epi, const DevLinear& W, int layout) {
   if (b->gemv) return batch_gemv_plan(b, epi, W).name;
-  return b->skinny ? sgemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name
-                   : gemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name;
+  return layout == llmrs::kActMfma ? sgemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name
+                                   : gemm_plan(b->m->wt, epi, b->B, W.n, ctx().num_cus).name;
+}
+
+// Operand order of the B rows a linear layer reads, which is also its kernel:
+// `mode` is LLMRS_BATCH_GEMM, empty for the faster one.  Both give the same
+// bits.  8B, us a step (128256-row head, one layer), all skinny / all tiles /
+// per launch: 64 sequences 352 / 371 / 302, 128 596 / 495 / 459, 160 734 / 678 / 665.
+int batch_layout(const llmrs_batch* b, const char* epi, const DevLinear& W, const std::string& mode) {
+  if (b->gemv || mode == "prefill" || !sgemm_serves(b->B, W.k)) return llmrs::kActNatural;
+  return mode == "skinny" || sgemm_faster(b->m->wt, epi, b->B, W.n, W.k, ctx().num_cus) ? llmrs::kActMfma
+                                                                                       : llmrs::kActNatural;
 }
 
 // One greedy step of every sequence of the batch.
@@ -2008,10 +2017,10 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
   const int B = b->B, H = c.hidden, hd = c.head_dim, nq = c.n_heads, nkv = c.n_kv_heads;
   const dim3 blk(256);
   // One linear layer over the B rows: Y = X W^T (+ res), or the SwiGLU
-  // product's Q8_0 codes; work figure = the weight bytes.
-  auto linear = [&](const char* epi, const DevLinear& W, const int8_t* xq, const float* xd, float* y,
+  // product's Q8_0 codes (in the down projection's order); work figure = the weight bytes.
+  auto linear = [&](const char* epi, const DevLinear& W, int layout, const int8_t* xq, const float* xd, float* y,
                     const float* res, int8_t* yq, float* yd) {
-    const std::string name = batch_linear_kernel(b, epi, W);
+    const std::string name = batch_linear_kernel(b, epi, W, layout);
     const bool silu = std::string(epi) == "silu";
     const double wb = linear_weight_bytes(m, W);
     if (b->gemv) {
@@ -2030,13 +2039,13 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
       g.batch_rows = B;
       g.batch_nwg = (int)p.grid;
       L(name, wb, dim3(8u * (unsigned)B * ((p.grid + 7) / 8)), dim3(p.threads), p.lds, g);
-    } else if (b->skinny) {
-      SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, W.n, b->layout};
+    } else if (layout == llmrs::kActMfma) {
+      SgemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, W.n, b->lay_down};
       const SgemmPlan p = sgemm_plan(m->wt, epi, B, W.n, ctx().num_cus);
       L(p.name, wb, dim3(p.grid), dim3(p.threads), 0, g);
     } else {
       PrefillGemmArgs g{xq, xd, W.codes, W.scales, y, res, yq, yd, B, W.n, W.k, silu ? W.n / 2 : W.n, gemm_group_m(),
-                        llmrs::kActNatural};
+                        b->lay_down};
       const GemmPlan p = gemm_plan(m->wt, epi, B, W.n, ctx().num_cus);
       L(p.name, wb, p.grid, dim3(llmrs::kGemmThreads), p.lds, g);
     }
@@ -2047,10 +2056,10 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
   for (int li = 0; li < c.n_layers; ++li) {
     LayerBufs& Lb = m->layers[li];
     {  // RMSNorm + Q8_0 of each sequence's row (layer.rs:377)
-      PrefillRowArgs r{b->x, Lb.norm[0], b->aq, b->ad, B, H, c.rms_eps, b->layout};
+      PrefillRowArgs r{b->x, Lb.norm[0], b->aq, b->ad, B, H, c.rms_eps, b->lay_qkv};
       L("prefill_rows_q8", 5.0 * H * B, dim3((unsigned)B), blk, gemv_act_lds_host(H), r);
     }
-    linear("store", Lb.qkv, b->aq, b->ad, b->qkv, nullptr, nullptr, nullptr);  // Q|K|V
+    linear("store", Lb.qkv, b->lay_qkv, b->aq, b->ad, b->qkv, nullptr, nullptr, nullptr);  // Q|K|V
     {  // decode attention, one grid slice per sequence (RoPE and the K/V append inside)
       AttnArgs a{};
       a.qkv = b->qkv;
@@ -2072,21 +2081,21 @@ void enqueue_batch_step(llmrs_batch* b, Launcher& L) {
       a.nsplit = b->nsplit;
       a.scale = 1.0f / std::sqrt((float)hd);  // layer.rs:258
       a.kv_batch_bytes = b->kv_bytes;
-      a.ctx_layout = b->layout;
+      a.ctx_layout = b->lay_o;
       L(attn_kernel(m), 0.0, dim3((unsigned)b->nsplit, (unsigned)nkv, (unsigned)B), dim3(attn_threads(m)), 0, a);
     }
-    linear("resid", Lb.o, b->ctx_q, b->ctx_d, b->h, b->x, nullptr, nullptr);  // O + residual (layer.rs:386)
+    linear("resid", Lb.o, b->lay_o, b->ctx_q, b->ctx_d, b->h, b->x, nullptr, nullptr);  // O + residual (layer.rs:386)
     {  // post-attention RMSNorm + Q8_0
-      PrefillRowArgs r{b->h, Lb.norm[1], b->aq, b->ad, B, H, c.rms_eps, b->layout};
+      PrefillRowArgs r{b->h, Lb.norm[1], b->aq, b->ad, B, H, c.rms_eps, b->lay_gu};
       L("prefill_rows_q8", 5.0 * H * B, dim3((unsigned)B), blk, gemv_act_lds_host(H), r);
     }
-    linear("silu", Lb.gu, b->aq, b->ad, nullptr, nullptr, b->m_q, b->m_d);  // gate|up + SwiGLU + Q8_0 of m
-    linear("resid", Lb.down, b->m_q, b->m_d, b->x, b->h, nullptr, nullptr);  // down + residual (layer.rs:403)
+    linear("silu", Lb.gu, b->lay_gu, b->aq, b->ad, nullptr, nullptr, b->m_q, b->m_d);  // gate|up + SwiGLU + Q8_0 of m
+    linear("resid", Lb.down, b->lay_down, b->m_q, b->m_d, b->x, b->h, nullptr, nullptr);  // down + residual (layer.rs:403)
   }
   {  // final RMSNorm (model.rs:39) + lm_head over the B rows, then each row's greedy step
-    PrefillRowArgs r{b->x, m->final_norm, b->aq, b->ad, B, H, c.rms_eps, b->layout};
+    PrefillRowArgs r{b->x, m->final_norm, b->aq, b->ad, B, H, c.rms_eps, b->lay_head};
     L("prefill_rows_q8", 5.0 * H * B, dim3((unsigned)B), blk, gemv_act_lds_host(H), r);
-    linear("store", m->lm_head, b->aq, b->ad, b->logits, nullptr, nullptr, nullptr);
+    linear("store", m->lm_head, b->lay_head, b->aq, b->ad, b->logits, nullptr, nullptr, nullptr);
     ArgmaxBatchArgs am{b->logits, c.vocab, b->pos, b->tokens, b->gen, b->cap};
     L("argmax_batch", 4.0 * c.vocab * B, dim3((unsigned)B), dim3(1024), 0, am);
   }
@@ -2168,20 +2177,25 @@ int llmrs_batch_create(llmrs_model* m, int32_t batch, llmrs_batch** out) {
     b->gen = b->dalloc<int>(B * b->cap);
     b->host_pos.assign(B, 0);
     b->begun.assign(B, 0);
-    const int qdim = c.n_heads * c.head_dim;
     const std::string bg = env_str("LLMRS_BATCH_GEMM");  // gemv, skinny or prefill forces one
     b->gemv = bg == "gemv" || (bg.empty() && batch <= kBatchGemvMax);
-    b->skinny = !b->gemv && bg != "prefill" && sgemm_serves(batch, c.hidden) && sgemm_serves(batch, c.ffn) &&
-                sgemm_serves(batch, qdim);
-    b->layout = b->skinny ? llmrs::kActMfma : llmrs::kActNatural;
+    const LayerBufs& L0 = m->layers[0];  // every layer has its shapes
+    b->lay_qkv = batch_layout(b.get(), "store", L0.qkv, bg);
+    b->lay_o = batch_layout(b.get(), "resid", L0.o, bg);
+    b->lay_gu = batch_layout(b.get(), "silu", L0.gu, bg);
+    b->lay_down = batch_layout(b.get(), "resid", L0.down, bg);
+    b->lay_head = batch_layout(b.get(), "store", m->lm_head, bg);
     b->nsplit = std::max(1, std::min(m->nsplit, (2 * ctx().num_cus + batch * c.n_kv_heads - 1) /
                                                      (batch * c.n_kv_heads)));
     LLMRS_HIP(hipStreamSynchronize(ctx().stream));
     (void)kernel("argmax_batch", dim3(1024));
-    const LayerBufs& L0 = m->layers[0];  // every linear layer's kernel, so graph capture never looks one up
-    for (const auto& [epi, W] : {std::pair<const char*, const DevLinear*>{"store", &L0.qkv}, {"store", &m->lm_head},
-                                 {"resid", &L0.o}, {"resid", &L0.down}, {"silu", &L0.gu}})
-      (void)kernel(batch_linear_kernel(b.get(), epi, *W), dim3(256));
+    // every linear layer's kernel, so graph capture never looks one up
+    for (const auto& [epi, W, layout] : {std::tuple<const char*, const DevLinear*, int>{"store", &L0.qkv, b->lay_qkv},
+                                         {"store", &m->lm_head, b->lay_head},
+                                         {"resid", &L0.o, b->lay_o},
+                                         {"resid", &L0.down, b->lay_down},
+                                         {"silu", &L0.gu, b->lay_gu}})
+      (void)kernel(batch_linear_kernel(b.get(), epi, *W, layout), dim3(256));
     *out = b.release();
     ++m->live_batches;
   });

@@ -284,14 +284,23 @@ SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) 
   return p;
 }
 
-// Whether the skinny GEMM is the faster one for m rows that it can run.
-// Skinny / tile, us: 8B gate|up at 48 rows 39 / 55, 96 rows 74 / 76; O at 128
-// rows 22 / 29, 160 rows 32 / 31; 1B gate|up at 64 rows 18 / 33.
+// Whether the skinny GEMM is the faster one for m rows that it can run.  Where
+// the estimates are close it is, by up to 5 %, and up to 22 % for SwiGLU, whose
+// epilogue a tile's wave runs on 32 tokens at once; Q8_0's skinny kernels take
+// about 10 % longer than the estimate, which is Q4's, and its tiles do not.
+// Short rows (K = 1024) leave too little to pay for the skinny kernels' longer
+// start.  Skinny / tile under a kernel trace, us: 8B gate|up at 64 rows 54.0 /
+// 56.2, 96 rows 75.4 / 76.0; 8B O at 128 rows 20.4 / 28.9, 160 rows 29.6 / 31.7;
+// 70B O at 112 rows 48.1 / 55.1; 8B Q|K|V in Q8_0 at 128 rows 28.3 / 26.4; 8192 x
+// 1024 at 128 rows (a whole call) 12.5 / 11.8.  Over 400 shapes (16 to 160 rows, 17
+// [n, k], all weight types) the kernel taken is 0.15 % slower than the better of
+// the two (geometric mean), 0.43 % with the plain comparison.
 bool sgemm_faster(int wt, const std::string& epi, int m, int n, int k, int num_cus) {
   if (!sgemm_serves((size_t)m, (size_t)k)) return false;
   double units = 0;
   (void)gemm_tile(epi, m, n, num_cus, &units);
-  return sgemm_plan(wt, epi, m, n, num_cus).units < units;
+  const double margin = k < 2048 ? 1.0 : epi == "silu" ? 1.22 : 1.05;
+  return sgemm_plan(wt, epi, m, n, num_cus).units * (wt == WT_Q8H ? 1.10 : 1.0) < units * margin;
 }
 
 // ---- allocator -------------------------------------------------------------

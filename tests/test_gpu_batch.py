@@ -194,3 +194,50 @@ def test_model_free_refused_while_a_batch_lives(hip):
     assert e.value.code == hip.E_INVALID and "batch" in str(e.value)
     bt.close()
     gm.close()
+
+
+@pytest.mark.timeout(600)
+@pytest.mark.parametrize("B", [33, 72, 128, 161])
+def test_batch_kernel_per_layer(hip, orc, B, monkeypatch):
+    """Each linear layer of a larger batch runs on the GEMM that the rule gives
+    for its shape (at these sizes the head and some projections on tiles, others
+    on the skinny GEMM), rows passing between them in the consumer's order: the
+    kernels are the planned ones, logits and tokens those of either GEMM alone,
+    bit for bit, and three slots follow the oracle."""
+    spec = syn.with_sizes(syn.WORKLOADS[2], n_layers=1, vocab=32000)
+    w = syn.make_weights(spec)
+    gm = hip.HipModel(spec.config(32))
+    syn.load_model(gm, w)
+    ps = prompts(spec, B, seed=B)
+    steps, out = 5, {}
+    H, F, qkv = spec.hidden, spec.ffn, (spec.n_heads + 2 * spec.n_kv_heads) * spec.head_dim
+    shapes = [("store", qkv, H), ("resid", H, H), ("silu", 2 * F, H), ("resid", H, F), ("store", spec.vocab, H)]
+    for mode in ("", "skinny", "prefill"):
+        monkeypatch.setenv("LLMRS_BATCH_GEMM", mode)
+        bt = HipBatch(gm, B)
+        for s, p in enumerate(ps):
+            bt.begin(s, p)
+        bt.decode_steps(steps - 2)
+        names = [k.name for k in bt.profile_step() if "gemm" in k.name]  # one step launch by launch
+        if not mode:
+            assert names == [hip.probe_gemm_plan("q4h", e, B, n, k, hip.num_cus())[0] for e, n, k in shapes]
+        elif B <= 160:
+            assert all(n.startswith("sgemm" if mode == "skinny" else "gemm") for n in names)
+        out[mode] = (bt.logits(), [bt.tokens(s, p.size + steps) for s, p in enumerate(ps)])
+        bt.close()
+    for mode in ("skinny", "prefill"):
+        assert np.array_equal(out[""][0].view(np.uint32), out[mode][0].view(np.uint32)), mode
+        assert all(np.array_equal(a, b) for a, b in zip(out[""][1], out[mode][1])), mode
+    om = orc.OracleModel.from_spec(spec, max_seq=32)
+    om.load(w)
+    for s in (0, B // 2, B - 1):
+        toks = out[""][1][s]
+        ref, margins = om.generate(ps[s], steps)
+        check_stream(toks[ps[s].size:], ref, margins, min_steps=steps)
+        olg, _ = om.forward(toks[:-1], 0)
+        # activation codes that a sum in another order moves across a rounding
+        # midpoint change a row by up to 2e-2 of its norm (between the fast and the
+        # reference-order decode, where one layer's K, V and norms all differ); a
+        # row read in a wrong order would be off by its whole norm
+        assert np.linalg.norm(out[""][0][s] - olg) < 3e-2 * np.linalg.norm(olg), f"slot {s}"
+    gm.close()
