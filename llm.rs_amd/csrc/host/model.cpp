@@ -687,8 +687,11 @@ void ensure_prefill(llmrs_model* m) {
 // Operand order of the activation rows of a prefill linear layer: the skinny
 // GEMM's (sgemm.hip) or the tile GEMM's; both are bit-identical to the
 // reference's block loop, and each launch takes the faster.
+// LLMRS_PREFILL_SKINNY=0 keeps every prompt on the tile GEMM.
 int prefill_layout(const llmrs_model* m, const char* epi, int M, const DevLinear& W) {
-  return sgemm_faster(m->wt, epi, M, W.n, W.k, ctx().num_cus) ? llmrs::kActMfma : llmrs::kActNatural;
+  return env_int("LLMRS_PREFILL_SKINNY", 1) != 0 && sgemm_faster(m->wt, epi, M, W.n, W.k, ctx().num_cus)
+             ? llmrs::kActMfma
+             : llmrs::kActNatural;
 }
 
 // Device buffers a test probe adds to one prefill layer: ctx and the SwiGLU

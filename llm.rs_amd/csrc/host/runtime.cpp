@@ -178,12 +178,9 @@ GemvPlan gemv_plan(int wt, const std::string& kind, int n, int k, int num_cus) {
   return p;
 }
 
-// Whether M rows can run on the skinny GEMM: whole 128-element runs and up to
-// 160 rows.  LLMRS_PREFILL_SKINNY=0 keeps every GEMM on the tiles.
-bool sgemm_serves(size_t m, size_t k) {
-  const char* e = std::getenv("LLMRS_PREFILL_SKINNY");
-  return m <= 160 && k % 128 == 0 && !(e && *e == '0');
-}
+// Whether m rows can run on the skinny GEMM: whole 128-element runs and up to
+// 160 rows.
+bool sgemm_serves(size_t m, size_t k) { return m <= 160 && k % 128 == 0; }
 
 namespace {
 struct GemmTile {

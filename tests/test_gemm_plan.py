@@ -20,3 +20,14 @@ def test_tile_grid_covers_and_fits(weight, n, m):
         bm, bn = map(int, name.rsplit("_", 1)[1].split("x"))
         assert gx * bn >= n > (gx - 1) * bn and gy * bm >= m > (gy - 1) * bm, name
         assert gy <= MAX_GRID_Y, f"{name}: grid of {gy} token tiles"
+
+
+@pytest.mark.parametrize("value", ["0", "00", "1", ""])
+def test_prompt_switch_leaves_the_rule(value, monkeypatch):
+    """LLMRS_PREFILL_SKINNY is about prompts: the operators' and the batches'
+    rule does not read it."""
+    shapes = [(m, n, k) for m in (2, 16, 77, 160) for n, k in ((4096, 4096), (28672, 4096), (512, 512))]
+    want = [lh.probe_gemm_plan("q4h", "store", *s) for s in shapes]
+    assert any(name.startswith("sgemm") for name, _ in want)
+    monkeypatch.setenv("LLMRS_PREFILL_SKINNY", value)
+    assert [lh.probe_gemm_plan("q4h", "store", *s) for s in shapes] == want

@@ -241,3 +241,26 @@ def test_batch_kernel_per_layer(hip, orc, B, monkeypatch):
         # row read in a wrong order would be off by its whole norm
         assert np.linalg.norm(out[""][0][s] - olg) < 3e-2 * np.linalg.norm(olg), f"slot {s}"
     gm.close()
+
+
+def test_prompt_switch_is_about_prompts(hip, monkeypatch):
+    """LLMRS_PREFILL_SKINNY=0 keeps a prompt's layers on the tile GEMM, with the
+    same logits, and leaves the batch's linear layers where they were."""
+    spec = SPECS[0]
+    gm = hip.HipModel(spec.config(32))
+    syn.load_model(gm, syn.make_weights(spec))
+    ids = prompts(spec, 1)[0][:7]
+    ids = np.resize(ids, 7)
+    kernels, logits = {}, {}
+    for value in ("1", "0"):
+        monkeypatch.setenv("LLMRS_PREFILL_SKINNY", value)
+        bt = HipBatch(gm, 6)
+        for s in range(6):
+            bt.begin(s, ids)
+        logits[value] = gm.forward(ids, 0)[0]
+        kernels[value] = ({k.name.split("_")[0] for k in gm.profile_prefill(ids) if "gemm" in k.name},
+                          {k.name.split("_")[0] for k in bt.profile_step() if "gemm" in k.name})
+        bt.close()
+    assert kernels == {"1": ({"sgemm"}, {"sgemm"}), "0": ({"gemm"}, {"sgemm"})}
+    assert np.array_equal(logits["0"].view(np.uint32), logits["1"].view(np.uint32))
+    gm.close()
