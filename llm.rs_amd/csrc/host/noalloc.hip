@@ -13,8 +13,9 @@
 //
 // Calls that overlap on one device share its scratch and race; the stream
 // orders calls issued on it.  Nothing in the scratch has to start at zero:
-// prefill_rows_q8 writes every code and scale the GEMM reads (its loads are
-// clamped to the M rows written).
+// prefill_rows_q8 writes every code and scale that an output depends on (the
+// tile GEMM's loads are clamped to the M rows; the skinny GEMM also reads the rest
+// of the last 16-row tile, whose outputs it does not store).
 #include <hip/hip_runtime.h>
 
 #include <memory>
@@ -91,12 +92,11 @@ extern "C" int llmrs_matmul_transposed_noalloc(const llmrs_tensor* a, const llmr
     LLMRS_REQUIRE(m <= 65535 * 128, LLMRS_E_INVALID, "matmul_transposed: too many rows");
     LLMRS_REQUIRE(cx.noalloc_scratch, LLMRS_E_NOINIT,
                   "the scratch's device address was not resolved at init: " + cx.noalloc_error);
-    // few rows of whole 128-element runs: the skinny GEMM, where its whole
-    // 16-row tiles fit the scratch too
-    size_t tile_off = 0;
-    const bool skinny = sgemm_faster(b->wt, "store", (int)m, (int)n, (int)k, cx.num_cus) &&
-                        scratch_need(act_rows(m), k, &tile_off) <= kNoAllocScratchBytes;
-    if (skinny) scale_off = tile_off;
+    // few rows of whole 128-element runs: the skinny GEMM, whose 16-row tiles of
+    // up to 160 rows by 32768 always fit
+    static_assert((size_t)160 * 32768 * 9 / 8 + 256 <= kNoAllocScratchBytes, "skinny GEMM operands");
+    const bool skinny = sgemm_faster(b->wt, "store", (int)m, (int)n, (int)k, cx.num_cus);
+    if (skinny) (void)scratch_need(act_rows(m), k, &scale_off);
     int8_t* xq = (int8_t*)cx.noalloc_scratch;
     float* xd = (float*)((uint8_t*)cx.noalloc_scratch + scale_off);
     PrefillRowArgs r{(const float*)a->data, nullptr, xq, xd, (int)m, (int)k, 0.0f, skinny ? kActMfma : kActNatural};
