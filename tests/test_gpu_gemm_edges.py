@@ -10,20 +10,18 @@ import pytest
 pytestmark = pytest.mark.gpu
 F32 = np.float32
 
-# (m, n, k): the skinny GEMM's 16-row and 16-token tiles, its steps of 8 blocks
-# (k = 384: 12 blocks), its rounds of 64, 32 and 16 blocks, 1, 2 and 4 row
-# tiles per workgroup, and its last row (160) and the one after
+# Shapes (m, n, k) through the operator, which picks the kernel (which one each
+# kernel's own edges are tested with: test_gemm_variants below).  Few rows: ragged
+# 16-row and 16-token tiles, k = 384 (12 blocks, half a stage at the end), one to
+# many rounds, the last row count the skinny GEMM takes (160) and the one after
 SKINNY = [(2, 16, 128), (15, 33, 128), (16, 64, 256), (17, 100, 384), (31, 1, 640), (33, 4112, 2176),
           (64, 8200, 512), (65, 130, 4224), (160, 72, 1024), (161, 72, 1024)]
 
-# the tile GEMM: 64 x 64, 64 x 128 and 128 x 128 tiles with ragged tokens and
-# rows, K of less than a stage (4 or 8 blocks), of whole stages and of every
-# kind of remainder
+# more rows, or K not of whole runs of 128: ragged tokens and rows, K of less than a
+# stage (4 or 8 blocks), of whole stages and of every kind of remainder
 TILES = [(130, 200, 32), (165, 100, 224), (161, 65, 256), (200, 33, 288), (1000, 4090, 416), (2047, 4095, 288),
          (96, 6144, 1024), (100, 28672, 128)]
-# the skinny GEMM's wide kernels: one, two and three token tiles with ragged
-# last ones, rows past a 64-row set, less than a stage of eight blocks, half
-# stages at the end, fewer stages than buffers and more
+# few rows of wide weights
 WIDE = [(2, 32770, 128), (16, 32000, 384), (23, 28700, 640), (32, 28672, 256), (48, 28700, 1152), (64, 16400, 896)]
 
 
@@ -100,3 +98,46 @@ def test_gemm_near_overflow(hip, orc, rng, wtype, variant, epi):
     assert np.any(np.isfinite(y) & (np.abs(y) > 2.0 ** 124)) and np.any(np.isinf(y))
     res = (rng.normal(0, 1, (m, n)) * 1e37).astype(F32)
     check_variant(hip, orc, epi, variant, a, hip.Tensor.from_q4(qs, sc, n, k), y, res, order=1)
+
+
+VARIANTS = [(w, v, e) for w in ("q4_0", "q4_ref", "q8_0") for v, e in Q4_VARIANTS if w != "q8_0" or v != "w3"]
+# ragged rows and tokens for every tile: one stage of 4 blocks alone (all of a wide
+# kernel's loads partial, fewer stages than buffers), 12 and 36 blocks (half a stage
+# at the end), 68 (a round of the split kernels and 4 blocks); for the tiles also 3
+# and 33 blocks, less than a stage and an odd remainder
+SHAPES = [(7, 100, 128), (37, 130, 384), (53, 330, 1152), (70, 257, 2176)]
+TILE_SHAPES = [(37, 130, 96), (140, 257, 1056)]
+
+
+@pytest.mark.parametrize("wtype,variant,epi", VARIANTS, ids=["-".join(v) for v in VARIANTS])
+def test_gemm_variants(hip, orc, rng, wtype, variant, epi):
+    """Every kernel of the several-row GEMMs at the edges of its own tiles, each
+    with every epilogue and weight type, whatever the rule picks."""
+    for m, n, k in SHAPES + (TILE_SHAPES if "x" in variant else []):
+        n = (n + 63) // 64 * 64 if epi == "silu" else n
+        a = rng.normal(0, 1, (m, k)).astype(F32)
+        a[0, :32] = 0.0
+        if wtype == "q8_0":
+            qs, sc = hip.synth_q8(20260023, m + n + k, n, k, 2e-4, 3.5e-4)
+            w, y = hip.Tensor.from_q8_0(qs, sc, n, k), orc.matmul_transposed_q8w(a, qs, sc, n)
+        else:
+            if wtype == "q4_ref":
+                qs, sc = orc.quantize_q4(rng.uniform(-1, 1, (n, k)).astype(F32))
+            else:
+                qs, sc = hip.synth_q4(20260024, m + n + k, n, k, 0.003, 0.006)
+            w, y = hip.Tensor.from_q4(qs, sc, n, k), orc.matmul_transposed_q4(a, qs, sc, n)
+        res = rng.normal(0, 1, (m, n)).astype(F32)
+        for order in (0, 1) if epi == "silu" and n % 256 == 0 else (0,):
+            check_variant(hip, orc, epi, variant, a, w, np.asarray(y, F32).reshape(m, n), res, order)
+
+
+def test_gemm_probe_refuses(hip):
+    """What a kernel cannot run is refused before any launch."""
+    w = {n: hip.Tensor.from_q4(*hip.synth_q4(1, n, n, 96, 0.003, 0.006), n, 96) for n in (64, 65)}
+    a, a1 = (hip.Tensor.from_numpy(np.zeros((4, k), F32)) for k in (96, 128))
+    for args in [(a, w[64], "store", "r1"),      # K not of whole runs of 128
+                 (a, w[65], "silu", "64x128"),   # rows not in runs of 64
+                 (a1, w[64], "store", "64x64"),  # another K
+                 (a, w[64], "store", "32x32"), (a, w[64], "silu", "64x64"), (a, w[64], "resid", "64x64")]:
+        with pytest.raises(hip.LlmrsError):
+            hip.probe_gemm(*args)

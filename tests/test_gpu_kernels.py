@@ -284,8 +284,8 @@ def test_decode_attention_xcd_local(hip, orc, kv, head_dim, waves, splits, monke
 
 def check_prefill_layer(hip, orc, spec, start, M):
     """Every prefill kernel of one layer on M rows at positions start..:
-    GEMMs bit-exact on the GPU's own operands (the tile GEMM, or for up to
-    64 rows the skinny GEMM's exact launches)."""
+    GEMMs bit-exact on the GPU's own operands (each the tile GEMM or the skinny
+    GEMM, as a prompt of M rows picks it)."""
     def same(got, want, what):
         assert np.array_equal(got, want), f"{what} not bit-exact"
     gm, om, w = layer_models(hip, orc, spec, start + M)
@@ -349,20 +349,25 @@ def test_prefill_layer_kernels_ragged_after_cache(hip, orc):
 @pytest.mark.parametrize("index,start,M", [(3, 0, 24), (1, 300, 40), (2, 0, 5), (4, 0, 64)],
                          ids=["8b-24", "1b_q8-40-after-cache", "8b-5", "70b-64"])
 def test_prefill_layer_kernels_short(hip, orc, index, start, M):
-    """Prompts of up to 64 rows: the linear layers on the skinny GEMM's
-    exact launches (one, two and four 16-token tiles), Q4_0 and Q8_0
-    weights, the 70B widths, after a filled cache."""
+    """Prompts of up to 64 rows: the linear layers on the skinny GEMM's split
+    and wide kernels (at 64 rows of the 70B widths gate|up on tiles), Q4_0 and
+    Q8_0 weights, after a filled cache."""
     spec = syn.with_sizes(syn.WORKLOADS[index], n_layers=1, vocab=1024, prompt=M, decode=0, prefilled=0)
     check_prefill_layer(hip, orc, spec, start, M)
 
 
 @pytest.mark.timeout(900)
-@pytest.mark.parametrize("index,M", [(2, 100), (1, 100), (2, 48)], ids=["8b-100", "1b_q8-100", "8b-48"])
+@pytest.mark.parametrize("index,M", [(2, 100), (1, 100), (2, 112)], ids=["8b-100", "1b_q8-100", "8b-112"])
 def test_prefill_layer_kernels_mixed(hip, orc, index, M):
     """Rows at which one layer takes the skinny GEMM for some projections and
     the tile GEMM for others: the activation rows pass between them in the
     consumer's operand order."""
     spec = syn.with_sizes(syn.WORKLOADS[index], n_layers=1, vocab=1024, prompt=M, decode=0, prefilled=0)
+    H, F, qkv = spec.hidden, spec.ffn, (spec.n_heads + 2 * spec.n_kv_heads) * spec.head_dim
+    wt = "q8h" if spec.weight == DType.Q8_0 else "q4h"
+    names = [hip.probe_gemm_plan(wt, e, M, n, k, hip.num_cus())[0]
+             for e, n, k in (("store", qkv, H), ("resid", H, H), ("silu", 2 * F, H), ("resid", H, F))]
+    assert {n.split("_")[0] for n in names} == {"gemm", "sgemm"}, names
     check_prefill_layer(hip, orc, spec, 0, M)
 
 
