@@ -54,9 +54,11 @@ std::string env_str(const char* name) {
 }
 
 // Batched decode runs its linear layers on the row-batched decode GEMV up to
-// this many sequences (8B shape, ms per step GEMV / skinny GEMM: B = 1 1.63 /
-// 2.73, 2 1.94 / 2.84, 4 2.66 / 3.04, 8 4.00 / 3.26); LLMRS_BATCH_GEMM=gemv,
-// skinny or prefill forces one path.
+// this many sequences; LLMRS_BATCH_GEMM=gemv, skinny or prefill forces one path.
+// us a step of one layer with a 1000-row head, GEMV / skinny GEMM: 8B Q4_0 B = 1
+// 63.7 / 86.5, 2 72.9 / 85.1, 4 95.1 / 89.4; 8B Q8_0 (32000 rows) 1 107 / 133, 2 148 /
+// 133, 4 228 / 138.  The line dates from a slower skinny GEMM (8B Q4_0, ms a step of
+// 32 layers: 4 2.66 / 3.04, 8 4.00 / 3.26): it now lies at 3 for Q4_0 and 2 for Q8_0.
 constexpr int kBatchGemvMax = 4;
 
 }  // namespace

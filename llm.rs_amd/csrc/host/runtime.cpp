@@ -250,16 +250,22 @@ SgemmPlan sgemm_wide_plan(int wt, const std::string& epi, int m, int n, int tt) 
 }
 
 // The skinny GEMM's kernel for m rows (16-token tiles) x n weight rows, and its
-// time per block of 32 in gemm_tile's units.  The split kernels spread any
-// shape over the chip: 0.0070 for one token tile and n = the number of CUs.
-// Their row tiles per workgroup (R = 1, 2 or 4 tiles of 16 rows; eight waves
-// share them) are the most that still leave every CU two workgroups, since a
-// workgroup's rows share its activation loads (8B O at 23 rows: R = 1 8.0 us,
-// R = 2, 256 workgroups, 8.9); SwiGLU runs always span four.  The wide kernels
-// (64 rows x 1, 2 or 3 token tiles, a wave's tiles its own) win where that
-// grid fills the chip, by the same sum over the fullest CU as the tile GEMM's.
-// Split / wide, us: 8B gate|up at 16 rows 22.9 / 20.4, 23 rows 41.6 / 29.0, 48
-// rows 61 / 39; 1B gate|up at 64 rows 25.6 / 18.1; 8B O at 16 rows 5.9 / 12.9.
+// time per block of 32 in gemm_tile's units; the 3 to 5 us that every launch takes
+// besides are left out of all estimates.  The split kernels spread any shape over
+// the chip: 0.0070 per token tile and num_cus weight rows.  Their row tiles per
+// workgroup (R = 1, 2 or 4 tiles of 16 rows; eight waves share them) are the most
+// that still leave every CU two workgroups, since a workgroup's rows share its
+// activation loads; SwiGLU runs always span four.  The wide kernels (64 rows x 1, 2
+// or 3 token tiles, a wave's tiles its own) win where that grid fills the chip, by
+// the same sum over the fullest CU as the tile GEMM's.  Both sides, Q4_0, us under a
+// kernel trace: 8B O r1 / r2 / w1 / w2 at 16 rows 6.9 / 8.8 / 14.4 / 19.4, 32 rows 9.2 / 9.2 /
+// 14.4 / 20.2, 64 rows 15.8 / 13.8 / 15.3 / 21.2; 8B gate|up r4 / w1 / w2 / w3 at 16 rows
+// 22.6 / 20.1 / 28.1 / 37.8, 32 rows 40.9 / 35.0 / 29.7 / 38.6, 48 rows 60.4 / 50.5 / 53.8 /
+// 39.6; 1B gate|up at 64 rows 25.2 / 22.0 / 18.1 / 24.3.  The rule is not the best at every
+// shape: 1B gate|up at 32 rows takes w2 (13.6) where w1 takes 12.3, a 1024 x 1024
+// layer at 144 rows r1 (8.3) where r2 takes 5.4; over 400 shapes (16 to 160 rows, 17
+// [n, k], all weight types) its kernel is 3.6 % slower than the best one (geometric
+// mean).
 SgemmPlan sgemm_plan(int wt, const std::string& epi, int m, int n, int num_cus) {
   const long nt = (m + 15) / 16;
   int R = 4;

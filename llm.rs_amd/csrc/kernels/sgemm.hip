@@ -40,12 +40,12 @@
 // on one XCD back to back: the weights come from HBM about once and the other
 // token tiles read them from its L2.
 //
-// Measured (8B widths, us per launch at 16 rows, before -> now, where before
-// was one wave per 16 rows with row-strided loads): Q|K|V 12 -> 7.6, O and
-// down 14.5 -> 9.8, gate|up 35.7 -> 21.4 (66 MB of weights: 3.1 TB/s); exact
-// prompts of 23 rows: 15.1 -> 11.5, 30.5 -> 14.7, 55.5 -> 40; 37 rows: 29 ->
-// 15, 62 -> 19, 80 -> 52.  The rounds' phases (loads, products, LDS, adds)
-// overlap only across the two workgroups of a CU.
+// Measured (8B widths, Q4_0, us per launch; before: one wave per 16 rows with
+// row-strided loads): 16 rows Q|K|V 12 -> 7.6, O and down in the mean 14.5 -> 9.8
+// (5.5 and 14.1); 23 rows Q|K|V 15.1 -> 10.7, O and down 30.5 -> 13.8 (7.6 and 20.0).
+// gate|up goes to the wide kernels below (before 35.7, split 21.4, wide 18.6 at 16
+// rows).  The rounds' phases (loads, products, LDS, adds) overlap only across the
+// two workgroups of a CU.
 
 #include <type_traits>
 
@@ -321,9 +321,10 @@ __device__ __forceinline__ void sgemm_impl(const SgemmArgs& a) {
 // matrix instructions run one product ahead of the arithmetic.  The serial
 // chain of a stage (LDS reads, transposes, products, additions: 0.7 us for one
 // token tile) bounds it while a SIMD holds one or two waves.
-// Measured (gate|up, us, split kernel -> wide): 8B 16 rows 22.9 -> 20.4 (66
-// MB: 3.2 TB/s), 23 rows 41.6 -> 29.0, 48 rows 61 (tile GEMM 55) -> 39; 1B 64
-// rows 25.6 -> 18.1.
+// Measured, split kernel -> wide (us under a kernel trace, about 1 more than
+// without): 8B gate|up 16 rows 22.6 -> 20.1 (66 MB: 3.3 TB/s; Q8_0 27.2 -> 23.2), 32
+// rows 40.9 -> 29.7 (45.8 -> 32.8), 48 rows 60.4 (tile GEMM 55.1) -> 39.6; 1B gate|up
+// 64 rows 25.2 -> 18.1; a 32000-row head of 16 sequences 21.7 -> 18.8.
 template <int WT, int TT>
 struct WideStage {
   static constexpr int RC = kStep * (WT == WT_Q8H ? 2 : 1);  // 16-byte chunks of a row
