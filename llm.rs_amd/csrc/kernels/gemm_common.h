@@ -51,8 +51,10 @@ __device__ float q4_block_loop(const Args& a, int t, int n) {
   const int8_t* x = a.xq + act_row(t, a.K, LAYOUT);
   const float* xd = a.xd + act_scale_row(t, nb, LAYOUT);
   float total = 0.0f;
+  // a NaN stays one; rows with infinite scales come to it within a few blocks, so
+  // that a launch full of them is not left to this loop
 #pragma unroll 1
-  for (int b = 0; b < nb; ++b) {
+  for (int b = 0; b < nb && total == total; ++b) {
     const size_t wb = (size_t)n * nb + b;
     int isum = 0;
 #pragma unroll

@@ -20,8 +20,8 @@
 // identical activation codes.
 //
 // Three VALU operations per element and block (convert, multiply, add) bound
-// the kernel: at the 8B gate|up shape with 2048 tokens the VALU issues on 93 %
-// of its cycles and the matrix cores work on 23 %.  So everything else is kept
+// the kernel: at the 8B gate|up shape with 2048 tokens the VALU issues on 94 %
+// of its cycles and the matrix cores work on 24 %.  So everything else is kept
 // off the VALU.  Workgroup tile 128 tokens x 128 rows, four waves of 64 x 64
 // (2 x 2 MFMA tiles).  Operands reach LDS four blocks at a time by direct
 // loads (no registers, no LDS writes), double-buffered: a stage's loads are in

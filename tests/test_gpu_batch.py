@@ -33,7 +33,7 @@ def prompts(spec, B, seed=5):
 @pytest.mark.parametrize("spec", SPECS, ids=lambda s: s.name)
 def test_batch_streams_vs_oracle(hip, orc, spec, mode, monkeypatch):
     """The three linear-layer paths: the row-batched decode GEMV (the
-    default up to 4 sequences), the skinny GEMM (up to 64) and the prefill
+    default up to 4 sequences), the skinny GEMM (up to 160) and the prefill
     GEMM."""
     monkeypatch.setenv("LLMRS_BATCH_GEMM", mode)
     w = syn.make_weights(spec)
@@ -151,8 +151,8 @@ def test_batch_errors(hip):
 @pytest.mark.parametrize("B", [16, 64])
 def test_batch_8b_widths(hip, orc, B):
     """Two 8B-width layers with the full 128256-row lm_head, B sequences of
-    1-20 prompt tokens decoding 16 greedy steps on the skinny GEMM (its
-    8B-width launches, the ones the benchmark times): every slot's stream
+    1-20 prompt tokens decoding 16 greedy steps on the launches the benchmark
+    times (16: the skinny GEMM; 64: the head on tiles): every slot's stream
     identical to the oracle's for all 16 steps and its last logits within
     1e-2."""
     spec = syn.with_sizes(syn.WORKLOADS[2], n_layers=2)

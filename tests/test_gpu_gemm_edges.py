@@ -87,6 +87,7 @@ def test_gemm_near_overflow(hip, orc, rng, wtype, variant, epi):
     overflows the same way, whatever factor a kernel carries its codes with."""
     m, n, k = 70, 256, 640
     a = (rng.normal(0, 1, (m, k)) * 10.0 ** rng.uniform(34.0, 37.5, (m, 1))).astype(F32)
+    a[3, 70], a[4, 300], a[5, 64:96] = np.inf, np.nan, -np.inf  # scales that are not finite, a NaN that has no code
     qs = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
     sc = rng.uniform(0.1, 1.0, (n, k // 32)).astype(F32)
     if wtype == "q4_0":
